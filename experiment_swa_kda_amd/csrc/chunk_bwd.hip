@@ -21,9 +21,8 @@
 //    independent, so the 128x16 f32 slice of dS lives in VGPRs as MFMA accumulators of four
 //    compute waves, fed by two loader waves through an LDS ring of direct global->LDS loads.
 //    The launch also carries cache-warming workgroups for the CUs the scan leaves idle.
-//  * dense and decay VJPs: one workgroup per (chunk, head) tile, both bodies in one kernel
-//    (role by workgroup index) launched as full rounds over "all dense tiles, then all
-//    decay tiles".  Dense: 16x16x32 bf16 MFMA tiles with f32 accumulation, every global
+//  * dense and decay VJPs: one workgroup per (chunk, head) tile runs the dense and then the
+//    decay part, handing the dense results over on chip.  Dense: 16x16x32 bf16 MFMA tiles with f32 accumulation, every global
 //    operand requested in one batch.  Decay: the decay-scaled operands are built once per
 //    tile around the first (row side) or last (column side) row of each 16-row block, so
 //    every factor is <= 1 or bounded by the block's span; a tile with a block whose decay
@@ -711,8 +710,32 @@ struct NoGate {
   __device__ void operator()() const {}
 };
 
-template <int K, int V, class Gate = NoGate>
-__device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx, int4 ch, const Gate& gate = Gate()) {
+// What the decay part of a tile takes over from the dense part.  In one workgroup (CHIP) it
+// never leaves the chip: the raw dQg / dKd / dKb items in registers (exchanged through LDS
+// where the two parts own different items), dA, dM' and lam dL/dlam in LDS (TileSmem), the
+// dbeta partial in the registers of the first 64 threads.  Through the scratch buffer they
+// were 224 KB of stores and reloads per tile (K = V = 128), a quarter of the backward's
+// memory traffic, and the reloads a round trip each: fused call 90.3 -> 88.3 us at B2 T4096 H3,
+// 817 -> 774 us at B4 T8192 H6.  The separate dense and decay launches
+// of the stage entry points pass the same values through the scratch buffer.
+template <int K>
+struct DenseCarry {
+  f32x4 q[4 * (K / 16) / kDenseWaves], k[4 * (K / 16) / kDenseWaves], b[4 * (K / 16) / kDenseWaves];
+  float dbeta;
+};
+
+// LDS behind both parts' own regions: dA and dM' (bf16 [64][64 + 8]), lam dL/dlam (f32 [K]).
+template <int K>
+struct HandSmem {
+  static constexpr int AP = 64 + 8;
+  static constexpr size_t da = 0, dm = 64 * AP * 2, dgl = 2 * 64 * AP * 2;
+  static constexpr size_t bytes = dgl + K * 4;
+};
+
+// hand: offset of the HandSmem region (CHIP).
+template <int K, int V, bool CHIP, class Gate = NoGate>
+__device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx, int4 ch, DenseCarry<K>& cy,
+                                           size_t hand = 0, const Gate& gate = Gate()) {
   using L = DenseSmem<K, V>;
   constexpr int MP = L::TP, KP = L::KP, VP = L::VP;
   constexpr int kVjpThreads = kDenseThreads, kVjpWaves = kDenseWaves;
@@ -754,8 +777,11 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
   float* DQG = (float*)a.sc.p[S_DQG] + tile * 64 * K;
   float* DKD = (float*)a.sc.p[S_DKD] + tile * 64 * K;
   float* DKB = (float*)a.sc.p[S_DKB] + tile * 64 * K;
-  bf16* DA = (bf16*)a.sc.p[S_DA] + tile * 64 * 64;
-  bf16* DMP = (bf16*)a.sc.p[S_DMP] + tile * 64 * 64;
+  // dA, dM' and lam dL/dlam: to LDS for this workgroup's decay part, or to the scratch buffer
+  constexpr int DAP = CHIP ? HandSmem<K>::AP : 64;
+  bf16* DA = CHIP ? (bf16*)(smem + hand + HandSmem<K>::da) : (bf16*)a.sc.p[S_DA] + tile * 64 * 64;
+  bf16* DMP = CHIP ? (bf16*)(smem + hand + HandSmem<K>::dm) : (bf16*)a.sc.p[S_DMP] + tile * 64 * 64;
+  float* DGL = CHIP ? (float*)(smem + hand + HandSmem<K>::dgl) : (float*)a.sc.p[S_DGL] + tile * K;
 
   // PA's state rows: wave w owns key tile w / (4 / RPW) and RPW row tiles; its f32 S and
   // dS' rows are requested first, with everything P0 loads
@@ -861,7 +887,10 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
         accQ = mfma16(aO, sLo, accQ);
       }
       // raw dQg in C-layout item order (consumed with the same lane ownership)
-      *(f32x4*)(DQG + ((size_t)p * 64 + lane) * 4) = accQ;
+      if constexpr (CHIP)
+        cy.q[q] = accQ;
+      else
+        *(f32x4*)(DQG + ((size_t)p * 64 + lane) * 4) = accQ;
     }
   }
   // dA = tril(dO delta^T), 16x16 blocks of the lower triangle; upper blocks zero
@@ -869,7 +898,7 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
     const int ba = p / 4, bb = p % 4;
     if (bb > ba) {
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr) DA[(16 * ba + 4 * kg + rr) * 64 + 16 * bb + lr] = to_bf16(0.f);
+      for (int rr = 0; rr < 4; ++rr) DA[(16 * ba + 4 * kg + rr) * DAP + 16 * bb + lr] = to_bf16(0.f);
       continue;
     }
     const int i = 16 * ba + lr, j = 16 * bb + lr;
@@ -883,7 +912,7 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) {
       const int ii = 16 * ba + 4 * kg + rr;
-      DA[ii * 64 + jj] = to_bf16(jj <= ii ? acc[rr] : 0.f);
+      DA[ii * DAP + jj] = to_bf16(jj <= ii ? acc[rr] : 0.f);
     }
   }
 
@@ -965,7 +994,7 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
 #pragma unroll
       for (int e = 0; e < 8; ++e) dl = fmaf(xs[sv][e], to_f32(xd[sv][e]), dl);
     dl = swap32_sum(swap16_sum(dl));
-    if (rt0 == 0 && kg == 0) ((float*)a.sc.p[S_DGL])[tile * K + c] = dl * lamc;
+    if (rt0 == 0 && kg == 0) DGL[c] = dl * lamc;
 #pragma unroll
     for (int q = 0; q < RPW; ++q) {
       const int rt = rt0 + q, i = 16 * rt + lr;
@@ -982,7 +1011,10 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
         accW = mfma16(uHi, sHi, accW);
         accW = mfma16(uHi, sLo, accW);
       }
-      *(f32x4*)(DKD + ((size_t)p * 64 + lane) * 4) = accK;
+      if constexpr (CHIP)
+        cy.k[q] = accK;
+      else
+        *(f32x4*)(DKD + ((size_t)p * 64 + lane) * 4) = accK;
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) sDW[(16 * rt + 4 * kg + rr) * KP + c] = to_bf16(-accW[rr]);
     }
@@ -1067,13 +1099,16 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
     }
   }
   // d(beta kh e^G) = T^T dW, raw in C-layout item order (the decay kernel applies it)
-  for (int p = wave; p < NKT; p += kVjpWaves) {
-    const int rt = p % 4, ct = p / 4;
-    const int j = 16 * rt + lr, c = 16 * ct + lr;
+#pragma unroll
+  for (int n = 0; n < NKT / kVjpWaves; ++n) {
+    const int p = wave + kVjpWaves * n, rt = p % 4, ct = p / 4;
     f32x4 acc = zero4();
     for (int s = (16 * rt) / 32; s < 2; ++s)
       acc = mfma16(lds_col_frag(sT, MP, 32 * s, 16 * rt, lane), lds_col_frag(sDW, KP, 32 * s, 16 * ct, lane), acc);
-    *(f32x4*)(DKB + ((size_t)p * 64 + lane) * 4) = acc;
+    if constexpr (CHIP)
+      cy.b[n] = acc;
+    else
+      *(f32x4*)(DKB + ((size_t)p * 64 + lane) * 4) = acc;
   }
   __syncthreads();
 
@@ -1106,7 +1141,7 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
     for (int rr = 0; rr < 4; ++rr) {
       const int ii = 16 * ba + 4 * kg + rr;
       const float dm = jj < ii ? -acc[rr] : 0.f;
-      DMP[ii * 64 + jj] = to_bf16(sB[ii] * dm);
+      DMP[ii * DAP + jj] = to_bf16(sB[ii] * dm);
       float part = dm * mp[rr];
       part = group_sum<16>(part);
       if (lr == 0) sPM[bb * 64 + ii] = part;
@@ -1114,7 +1149,7 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
   }
   for (int idx = tid; idx < 64 * 64; idx += kVjpThreads) {
     const int ii = idx / 64, jj = idx % 64;
-    if (jj / 16 > ii / 16) DMP[idx] = to_bf16(0.f);
+    if (jj / 16 > ii / 16) DMP[ii * DAP + jj] = to_bf16(0.f);
   }
   __syncthreads();
 
@@ -1123,7 +1158,10 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
     float db = 0.f;
     for (int c = 0; c < V / 16; ++c) db += sPV[c * 64 + tid];
     for (int b = 0; b < 4; ++b) db += sPM[b * 64 + tid];
-    ((float*)a.sc.p[S_DBETA])[tile * 64 + tid] = db;
+    if constexpr (CHIP)
+      cy.dbeta = db;
+    else
+      ((float*)a.sc.p[S_DBETA])[tile * 64 + tid] = db;
   }
   asm volatile("" ::"v"(warm));
 }
@@ -1135,23 +1173,22 @@ template <int K>
 struct DecaySmem {
   static constexpr int QP = K + 8;                               // bf16 row stride of q, k
   static constexpr int GP = K + 4;                               // f32 row stride of G
-  static constexpr int AP = 64 + 8;                              // bf16 row stride of dA, dM'
+  static constexpr int AP = HandSmem<K>::AP;                     // bf16 row stride of dA, dM'
   static constexpr int HALF = K / 2;                             // key columns per pass
   static constexpr int OP = HALF + 8;                            // bf16 row stride of the operands
   static constexpr int NSEG = kVjpThreads / K;                   // cumsum segments per column
   static constexpr size_t off_q = 0;                             // bf16 [64][QP] q, later dq
   static constexpr size_t off_k = off_q + 64 * QP * 2;           // bf16 [64][QP] k, later dk
   static constexpr size_t off_g = off_k + 64 * QP * 2;           // f32 [64][GP] G, later dG
-  static constexpr size_t off_da = off_g + 64 * GP * 4;          // bf16 [64][AP] dA
-  static constexpr size_t off_dm = off_da + 64 * AP * 2;         // bf16 [64][AP] dM'
-  static constexpr size_t off_op = off_dm + 64 * AP * 2;         // bf16 6 x [64][OP] operands
+  static constexpr size_t off_op = off_g + 64 * GP * 4;          // bf16 6 x [64][OP] operands
   static constexpr size_t off_pb = off_op + 6 * 64 * OP * 2;     // f32 [K/16][64] dbeta partials
   static constexpr size_t off_pq = off_pb + (K / 16) * 64 * 4;   // f32 [K/16][64] qh . dqh
   static constexpr size_t off_pk = off_pq + (K / 16) * 64 * 4;   // f32 [K/16][64] kh . dkh
   static constexpr size_t off_gl = off_pk + (K / 16) * 64 * 4;   // f32 [4][K] dG_last partials
   static constexpr size_t off_row = off_gl + 4 * K * 4;          // f32 [5][64] beta, rq, rk, fq, fk
   static constexpr size_t off_f = off_row + 5 * 64 * 4;          // int [4] unsafe-block flags
-  static constexpr size_t bytes = off_f + 16;
+  static constexpr size_t off_hand = off_f + 16;                 // HandSmem (separate decay launch)
+  static constexpr size_t bytes = off_hand + HandSmem<K>::bytes;
   // after the item phase the operand region holds the cumsum segments and parameter partials
   static constexpr size_t off_seg = off_op;                      // f32 [NSEG][K]
   static constexpr size_t off_p0 = off_seg + NSEG * K * 4;       // f32 [NSEG][K]
@@ -1179,8 +1216,17 @@ struct DecaySmem {
 // layout, the layout in which the dense kernel stored dQg, dKd and dKb, so every
 // per-element term stays in registers.  The key columns go in two passes of K/2 (the
 // operands of one pass fit in LDS beside q, k and G).
-template <int K, class Gate = NoGate>
-__device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx, int4 ch, const Gate& gate = Gate()) {
+// LDS of a tile whose dense and decay parts run in one workgroup.
+template <int K, int V>
+struct TileSmem {
+  static constexpr size_t hand = cmax_sz(DenseSmem<K, V>::bytes, DecaySmem<K>::off_hand);
+  static constexpr size_t bytes = hand + HandSmem<K>::bytes;
+  static_assert(3 * 64 * K * 4 <= DecaySmem<K>::off_hand && 2 * 64 * K * 4 <= hand, "item exchange");
+};
+
+template <int K, bool CHIP>
+__device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx, int4 ch, const DenseCarry<K>& cy,
+                                           size_t hand) {
   using L = DecaySmem<K>;
   constexpr int QP = L::QP, GP = L::GP, AP = L::AP, HALF = L::HALF, OP = L::OP, NSEG = L::NSEG;
   constexpr int NKT = 4 * (K / 16);
@@ -1191,8 +1237,8 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
   bf16* sQ = (bf16*)(smem + L::off_q);
   bf16* sK = (bf16*)(smem + L::off_k);
   float* sG = (float*)(smem + L::off_g);
-  bf16* sDA = (bf16*)(smem + L::off_da);
-  bf16* sDM = (bf16*)(smem + L::off_dm);
+  bf16* sDA = (bf16*)(smem + hand + HandSmem<K>::da);
+  bf16* sDM = (bf16*)(smem + hand + HandSmem<K>::dm);
   bf16* sKRh = (bf16*)(smem + L::off_op);
   bf16* sKRl = sKRh + 64 * OP;
   bf16* sQCh = sKRl + 64 * OP;
@@ -1226,8 +1272,9 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
   const float* DQG = (const float*)a.sc.p[S_DQG] + tile * 64 * K;
   const float* DKD = (const float*)a.sc.p[S_DKD] + tile * 64 * K;
   const float* DKB = (const float*)a.sc.p[S_DKB] + tile * 64 * K;
-  // each wave's dqh, dkh and dG of its item in pass 0 and pass 1, held in registers across
-  // the barrier that completes the per-row dot products
+  // each wave's raw dQg, dKd and dKb of its item in pass 0 and pass 1 (loaded per pass from
+  // the scratch buffer in the separate decay launch), replaced by its dqh, dkh and dG, which
+  // are held in registers across the barrier that completes the per-row dot products
   f32x4 keep_q[2], keep_k[2], keep_g[2];
 
   // ---- P0: stage q, k (bf16), G, dA, dM' (bf16), beta and the per-row norm factors ----
@@ -1246,11 +1293,38 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
     const float bt = ((const float*)a.ws.p[R_BETA])[tile * 64 + tc];
     float gv[8];
     load8f(Gg + tc * K + c0, gv);
-    gate();  // everything below reads the dense role's results
-    // dA, dM': 64 x 64 f32 each, 4 consecutive per thread
+    // dA, dM': 64 x 64 bf16 each, 4 consecutive per thread
     const int ai = tid * 4;
     bf16x4 ya = {}, ym = {};
-    if (ai < 64 * 64) {
+    if constexpr (CHIP) {
+      // the dense part's items to the waves that own them here, while the loads above are in
+      // flight (the dense part's LDS is consumed; dKb has the same owners when a pass has an
+      // item for every wave)
+      constexpr int IPD = NKT / kDenseWaves;
+      constexpr bool kMoveB = NIH != kVjpWaves;
+      f32x4* sx = (f32x4*)smem;
+#pragma unroll
+      for (int n = 0; n < IPD; ++n) {
+        const int pd = (wave % (4 / IPD)) * IPD + n + 4 * (wave / (4 / IPD));
+        sx[pd * 64 + lane] = cy.q[n];
+        sx[(NKT + pd) * 64 + lane] = cy.k[n];
+        if constexpr (kMoveB) sx[(2 * NKT + wave + kDenseWaves * n) * 64 + lane] = cy.b[n];
+      }
+      __syncthreads();
+      if (wave < NIH) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          const int p = wave % 4 + 4 * (n * (HALF / 16) + wave / 4);
+          keep_q[n] = sx[p * 64 + lane];
+          keep_k[n] = sx[(NKT + p) * 64 + lane];
+          if constexpr (kMoveB)
+            keep_g[n] = sx[(2 * NKT + p) * 64 + lane];
+          else
+            keep_g[n] = cy.b[n];
+        }
+      }
+      __syncthreads();
+    } else if (ai < 64 * 64) {
       ya = *(const bf16x4*)(DA + ai);
       ym = *(const bf16x4*)(DMP + ai);
     }
@@ -1282,7 +1356,7 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
         sBeta[t] = bt;
       }
     }
-    if (ai < 64 * 64) {
+    if (!CHIP && ai < 64 * 64) {
       *(bf16x4*)(sDA + (ai / 64) * AP + ai % 64) = ya;
       *(bf16x4*)(sDM + (ai / 64) * AP + ai % 64) = ym;
     }
@@ -1298,7 +1372,7 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
   const bool unsafe = (sF[0] | sF[1] | sF[2] | sF[3]) != 0;
 
   // the dense part's dbeta partial of row tid (needed after P1; requested now)
-  const float dbeta_dense = tid < 64 ? ((const float*)a.sc.p[S_DBETA])[tile * 64 + tid] : 0.f;
+  const float dbeta_dense = CHIP ? cy.dbeta : tid < 64 ? ((const float*)a.sc.p[S_DBETA])[tile * 64 + tid] : 0.f;
   // ---- P1: per pass (K/2 key columns) build the decay-scaled operands, then one item per
   // wave: row side + column side + all per-element terms ----
 #pragma unroll 1
@@ -1314,9 +1388,16 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
     const int p = rt + 4 * ct;
     const int c = 16 * ct + lr;
     const int pi = wave < NIH ? p : 0;
-    const f32x4 rdQ = *(const f32x4*)(DQG + ((size_t)pi * 64 + plane) * 4);
-    const f32x4 rdK = *(const f32x4*)(DKD + ((size_t)pi * 64 + plane) * 4);
-    const f32x4 rdB = *(const f32x4*)(DKB + ((size_t)pi * 64 + plane) * 4);
+    f32x4 rdQ, rdK, rdB;
+    if constexpr (CHIP) {
+      rdQ = pass == 0 ? keep_q[0] : keep_q[1];
+      rdK = pass == 0 ? keep_k[0] : keep_k[1];
+      rdB = pass == 0 ? keep_g[0] : keep_g[1];
+    } else {
+      rdQ = *(const f32x4*)(DQG + ((size_t)pi * 64 + plane) * 4);
+      rdK = *(const f32x4*)(DKD + ((size_t)pi * 64 + plane) * 4);
+      rdB = *(const f32x4*)(DKB + ((size_t)pi * 64 + plane) * 4);
+    }
     if (!unsafe) {
       // operand group: row t, 4 consecutive columns
       const int t = ptid / (HALF / 4), c4 = (ptid % (HALF / 4)) * 4;
@@ -1404,7 +1485,7 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
         }
       } else {
         // a block whose decay spans more than 80 nats: exact per-pair f32 factors (dA, dM'
-        // as the dense part stored them, bf16)
+        // as the dense part rounded them, bf16)
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) {
           const int ii = 16 * rt + 4 * kg + rr;
@@ -1412,14 +1493,14 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
           float sq = 0.f, sk = 0.f;
           for (int j = 0; j <= ii; ++j) {
             const float kj = to_f32(sK[j * QP + c]) * sRk[j] * expf(gi - sG[j * GP + c]);
-            sq = fmaf(to_f32(DA[ii * 64 + j]), kj, sq);
-            sk = fmaf(to_f32(DMP[ii * 64 + j]), kj, sk);
+            sq = fmaf(to_f32(sDA[ii * AP + j]), kj, sq);
+            sk = fmaf(to_f32(sDM[ii * AP + j]), kj, sk);
           }
           float tq = 0.f, tk = 0.f;
           for (int i = ii; i < 64; ++i) {
             const float e = expf(sG[i * GP + c] - gi);
-            tq = fmaf(to_f32(DA[i * 64 + ii]), to_f32(sQ[i * QP + c]) * sRq[i] * e, tq);
-            tk = fmaf(to_f32(DMP[i * 64 + ii]), to_f32(sK[i * QP + c]) * sRk[i] * e, tk);
+            tq = fmaf(to_f32(sDA[i * AP + ii]), to_f32(sQ[i * QP + c]) * sRq[i] * e, tq);
+            tk = fmaf(to_f32(sDM[i * AP + ii]), to_f32(sK[i * QP + c]) * sRk[i] * e, tk);
           }
           rq[rr] = sq;
           rk[rr] = sk;
@@ -1541,7 +1622,7 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
   // K3: this thread's raw gate values, requested together before the segment sums (rows
   // past the chunk end read the last row and are not used), with the column's dG_last part
   // and gate parameters (loaded after the barrier they were a round trip of their own)
-  const float dgl = ((const float*)a.sc.p[S_DGL])[tile * K + c];
+  const float dgl = CHIP ? ((const float*)(smem + hand + HandSmem<K>::dgl))[c] : ((const float*)a.sc.p[S_DGL])[tile * K + c];
   const float alog = k3 ? a.A_log[h] : 0.f;
   const float bias = k3 ? a.dt_bias[h * K + c] : 0.f;
   float graw[RPS];
@@ -1605,25 +1686,33 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
 }
 
 // ---------------------------------------------------------------------------
-// dense and decay tiles in one launch
+// tile kernels
 // ---------------------------------------------------------------------------
-// Workgroup i < dense_count runs the dense VJP of tile dense_begin + i; the others run the
-// decay VJP of tile decay_begin + (i - dense_count).  The backward cuts the sequence "all
-// dense tiles, then all decay tiles" into launches of one workgroup per CU, so a launch that
-// finishes the dense tiles also starts the decay tiles whose dense tiles an earlier launch
-// completed: no round runs half empty, and no workgroup waits on another.
+// The dense or the decay part alone (the stage entry points), passing the dense part's results
+// through the scratch buffer.
 static_assert(kDenseThreads == kVjpThreads, "dense and decay tiles share the block size");
 template <int K, int V>
-__global__ __launch_bounds__(kVjpThreads) void chunk_bwd_vjp_kernel(BwdArgs a, int dense_begin, int dense_count,
-                                                                    int decay_begin) {
-  const int item = blockIdx.x;
-  if (item < dense_count) {
-    const int t = dense_begin + item;
-    dense_tile<K, V>(a, t / a.H, t % a.H, chunk_entry(a, t / a.H));
-  } else {
-    const int t = decay_begin + item - dense_count;
-    decay_tile<K>(a, t / a.H, t % a.H, chunk_entry(a, t / a.H));
-  }
+__global__ __launch_bounds__(kVjpThreads) void chunk_bwd_part_kernel(BwdArgs a, bool dense) {
+  const int cidx = blockIdx.x / a.H, h = blockIdx.x % a.H;
+  const int4 ch = chunk_entry(a, cidx);
+  DenseCarry<K> none;
+  if (dense)
+    dense_tile<K, V, false>(a, cidx, h, ch, none);
+  else
+    decay_tile<K, false>(a, cidx, h, ch, none, DecaySmem<K>::off_hand);
+}
+
+// Both parts of tile blockIdx.x in one workgroup, after a scan launch.  At 3,072 tiles (B4
+// T8192 H6, K = V = 128) the dense and decay parts as 24 launches of 256 workgroups took
+// 631 us, this one launch 458 us.
+template <int K, int V>
+__global__ __launch_bounds__(kVjpThreads) void chunk_bwd_tile_kernel(BwdArgs a) {
+  const int cidx = blockIdx.x / a.H, h = blockIdx.x % a.H;
+  const int4 ch = chunk_entry(a, cidx);
+  DenseCarry<K> cy;
+  dense_tile<K, V, true>(a, cidx, h, ch, cy, TileSmem<K, V>::hand);
+  __syncthreads();  // the dense part's LDS is consumed
+  decay_tile<K, true>(a, cidx, h, ch, cy, TileSmem<K, V>::hand);
 }
 
 // ---------------------------------------------------------------------------
@@ -1817,9 +1906,10 @@ __global__ __launch_bounds__(kVjpThreads) void chunk_bwd_fused_kernel(BwdArgs a,
     need = tp.need;
   }
   ScanGate gate{sv.base + kSyncRec + 32 * rec, V / 16, need, sv.abort, spin_limit, &s_failed};
-  dense_tile<K, V>(a, cidx, h, ch, gate);
-  __syncthreads();  // the dense part's stores are complete and visible to this workgroup
-  decay_tile<K>(a, cidx, h, ch);
+  DenseCarry<K> cy;
+  dense_tile<K, V, true>(a, cidx, h, ch, cy, TileSmem<K, V>::hand, gate);
+  __syncthreads();  // the dense part's LDS is consumed
+  decay_tile<K, true>(a, cidx, h, ch, cy, TileSmem<K, V>::hand);
   __syncthreads();
   if (s_failed && ch.y > 0) poison_tile<K, V>(a, cidx, h);  // computed from unwritten histories
 }
@@ -1922,7 +2012,7 @@ static int launch_backward(const kda_chunk_problem* p, const ChunkGeom& g, BwdAr
   if ((stages & all) == all && p->num_seqs > 0 && g.max_chunks > 0 && fused_backward_enabled()) {
     // one launch: scan members + prep workgroups + dense / decay tiles (see chunk_bwd_fused_kernel)
     constexpr size_t smem =
-        cmax_sz(kFusedSPW * BwdScanLds<K, V>::bytes + 2048, cmax_sz(DenseSmem<K, V>::bytes, DecaySmem<K>::bytes));
+        cmax_sz(kFusedSPW * BwdScanLds<K, V>::bytes + 2048, TileSmem<K, V>::bytes);
     static_assert(smem + 16 <= 160 * 1024, "fused backward LDS");
     static_assert(PrepLds<K, V>::bytes <= smem, "fused backward LDS (prep workgroups)");
     auto fused = chunk_bwd_fused_kernel<K, V>;
@@ -1982,38 +2072,23 @@ static int launch_backward(const kda_chunk_problem* p, const ChunkGeom& g, BwdAr
     hipLaunchKernelGGL(scan, dim3(grid + extra), dim3(kBwdThreads), smem_s, stream, a, pf, grid);
     KDA_LAUNCH_CHECK("chunk_backward scan");
   }
-  if (g.max_chunks > 0) {
-    constexpr size_t smem = DenseSmem<K, V>::bytes > DecaySmem<K>::bytes ? DenseSmem<K, V>::bytes
-                                                                          : DecaySmem<K>::bytes;
-    auto vjp = chunk_bwd_vjp_kernel<K, V>;
-    if (ensure_lds_limit((const void*)vjp, (int)smem) != hipSuccess)
+  const bool dense = stages & (1 << (KDA_STAGE_BWD_DENSE - 10));
+  const bool decay = stages & (1 << (KDA_STAGE_BWD_DECAY - 10));
+  if (g.max_chunks > 0 && dense && decay) {
+    auto tiles = chunk_bwd_tile_kernel<K, V>;
+    constexpr size_t smem = TileSmem<K, V>::bytes;
+    if (ensure_lds_limit((const void*)tiles, (int)smem) != hipSuccess)
+      return set_error(KDA_ERR_LAUNCH, "chunk_backward: tile LDS attribute failed");
+    hipLaunchKernelGGL(tiles, dim3(g.max_chunks * p->heads), dim3(kVjpThreads), smem, stream, a);
+    KDA_LAUNCH_CHECK("chunk_backward tiles");
+  } else if (g.max_chunks > 0 && (dense || decay)) {
+    // one part alone (the stage entry points)
+    constexpr size_t smem = cmax_sz(DenseSmem<K, V>::bytes, DecaySmem<K>::bytes);
+    auto part = chunk_bwd_part_kernel<K, V>;
+    if (ensure_lds_limit((const void*)part, (int)smem) != hipSuccess)
       return set_error(KDA_ERR_LAUNCH, "chunk_backward: LDS attribute failed");
-    const bool dense = stages & (1 << (KDA_STAGE_BWD_DENSE - 10));
-    const bool decay = stages & (1 << (KDA_STAGE_BWD_DECAY - 10));
-    const int N = g.max_chunks * p->heads;
-    const int R = device_cu_count();
-    auto launch = [&](int dense_begin, int dense_count, int decay_begin, int items) {
-      hipLaunchKernelGGL(vjp, dim3(items), dim3(kVjpThreads), smem, stream, a, dense_begin, dense_count, decay_begin);
-    };
-    if (dense && decay && R > 0 && N >= R) {
-      // items 0..N-1 dense, N..2N-1 decay, in launches of R: decay tile j (item N + j) is
-      // always in a later launch than dense tile j (item j) because N >= R
-      for (int start = 0; start < 2 * N; start += R) {
-        const int end = start + R < 2 * N ? start + R : 2 * N;
-        const int dcount = start < N ? (end < N ? end : N) - start : 0;
-        launch(start < N ? start : 0, dcount, (start > N ? start : N) - N, end - start);
-        KDA_LAUNCH_CHECK("chunk_backward dense/decay");
-      }
-    } else {
-      if (dense) {
-        launch(0, N, 0, N);
-        KDA_LAUNCH_CHECK("chunk_backward dense");
-      }
-      if (decay) {
-        launch(0, 0, 0, N);
-        KDA_LAUNCH_CHECK("chunk_backward decay");
-      }
-    }
+    hipLaunchKernelGGL(part, dim3(g.max_chunks * p->heads), dim3(kVjpThreads), smem, stream, a, dense);
+    KDA_LAUNCH_CHECK("chunk_backward dense / decay");
   }
   if (p->gate_mode == KDA_GATE_K3 && (stages & (1 << (KDA_STAGE_BWD_PARAMS - 10)))) {
     auto params = chunk_bwd_params_kernel<K>;

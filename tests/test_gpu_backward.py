@@ -369,3 +369,44 @@ def test_norm_gate_backward_strided_gate_equals_dense(D):
     assert torch.equal(out[..., 16:16 + H * D].view(B, T, H, D), ref[1])
     assert torch.equal(out[..., :16], torch.full_like(out[..., :16], 3.0))
     assert torch.equal(out[..., 16 + H * D:], torch.full_like(out[..., 16 + H * D:], 3.0))
+
+
+@pytest.mark.parametrize("KV", [(128, 128), (64, 64), (128, 64), (64, 128)])
+@pytest.mark.parametrize("T,gate", [(1, "k3"), (65, "precomputed"), (200, "k3")])
+def test_tile_handoff_equals_separate_parts(KV, T, gate):
+    """A tile's dense part hands its results to the decay part on chip, in the fused launch
+    and in the tile launch after a scan; the separate launches of the two parts pass them
+    through the scratch buffer.  The same values either way, at every head size (item owners
+    differ between the parts at K = 64) and at partial and single-token chunks, up to the
+    compiler's choice of fused multiply-adds in the decay part's f32 terms: a few roundings of
+    2^-24 in sums of some ten terms and a 64-row cumulative sum, so f32 gradients agree to 1e-6
+    (2-norm) and a bf16 gradient differs only where such a difference crosses a rounding
+    boundary (2^-8 of the value in at most one element of a thousand: 1.3e-4)."""
+    import ctypes
+    from experiment_swa_kda_amd import _lib
+    from experiment_swa_kda_amd._lib import ptr
+    K, V = KV
+    d = make_kda_inputs(2, T, 3, K, V, seed=K + V + T, gate=gate, dist="baseline")
+    do, _ = cotangents(d, 23)
+    full = gpu_grads(d, gate, do, None)
+    k3 = gate == "k3"
+    A, dt = (d["A_log"], d["dt_bias"]) if k3 else (None, None)
+    _, _, ws = ops.chunk_forward(d["q"], d["k"], d["v"], d["g"], d["beta"], A, dt, None, False, -5.0, K ** -0.5,
+                                 gate=gate)
+    p = ops._problem(d["q"], d["v"], None, ops.GATE_MODES[gate], -5.0, K ** -0.5)
+    lib = _lib.load()
+    nbytes = lib.kda_chunk_backward_scratch_bytes(ctypes.byref(p))
+    for stages in ((10, 11, 12, 13), (10, 14, 13)):
+        scratch = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        outs = [torch.empty_like(d[n]) for n in ("q", "k", "v", "g", "beta")]
+        par = [torch.empty_like(d["A_log"]), torch.empty_like(d["dt_bias"])] if k3 else [None, None]
+        args = (ptr(d["q"]), ptr(d["k"]), ptr(d["v"]), ptr(d["g"]), ptr(d["beta"]), ptr(A), ptr(dt), None, ptr(ws),
+                ptr(do), None, *[ptr(x) for x in outs], *[ptr(x) for x in par], None, ptr(scratch),
+                torch.cuda.current_stream().cuda_stream)
+        for stage in stages:
+            _lib.check(lib.kda_chunk_backward_stage(stage, ctypes.byref(p), *args), f"stage {stage}")
+        torch.cuda.synchronize()
+        for i, (x, y) in enumerate(zip(full[:7], outs + par)):
+            if y is not None:
+                bound = 1e-6 if y.dtype == torch.float32 else 1.3e-4
+                assert rel_err(y.reshape(-1), x.reshape(-1)) <= bound, (stages, i)
