@@ -1678,9 +1678,9 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
         p0 += sP0[s * K + tid];
         p1 += sP1[s * K + tid];
       }
-      float* PP = (float*)a.sc.p[S_PP] + tile * 2 * K;
-      PP[tid] = p0;
-      PP[K + tid] = p1;
+      ((float*)a.sc.p[S_PP])[tile * K + tid] = p0;
+      p1 = wave_sum(p1);  // over 64 channels; the K / 64 sums go to chunk_bwd_params_kernel
+      if (lane == 0) ((float*)a.sc.p[S_PA])[tile * (K / 64) + wave] = p1;
     }
   }
 }
@@ -1816,7 +1816,10 @@ __device__ void poison_tile(const BwdArgs& a, int cidx, int h) {
     a.dv[(size_t)(row0 + i / V) * a.gld_v + (size_t)h * V + i % V] = nanb;
   for (int t = threadIdx.x; t < len; t += blockDim.x) a.dbeta[(size_t)(row0 + t) * a.dbeta_ld + h] = nanb;
   if (a.gate_mode == KDA_GATE_K3)
-    for (int i = threadIdx.x; i < 2 * K; i += blockDim.x) ((float*)a.sc.p[S_PP])[tile * 2 * K + i] = nan;
+    for (int i = threadIdx.x; i < K; i += blockDim.x) {
+      ((float*)a.sc.p[S_PP])[tile * K + i] = nan;
+      if (i < K / 64) ((float*)a.sc.p[S_PA])[tile * (K / 64) + i] = nan;
+    }
 }
 
 // Clears the sync words and writes the chunk order: chunk c of sequence s with n chunks
@@ -1919,56 +1922,50 @@ __global__ __launch_bounds__(kVjpThreads) void chunk_bwd_fused_kernel(BwdArgs a,
 // ---------------------------------------------------------------------------
 constexpr int kParamThreads = 1024;
 
-// Thread (part, c) sums the chunks part, part + P, ... (P = kParamThreads / K) in order;
-// the P partials and then the K channels are combined in a fixed order.
+// ddt_bias[c] = sum over the chunks of the tiles' partials, dA_log = sum over the chunks of
+// their channel sums.  Workgroup (h, g): g < K / 16 sums 16 channels of head h (64 parts of the
+// chunks, every kParamBatch loads of a thread in flight together), g = K / 16 sums dA_log.
+// One workgroup per head read all 2 K partials of every chunk: 37 us at 512 chunks x 6 heads;
+// split over the channels, with dA_log's channel sum already taken in the tile, 6 us.
+constexpr int kParamBatch = 8;
+
 template <int K>
 __global__ __launch_bounds__(kParamThreads) void chunk_bwd_params_kernel(BwdArgs a, int max_chunks) {
-  constexpr int P = kParamThreads / K;
-  __shared__ float s0[P][K], s1[P][K];
-  const int h = blockIdx.x, c = threadIdx.x % K, part = threadIdx.x / K;
+  constexpr int kWaves = kParamThreads / kWave;
+  __shared__ float part[kWaves][16];
+  const int h = blockIdx.x, g = blockIdx.y, wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const bool bias = g < K / 16;
+  // term e of chunk chn: 16 channels (bias), or the K / 64 channel sums of the tile
+  const int E = bias ? 16 : K / 64, parts = kParamThreads / E;
+  const int e = threadIdx.x % E, p = threadIdx.x / E;
+  const float* src = bias ? (const float*)a.sc.p[S_PP] + 16 * g + e : (const float*)a.sc.p[S_PA] + e;
+  const size_t ld = bias ? K : K / 64;
   const int4* chunks = (const int4*)a.ws.p[R_CHUNKS];
-  const float* PP = (const float*)a.sc.p[S_PP];
-  float p0 = 0.f, p1 = 0.f;
-  // batches of 16 chunks (one batch per part at 128 chunks): every load of a batch is issued
-  // before any is used (empty chunks' partials were never written and are selected away,
-  // not multiplied)
-  constexpr int U = 16;
-  for (int chn0 = part; chn0 < max_chunks; chn0 += U * P) {
-    float x0[U], x1[U];
-    bool live[U];
+  float sum = 0.f;
+  // empty chunks' partials were never written and are selected away, not multiplied
+  for (int c0 = p; c0 < max_chunks; c0 += kParamBatch * parts) {
+    float x[kParamBatch];
+    bool live[kParamBatch];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int chn = min(chn0 + u * P, max_chunks - 1);
-      const size_t tile = (size_t)chn * a.H + h;
-      live[u] = chn0 + u * P < max_chunks && chunks[chn].y > 0;
-      x0[u] = PP[tile * 2 * K + c];
-      x1[u] = PP[tile * 2 * K + K + c];
+    for (int u = 0; u < kParamBatch; ++u) {
+      const int chn = min(c0 + u * parts, max_chunks - 1);
+      live[u] = c0 + u * parts < max_chunks && (a.fixed_T > 0 || chunks[chn].y > 0);
+      x[u] = src[((size_t)chn * a.H + h) * ld];
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      p0 += live[u] ? x0[u] : 0.f;
-      p1 += live[u] ? x1[u] : 0.f;
-    }
+    for (int u = 0; u < kParamBatch; ++u) sum += live[u] ? x[u] : 0.f;
   }
-  s0[part][c] = p0;
-  s1[part][c] = p1;
+  // the lanes of a wave, then the waves, in a fixed order
+  sum = bias ? lane_stride_sum<16>(sum) : wave_sum(sum);
+  if (lane < 16) part[wave][lane] = sum;
   __syncthreads();
-  __shared__ float s_wave[K / 64];
-  if (part == 0) {
-    float t0 = 0.f, t1 = 0.f;
-    for (int q = 0; q < P; ++q) {
-      t0 += s0[q][c];
-      t1 += s1[q][c];
-    }
-    a.ddt_bias[h * K + c] = t0;
-    t1 = wave_sum(t1);  // fixed butterfly order within the wave
-    if (c % 64 == 0) s_wave[c / 64] = t1;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < (bias ? 16 : 1)) {
     float t = 0.f;
-    for (int q = 0; q < K / 64; ++q) t += s_wave[q];
-    a.dA_log[h] = t;
+    for (int w = 0; w < kWaves; ++w) t += part[w][threadIdx.x];
+    if (bias)
+      a.ddt_bias[h * K + 16 * g + threadIdx.x] = t;
+    else
+      a.dA_log[h] = t;
   }
 }
 
@@ -2092,7 +2089,7 @@ static int launch_backward(const kda_chunk_problem* p, const ChunkGeom& g, BwdAr
   }
   if (p->gate_mode == KDA_GATE_K3 && (stages & (1 << (KDA_STAGE_BWD_PARAMS - 10)))) {
     auto params = chunk_bwd_params_kernel<K>;
-    hipLaunchKernelGGL(params, dim3(p->heads), dim3(kParamThreads), 0, stream, a, g.max_chunks);
+    hipLaunchKernelGGL(params, dim3(p->heads, K / 16 + 1), dim3(kParamThreads), 0, stream, a, g.max_chunks);
     KDA_LAUNCH_CHECK("chunk_backward params");
   }
   return KDA_OK;

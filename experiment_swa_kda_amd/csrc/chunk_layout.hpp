@@ -77,7 +77,8 @@ enum ScRegion {
   S_DQG,      // f32  [tile][item][64 lane][4]  dL/dQg  in MFMA C layout (item = row tile + 4 col tile)
   S_DKD,      // f32  [tile][item][64 lane][4]  dL/dKd  (same layout)
   S_DKB,      // f32  [tile][item][64 lane][4]  dL/d(beta kh exp(G))  (same layout)
-  S_PP,       // f32  [tile][2][K]   gate parameter partials {sum draw, sum draw*(z+b)}
+  S_PP,       // f32  [tile][K]      gate bias partials: sum over the chunk of draw
+  S_PA,       // f32  [tile][K/64]   gate scale partials: sum over 64 channels of draw*(z+b)
   S_DGL,      // f32  [tile][K]      lam * dL/dlam (the state-decay part of dL/dG_last)
   S_DBETA,    // f32  [tile][64]     dL/dbeta from the dense VJP (U, M' terms)
   S_SYNC,     // int  fused backward: ticket, abort, per-record step counts, per-tile strip arrivals
@@ -128,7 +129,8 @@ __host__ __device__ inline size_t sc_region_bytes(const ChunkGeom& g, int r) {
     case S_E: return nt * K * V * kEBytes;
     case S_DA: case S_DMP: return nt * 64 * 64 * 2;
     case S_DQG: case S_DKD: case S_DKB: return nt * 64 * K * 4;
-    case S_PP: return nt * 2 * K * 4;
+    case S_PP: return nt * K * 4;
+    case S_PA: return nt * (K / 64) * 4;
     case S_DGL: return nt * K * 4;
     case S_DBETA: return nt * 64 * 4;
     case S_SYNC: return (32 + 32 * (size_t)g.num_seqs * g.heads + nt) * 4;

@@ -410,3 +410,20 @@ def test_tile_handoff_equals_separate_parts(KV, T, gate):
             if y is not None:
                 bound = 1e-6 if y.dtype == torch.float32 else 1.3e-4
                 assert rel_err(y.reshape(-1), x.reshape(-1)) <= bound, (stages, i)
+
+
+@pytest.mark.parametrize("T,H,K", [(33000, 1, 64), (700, 3, 128), (63, 2, 64)])
+def test_gate_parameter_sums(T, H, K):
+    """dt_bias and A_log gradients are the sums over tokens of draw_gate and of
+    draw_gate (z + b) (dz = draw_gate is returned rounded to bf16): one chunk, a few, and more
+    than one batch of loads per part (516 chunks).  Each returned term is off by at most 2^-9
+    of itself, so a sum differs by 2^-9 times the root of the sum of squares, with six
+    deviations of room."""
+    d = make_kda_inputs(1, T, H, K, K, seed=T + K, state=False)
+    do, _ = cotangents(d, 3)
+    _, _, _, dz, _, dA, ddt, _ = gpu_grads(d, "k3", do, None)
+    dz, pre = dz.double()[0], d["g"].double()[0] + d["dt_bias"].double().view(H, K)
+    bound = 6 * 2.0 ** -9
+    assert ((ddt.double().view(H, K) - dz.sum(0)).abs() <= bound * dz.square().sum(0).sqrt() + 1e-12).all()
+    t = dz * pre
+    assert ((dA.double() - t.sum((0, 2))).abs() <= bound * t.square().sum((0, 2)).sqrt() + 1e-12).all()
