@@ -33,6 +33,7 @@
 //    chunk_bwd_fused_kernel).  The staged entry points keep the separate launches.
 #include "chunk_host.hpp"
 #include "kda_device.hpp"
+#include "seg_combine.hpp"
 
 #include <atomic>
 #include <cstdlib>
@@ -389,25 +390,59 @@ __device__ __forceinline__ void publish_strip(int* sync, int rec, int strip, int
 // operands into L2 ahead of the steps, the rest exit, and after each step's history (X_c)
 // is stored the strip's progress word is raised: r + 1 means the strip has finished the
 // r + 1 last chunks of the sequence.
-template <int K, int V, bool PUB, int SPW>
+//
+// Segments: a sequence of many chunks with few strips is a chain that leaves the chip idle
+// (512 steps of 0.45 us on 8 workgroups at B1 T32768 H1).  One chunk maps X affinely,
+// X_{c-1} = (diag(lam) - G_c) X_c + E_c, so a segment of chunks maps the gradient at its end to
+// the one at its start as P X + Sigma, P = the product of its (diag(lam) - G).  kScanLocal runs
+// every segment but the last (segments count from the sequence's end, as the scan walks) from
+// [0 | I]: Sigma (V / 16 strips) and P (K / 16 strips, E = 0); seg_combine_kernel chains
+// X_in(j + 1) = P_j X_in(j) + Sigma_j; kScanReplay reruns every segment from its true X_in and
+// writes the histories and the initial-state gradient.
+enum ScanMode { kScanWhole, kScanLocal, kScanReplay };
+
+// Hand-off of the segmented scan, in the scratch regions that only the separate dense and
+// decay launches use (no scratch of its own; bwd_segmented checks that it fits):
+//   P     bf16 [rec][segment][hi, lo] K x K A fragments, permuted      (S_DQG)
+//   sigma f32  [rec][segment][V][K]                                    (S_DKD)
+//   xin   f32  [rec][segment][V][K], segments >= 1                     (S_DKB)
+struct SegArgs {
+  int len = 0, max = 1;  // chunks per segment, segments of the longest sequence
+};
+
+template <int K, int V, bool PUB, int SPW, int MODE = kScanWhole>
 __device__ __forceinline__ void bwd_scan_body(const BwdArgs& a, int* progress, const int* prep_flags = nullptr,
-                                              long long spin_limit = 0) {
+                                              long long spin_limit = 0, const SegArgs& sa = SegArgs()) {
+  static_assert(MODE == kScanWhole || (!PUB && SPW == 1), "segments run in launches of their own");
   using L = BwdScanLds<K, V>;
   constexpr int CW = kScanCW, KT = K / 16 / CW, NB = K / 32, SP = L::SP;
   static_assert(KT >= 1 && KT * CW == K / 16, "X tiles split evenly over the compute waves");
-  constexpr int NSG = V / 16 / SPW;  // strip groups (workgroups) per record
+  constexpr int NSG = (MODE == kScanLocal ? V + K : V) / 16 / SPW;  // strip groups (workgroups) per record
   constexpr int kLoader = CW * SPW, kHistory = kLoader + 1, kPrefetch0 = kLoader + 2;
   constexpr int kPrefetchWaves = 2 * SPW;  // look-ahead lanes: this group's shared lines + its E lines
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int H = a.H;
   int rec, sg;
-  if (!xcd_strip_coords(a.num_seqs * H, NSG, rec, sg)) return;
+  if (!xcd_strip_coords(a.num_seqs * H * (MODE == kScanWhole ? 1 : sa.max), NSG, rec, sg)) return;
+  const int seg = MODE == kScanWhole ? 0 : rec % sa.max, rseg = rec;
+  if (MODE != kScanWhole) rec /= sa.max;
   const int seq = rec / H, h = rec % H;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const int lr = lane % 16, kg = lane / 16;
   const int2 sq = seq_entry(a, seq);  // {first chunk, chunk count}
-  const int n = sq.y;
-  auto tile_of = [&](int r) { return (size_t)(sq.x + max(n - 1 - r, 0)) * H + h; };  // step r's chunk
+  // this workgroup's steps: chunk c_end - 1 first, n of them
+  int n = sq.y, c_end = sq.x + sq.y;
+  bool last_seg = true;
+  if (MODE != kScanWhole) {
+    const int nseg = (sq.y + sa.len - 1) / sa.len;
+    if (MODE == kScanLocal ? seg + 1 >= nseg : seg >= max(nseg, 1)) return;
+    last_seg = seg + 1 >= nseg;
+    n = min(sq.y - seg * sa.len, sa.len);
+    c_end -= seg * sa.len;
+  }
+  const bool pstrip = MODE == kScanLocal && sg >= V / 16;  // a strip of P (E = 0)
+  const int vsg = MODE == kScanLocal ? min(sg, V / 16 - 1) : sg;
+  auto tile_of = [&](int r) { return (size_t)(c_end - 1 - min(r, n - 1)) * H + h; };  // step r's chunk
   auto group = [&](int g) { return smem + g * L::bytes; };  // a strip's LDS (E ring, X staging)
   // Fused launch with the prep inside it: a chunk's -G and E exist once its prep workgroup
   // raised the chunk's flag (after its write-through stores completed).  The loader waits for
@@ -485,7 +520,7 @@ __device__ __forceinline__ void bwd_scan_body(const BwdArgs& a, int* progress, c
 #pragma unroll
       for (int g = 0; g < SPW; ++g) {
         char* slot = group(g) + (r % kBwdRing) * L::slot;
-        const char* e = (const char*)a.sc.p[S_E] + (tile * K * V + (size_t)(sg * SPW + g) * K * 16) * kEBytes + lane * 16;
+        const char* e = (const char*)a.sc.p[S_E] + (tile * K * V + (size_t)(vsg * SPW + g) * K * 16) * kEBytes + lane * 16;
 #pragma unroll
         for (int b = 0; b < (K * 16 * kEBytes) / 1024; ++b) dma16(e + b * 1024, slot + L::off_e + b * 1024);
         if (lane < K / 4) dma16((const float*)a.ws.p[R_LAM] + tile * K + lane * 4, slot + L::off_lam);
@@ -509,6 +544,7 @@ __device__ __forceinline__ void bwd_scan_body(const BwdArgs& a, int* progress, c
     return;
   }
   if (wave == kHistory) {
+    if (MODE == kScanLocal) return;  // (an ended wave takes no part in the barriers)
     // ---- history wave: X_c of step r (bf16 [v][k] in LDS) is read after S(r) and stored
     // into each strip's [K][16] block of the strip-major history, 512 contiguous bytes per
     // store instruction.  In the fused launch step r - kPubLag is published once its stores
@@ -560,7 +596,13 @@ __device__ __forceinline__ void bwd_scan_body(const BwdArgs& a, int* progress, c
 #pragma unroll
   for (int kt = 0; kt < KT; ++kt) {
     const int k0 = 16 * (cw * KT + kt) + 4 * kg;
-    if (a.dsfin) {
+    if (MODE == kScanLocal) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) X[kt][q] = pstrip && k0 + q == 16 * (sg - V / 16) + lr ? 1.f : 0.f;
+    } else if (MODE == kScanReplay && seg > 0) {
+      const float4 s = *(const float4*)((const float*)a.sc.p[S_DKB] + ((size_t)rseg * V + v0 + lr) * K + k0);
+      X[kt][0] = s.x; X[kt][1] = s.y; X[kt][2] = s.z; X[kt][3] = s.w;
+    } else if (a.dsfin) {
       const float4 s = *(const float4*)(a.dsfin + (((size_t)seq * H + h) * V + v0 + lr) * K + k0);
       X[kt][0] = s.x; X[kt][1] = s.y; X[kt][2] = s.z; X[kt][3] = s.w;
     } else {
@@ -618,6 +660,7 @@ __device__ __forceinline__ void bwd_scan_body(const BwdArgs& a, int* progress, c
       } else {
         e = *(const f32x4*)(slot + L::off_e + (ktg * 64 + lane) * 16);
       }
+      if (pstrip) e = zero4();
       f32x4 acc;
       acc[0] = fmaf(lam.x, X[kt][0], e[0]);
       acc[1] = fmaf(lam.y, X[kt][1], e[1]);
@@ -640,7 +683,27 @@ __device__ __forceinline__ void bwd_scan_body(const BwdArgs& a, int* progress, c
     }
   }
   if (PUB) ring_barrier();  // final
-  if (a.ds0) {
+  if constexpr (MODE == kScanLocal) {
+    if (!pstrip) {
+      float* sg_out = (float*)a.sc.p[S_DKD] + ((size_t)rseg * V + v0 + lr) * K;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+        *(float4*)(sg_out + 16 * (cw * KT + kt) + 4 * kg) = make_float4(X[kt][0], X[kt][1], X[kt][2], X[kt][3]);
+    } else {
+      bf16* hi = (bf16*)a.sc.p[S_DQG] + (size_t)rseg * 2 * K * K;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const size_t o = perm_frag_elem(K, 16 * (cw * KT + kt) + 4 * kg + q, 16 * (sg - V / 16) + lr);
+          const bf16 x = to_bf16(X[kt][q]);
+          hi[o] = x;
+          hi[(size_t)K * K + o] = to_bf16(X[kt][q] - to_f32(x));
+        }
+    }
+    return;
+  }
+  if (a.ds0 && last_seg) {
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
       const int k0 = 16 * (cw * KT + kt) + 4 * kg;
@@ -658,6 +721,11 @@ __global__ __launch_bounds__(kBwdThreads) void chunk_bwd_scan_kernel(BwdArgs a, 
     return;
   }
   bwd_scan_body<K, V, false, 1>(a, nullptr);
+}
+
+template <int K, int V, int MODE>
+__global__ __launch_bounds__(kBwdThreads) void chunk_bwd_seg_kernel(BwdArgs a, SegArgs sa) {
+  bwd_scan_body<K, V, false, 1, MODE>(a, nullptr, nullptr, 0, sa);
 }
 
 // ---------------------------------------------------------------------------
@@ -1977,8 +2045,23 @@ static long long wait_limit_ticks() {
   return v < 0 ? kSpinLimitDefault : v;
 }
 
-// KDA_BWD_FUSED=0 selects the three-launch backward (scan, then rounds of dense / decay
-// tiles).
+// Segments of the reverse scan (len 0: whole sequences in one pass): the forward's segments,
+// where the strips are few enough that two shorter passes beat the one long chain (whole K3
+// backward, K = V = 128, without and with segments): 345 -> 168 us at 8 strips x 512 chunks
+// (B1 T32768 H1), 122 -> 95 at 16 x 128, 432 -> 395 at 24 x 512 and 132 -> 133 at 24 x 128; at
+// 32 x 128 the fused launch takes 135 us, segments 149.  The hand-off must fit the scratch
+// regions it borrows (see SegArgs): at most max_chunks / 2 segments in all.
+constexpr long kBwdSegStrips = 24;
+static SegArgs bwd_segments(const ChunkGeom& g) {
+  SegArgs sa;
+  const long strips = (long)g.num_seqs * g.heads * (g.V / 16);
+  if (g.seg_len == 0 || strips > kBwdSegStrips || 2L * g.num_seqs * g.max_segs > g.max_chunks) return sa;
+  sa.len = g.seg_len;
+  sa.max = g.max_segs;
+  return sa;
+}
+
+// KDA_BWD_FUSED=0 selects the separate launches (prep, scan, tiles) for every problem.
 static bool fused_backward_enabled() {
   static const bool on = [] {
     const char* e = getenv("KDA_BWD_FUSED");
@@ -1987,6 +2070,55 @@ static bool fused_backward_enabled() {
   return on;
 }
 
+// Fused launch or separate launches (prep, scan, tiles)?  In the fused launch the tiles hide
+// under the scan, but each scan member holds a CU that a tile could use, and the tiles' traffic
+// stretches the scan's step (0.45 -> 0.77 us).  It gains where the scan is a long chain on few
+// CUs with more than a round of tiles behind it (K = V = 128, whole K3 backward, fused against
+// separate launches): 98 against 121 us at 384 tiles x 48 strips (B2 T4096 H3), 135 / 165 at
+// 512 x 32, 173 / 176 at 768 x 96.  It loses when the strips fill the chip: 122 / 115 at 512 x
+// 128, 433 / 322 at 1,536 x 192, 795 / 636 at 3,072 x 192 (B4 T8192 H6); the limit is 3/8 of
+// the CUs.  Its scan members wait for prep workgroups of the same launch, so the strips must
+// leave CUs free in any case: at 256 strips no prep workgroup could start.  A problem of at
+// most a quarter round of tiles has nothing to hide (44 / 45 us at 8 tiles), and the separate
+// launches cannot fail in a wait, so their callers need not read the failure flag.  With
+// K V <= 64^2 a tile is half as long and the lines lie lower: 70 / 73 us at 384 tiles x 24
+// strips, but 50 / 41 at 128 x 16, 83 / 77 at 512 x 32, 192 / 182 at 1,536 x 96.
+static bool fused_backward(const ChunkGeom& g) {
+  if (!fused_backward_enabled()) return false;
+  const int cus = device_cu_count();
+  const long tiles = (long)g.max_chunks * g.heads, strips = (long)g.num_seqs * g.heads * (g.V / 16);
+  if (bwd_segments(g).len > 0) return false;
+  return g.K * g.V > 64 * 64 ? tiles > cus / 4 && 8 * strips <= 3L * cus : tiles > cus && 8 * strips <= cus;
+}
+
+template <int K, int V>
+static int launch_seg_scan(const BwdArgs& a, const SegArgs& sa, hipStream_t stream) {
+  auto local = chunk_bwd_seg_kernel<K, V, kScanLocal>;
+  auto replay = chunk_bwd_seg_kernel<K, V, kScanReplay>;
+  constexpr int smem = BwdScanLds<K, V>::bytes;
+  if (ensure_lds_limit((const void*)local, smem) != hipSuccess || ensure_lds_limit((const void*)replay, smem) != hipSuccess)
+    return set_error(KDA_ERR_LAUNCH, "chunk_backward: segmented scan LDS attribute failed");
+  const int nrec = a.num_seqs * a.H, groups = (nrec * sa.max + kXcds - 1) / kXcds;
+  hipLaunchKernelGGL(local, dim3(kXcds * ((V + K) / 16) * groups), dim3(kBwdThreads), smem, stream, a, sa);
+  KDA_LAUNCH_CHECK("chunk_backward segment maps");
+  CombineArgs c;
+  c.H = a.H;
+  c.num_seqs = a.num_seqs;
+  c.fixed_T = a.fixed_T;
+  c.seg_len = sa.len;
+  c.max_segs = sa.max;
+  c.seqs = (const int2*)a.ws.p[R_SEQS];
+  c.start = a.dsfin;
+  c.P = (const bf16*)a.sc.p[S_DQG];
+  c.sigma = (const float*)a.sc.p[S_DKD];
+  c.out = (float*)a.sc.p[S_DKB];
+  auto comb = seg_combine_kernel<K, V, true>;
+  hipLaunchKernelGGL(comb, dim3(kXcds * (V / 16) * ((nrec + kXcds - 1) / kXcds)), dim3(kCombThreads), 0, stream, c);
+  KDA_LAUNCH_CHECK("chunk_backward segment combine");
+  hipLaunchKernelGGL(replay, dim3(kXcds * (V / 16) * groups), dim3(kBwdThreads), smem, stream, a, sa);
+  KDA_LAUNCH_CHECK("chunk_backward segment replay");
+  return KDA_OK;
+}
 
 template <int K, int V>
 static int launch_backward(const kda_chunk_problem* p, const ChunkGeom& g, BwdArgs& a,
@@ -2006,7 +2138,7 @@ static int launch_backward(const kda_chunk_problem* p, const ChunkGeom& g, BwdAr
     KDA_LAUNCH_CHECK("chunk_backward prep");
     return KDA_OK;
   };
-  if ((stages & all) == all && p->num_seqs > 0 && g.max_chunks > 0 && fused_backward_enabled()) {
+  if ((stages & all) == all && p->num_seqs > 0 && g.max_chunks > 0 && fused_backward(g)) {
     // one launch: scan members + prep workgroups + dense / decay tiles (see chunk_bwd_fused_kernel)
     constexpr size_t smem =
         cmax_sz(kFusedSPW * BwdScanLds<K, V>::bytes + 2048, TileSmem<K, V>::bytes);
@@ -2033,19 +2165,20 @@ static int launch_backward(const kda_chunk_problem* p, const ChunkGeom& g, BwdAr
 #endif
     KDA_LAUNCH_CHECK("chunk_backward fused");
     stages &= ~all;
-  } else if ((stages & all) == all && g.max_chunks > 0) {
-    // the staged backward never waits; clearing the sync words keeps
-    // kda_chunk_backward_status meaningful after it
-    const int nrec = p->num_seqs * p->heads;
-    hipLaunchKernelGGL(chunk_bwd_sched_kernel, dim3(1), dim3(1024), 0, stream, a, g.max_chunks,
-                       sync_words(nrec, g.max_chunks * p->heads));
-    KDA_LAUNCH_CHECK("chunk_backward sched");
   }
   if (p->num_seqs > 0 && (stages & (1 << (KDA_STAGE_BWD_SCAN - 10)))) {
     if (g.max_chunks > 0) {
       int rc = launch_prep(0);
       if (rc != KDA_OK) return rc;
     }
+    const SegArgs sa = bwd_segments(g);
+    if (sa.len > 0) {
+      int rc = launch_seg_scan<K, V>(a, sa, stream);
+      if (rc != KDA_OK) return rc;
+      stages &= ~(1 << (KDA_STAGE_BWD_SCAN - 10));
+    }
+  }
+  if (p->num_seqs > 0 && (stages & (1 << (KDA_STAGE_BWD_SCAN - 10)))) {
     auto scan = chunk_bwd_scan_kernel<K, V>;
     constexpr size_t smem_s = BwdScanLds<K, V>::bytes;
     if (ensure_lds_limit((const void*)scan, (int)smem_s) != hipSuccess)
@@ -2217,7 +2350,9 @@ extern "C" int kda_chunk_backward_status(const kda_chunk_problem* p, const void*
               "chunk_backward_status: scratch must be non-null and 256-byte aligned");
   if (padded_route(p)) return padded_status(p, scratch, stream);
   if (generic_dims(p)) return KDA_OK;  // the token-serial backward has no waits
-  const Regions sc = sc_regions(make_geom(p), const_cast<void*>(scratch));
+  const ChunkGeom g = make_geom(p);
+  if (!fused_backward(g)) return KDA_OK;  // the separate launches wait on nothing inside a kernel
+  const Regions sc = sc_regions(g, const_cast<void*>(scratch));
   int word = 0;
   hipError_t e = hipMemcpyAsync(&word, sc.p[S_SYNC] + sizeof(int), sizeof(int), hipMemcpyDeviceToHost, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);

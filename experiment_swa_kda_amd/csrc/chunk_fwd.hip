@@ -31,6 +31,7 @@
 #include "chunk_host.hpp"
 #include "kda_device.hpp"
 #include "kda_host.hpp"
+#include "seg_combine.hpp"
 
 namespace kda {
 
@@ -1078,7 +1079,7 @@ __global__ __launch_bounds__(kScanThreads) void chunk_fwd_scan_kernel(FwdArgs a)
 //  1. local (chunk_fwd_seg_kernel<.., false>): every segment but the last of every
 //     recurrence runs its chunks from the augmented start [0 | I] (V + K columns; the
 //     identity columns see U = 0), giving [Sigma | P] -- segments run in parallel;
-//  2. combine (chunk_fwd_combine_kernel): S_in(j+1) = P_j S_in(j) + Sigma_j, sequential over
+//  2. combine (seg_combine_kernel): S_in(j+1) = P_j S_in(j) + Sigma_j, sequential over
 //     the segments of one recurrence, one wave per V strip (S as hi + lo bf16 operands);
 //  3. replay (chunk_fwd_seg_kernel<.., true>): every segment reruns its chunks from its true
 //     entering state and writes the state / delta histories exactly as the one-pass scan.
@@ -1328,113 +1329,6 @@ __global__ __launch_bounds__(kSegThreads) void chunk_fwd_seg_kernel(FwdArgs a, i
   }
 }
 
-// S_in(j+1) = P_j S_in(j) + Sigma_j over the segments of one recurrence.  One workgroup per
-// (recurrence, V strip); wave w owns state tiles w * TPW .. (w + 1) * TPW - 1.  Each step the
-// waves publish their tiles as hi + lo bf16 B-operand halves in LDS (about 16 mantissa
-// bits of the state), one barrier, and every wave multiplies its rows of P_j (bf16
-// fragments written by the local kernel, prefetched a step ahead) by the whole state.
-constexpr int kCombThreads = 4 * kWave;
-constexpr int kCombBatch = 8;
-
-template <int K, int V>
-__global__ __launch_bounds__(kCombThreads) void chunk_fwd_combine_kernel(FwdArgs a, int seg_len, int max_segs) {
-  constexpr int KT = K / 16, NB = K / 32, VS = V / 16, TPW = KT / 4;
-  __shared__ __attribute__((aligned(16))) char sB[2][2][NB][kWave * 16];  // [parity][hi/lo][frag]
-  const int H = a.H;
-  int rec, strip;
-  if (!xcd_strip_coords(a.num_seqs * H, VS, rec, strip)) return;
-  const int seq = rec / H, h = rec % H;
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, lr = lane % 16, kg = lane / 16;
-  const int n = seq_entry(a, seq).y;
-  const int nseg = (n + seg_len - 1) / seg_len;
-  if (nseg <= 1) return;
-  const int v = 16 * strip + lr;
-  f32x4 S[TPW];
-#pragma unroll
-  for (int t = 0; t < TPW; ++t) {
-    const int kt = wave * TPW + t;
-    if (a.s0) {
-      const float4 x = *(const float4*)(a.s0 + (((size_t)seq * H + h) * V + v) * K + 16 * kt + 4 * kg);
-      S[t][0] = x.x; S[t][1] = x.y; S[t][2] = x.z; S[t][3] = x.w;
-    } else {
-      S[t] = zero4();
-    }
-  }
-  const bf16* P0 = (const bf16*)a.ws.p[R_SEGP] + (size_t)rec * max_segs * K * K;
-  const float* G0 = (const float*)a.ws.p[R_SEGS] + (size_t)rec * max_segs * V * K + (size_t)v * K;
-  // every step's P rows and Sigma for this wave, requested up front in batches of
-  // kCombBatch steps (one memory round trip per batch instead of one per step)
-  bf16x8 pa[kCombBatch][TPW][NB];
-  float4 sg[kCombBatch][TPW];
-  for (int j = 0; j + 1 < nseg; ++j) {
-    const int jb = j % kCombBatch;
-    if (jb == 0) {
-#pragma unroll
-      for (int b = 0; b < kCombBatch; ++b) {
-        const int jj = min(j + b, nseg - 2);
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) {
-          const int kt = wave * TPW + t;
-#pragma unroll
-          for (int s = 0; s < NB; ++s)
-            pa[b][t][s] = *(const bf16x8*)(P0 + (size_t)jj * K * K + (((size_t)kt * NB + s) * 64 + lane) * 8);
-          sg[b][t] = *(const float4*)(G0 + (size_t)jj * V * K + 16 * kt + 4 * kg);
-        }
-      }
-    }
-    char(*buf)[NB][kWave * 16] = sB[j & 1];
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      const int kt = wave * TPW + t;
-      bf16x4 hi, lo;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        hi[r] = to_bf16(S[t][r]);
-        lo[r] = to_bf16(S[t][r] - to_f32(hi[r]));
-      }
-      *(bf16x4*)(buf[0][kt / 2] + lane * 16 + (kt % 2) * 8) = hi;
-      *(bf16x4*)(buf[1][kt / 2] + lane * 16 + (kt % 2) * 8) = lo;
-    }
-    // LDS only: a fence-free barrier (the prefetched loads and earlier stores stay in flight)
-    wait_lgkm0();
-    ring_barrier();
-    bf16x8 Bh[NB], Bl[NB];
-#pragma unroll
-    for (int s = 0; s < NB; ++s) {
-      Bh[s] = *(const bf16x8*)(buf[0][s] + lane * 16);
-      Bl[s] = *(const bf16x8*)(buf[1][s] + lane * 16);
-    }
-    // pick this step's operands (jb is uniform; unrolled select keeps them in registers)
-    bf16x8 pc[TPW][NB];
-    float4 gc[TPW];
-#pragma unroll
-    for (int b = 0; b < kCombBatch; ++b)
-      if (b == jb) {
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) {
-          gc[t] = sg[b][t];
-#pragma unroll
-          for (int s = 0; s < NB; ++s) pc[t][s] = pa[b][t][s];
-        }
-      }
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      f32x4 acc;
-      acc[0] = gc[t].x; acc[1] = gc[t].y; acc[2] = gc[t].z; acc[3] = gc[t].w;
-#pragma unroll
-      for (int s = 0; s < NB; ++s) {
-        acc = mfma16(pc[t][s], Bh[s], acc);
-        acc = mfma16(pc[t][s], Bl[s], acc);
-      }
-      S[t] = acc;
-    }
-    float* out = (float*)a.ws.p[R_SIN] + ((size_t)rec * max_segs + j + 1) * V * K + (size_t)v * K;
-#pragma unroll
-    for (int t = 0; t < TPW; ++t)
-      *(float4*)(out + 16 * (wave * TPW + t) + 4 * kg) = make_float4(S[t][0], S[t][1], S[t][2], S[t][3]);
-  }
-}
-
 // ---------------------------------------------------------------------------
 // output:  O = Qg S + A delta  (chunk-parallel, after the scan)
 // ---------------------------------------------------------------------------
@@ -1649,9 +1543,19 @@ static int launch_forward(const kda_chunk_problem* p, const ChunkGeom& g, FwdArg
       hipLaunchKernelGGL(local, dim3(kXcds * CL::GROUPS * ((nrs + kXcds - 1) / kXcds)), dim3(kSegThreads),
                          CL::bytes, stream, a, g.seg_len, g.max_segs);
       KDA_LAUNCH_CHECK("chunk_forward segment maps");
-      auto comb = chunk_fwd_combine_kernel<K, V>;
-      hipLaunchKernelGGL(comb, dim3(kXcds * (V / 16) * ((nrec + kXcds - 1) / kXcds)), dim3(kCombThreads), 0, stream,
-                         a, g.seg_len, g.max_segs);
+      CombineArgs c;
+      c.H = a.H;
+      c.num_seqs = a.num_seqs;
+      c.fixed_T = a.fixed_T;
+      c.seg_len = g.seg_len;
+      c.max_segs = g.max_segs;
+      c.seqs = (const int2*)a.ws.p[R_SEQS];
+      c.start = a.s0;
+      c.P = (const bf16*)a.ws.p[R_SEGP];
+      c.sigma = (const float*)a.ws.p[R_SEGS];
+      c.out = (float*)a.ws.p[R_SIN];
+      auto comb = seg_combine_kernel<K, V, false>;
+      hipLaunchKernelGGL(comb, dim3(kXcds * (V / 16) * ((nrec + kXcds - 1) / kXcds)), dim3(kCombThreads), 0, stream, c);
       KDA_LAUNCH_CHECK("chunk_forward segment combine");
       hipLaunchKernelGGL(replay, dim3(kXcds * CR::GROUPS * ((nrs + kXcds - 1) / kXcds)), dim3(kSegThreads),
                          CR::bytes, stream, a, g.seg_len, g.max_segs);

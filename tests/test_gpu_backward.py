@@ -427,3 +427,23 @@ def test_gate_parameter_sums(T, H, K):
     assert ((ddt.double().view(H, K) - dz.sum(0)).abs() <= bound * dz.square().sum(0).sqrt() + 1e-12).all()
     t = dz * pre
     assert ((dA.double() - t.sum((0, 2))).abs() <= bound * t.square().sum((0, 2)).sqrt() + 1e-12).all()
+
+
+@pytest.mark.parametrize("lens,H,KV,gate", [([6400], 3, (128, 128), "precomputed"),        # 10 whole segments of 10 chunks
+                                             ([5000, 0, 1300, 100], 1, (64, 64), "k3"),     # none, 2 segments, part of one
+                                             ([3001, 3500], 1, (64, 128), "precomputed"),
+                                             ([8192], 2, (128, 64), "k3")])
+def test_segmented_reverse_scan(lens, H, KV, gate):
+    """From 96 chunks on with few strips the reverse scan runs in segments (maps, combine,
+    replay): whole and partial last segments, sequences of one segment and of none, packed
+    and not, an initial state and a final-state gradient, every head size, against the
+    float64 oracle."""
+    K, V = KV
+    T, n = sum(lens), len(lens)
+    d = make_kda_inputs(1, T, H, K, V, seed=T, gate=gate, state=True, dist="baseline")
+    cu = None
+    if n > 1:
+        cu = torch.tensor(np.cumsum([0] + lens), dtype=torch.int32, device="cuda")
+        d["s0"] = torch.randn(n, H, V, K, generator=torch.Generator().manual_seed(3)).cuda() * 0.05
+    do, dsT = cotangents(d, 11, n_states=n)
+    check(gpu_grads(d, gate, do, dsT, cu), oracle_grads(d, gate, do, dsT, cu))
