@@ -755,29 +755,95 @@ int generic_backward(const kda_chunk_problem* p, const void* q, const void* k, c
 // live behind the chunked workspace, so the backward reads the same padded inputs.
 // ---------------------------------------------------------------------------
 
-// dst[t][h][c] = c < w_src ? src[t][h][c] : 0 for c < w_dst, rows of H heads; token strides
-// ld_src / ld_dst (elements), head strides w_src / w_dst.  One wave per (token, head) row.
-template <typename T>
-__global__ __launch_bounds__(256) void pad_rows_kernel(int nrows, int H, int w_src, long ld_src, int w_dst,
-                                                       long ld_dst, const T* __restrict__ src, T* __restrict__ dst) {
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  for (int r = blockIdx.x * 4 + wave; r < nrows; r += gridDim.x * 4) {
-    const int t = r / H, h = r - t * H;
-    const T* s = src + (size_t)t * ld_src + (size_t)h * w_src;
-    T* d = dst + (size_t)t * ld_dst + (size_t)h * w_dst;
-    for (int c = lane; c < w_dst; c += kWave) d[c] = c < w_src ? s[c] : T(0.f);
+// dst[t][h][c] = h < h_src and c < w_src ? src[t][h][c] : 0 for h < h_dst, c < w_dst: zero-padded
+// copies and the slices back out, as bytes (zero is zero in every type).  All copies of a side
+// of a call are the jobs of one launch, each moved in the widest units its pointers, strides
+// and widths allow.  Bound by memory at ~15 MB a launch; as a launch per tensor with one wave
+// per row of 2-byte accesses, and 6 waves for the 6 states' tails, the copies took 180 of the
+// 304 us of a forward + backward at B2 T1999 H3, K = V = 96 with states; now 24.
+struct PadJob {
+  const char* src;
+  char* dst;
+  long ld_src, ld_dst;  // bytes between tokens
+  int rows;             // tokens x h_dst
+  int h_src, h_dst, w_src, w_dst;  // heads; bytes per head
+  int unit;             // bytes per access
+  int first_block;
+};
+constexpr int kMaxPadJobs = 6, kPadThreads = 256;
+struct PadJobs {
+  PadJob job[kMaxPadJobs];
+  int n = 0, blocks = 0;
+};
+
+__host__ __device__ inline int pad_lanes(const PadJob& j) {  // lanes per row: a power of two
+  int l = 1;
+  while (l < kWave && l * j.unit < j.w_dst) l *= 2;
+  return l;
+}
+constexpr int kPadRowsPerLaneGroup = 4;
+
+template <typename U>
+__device__ __forceinline__ void pad_rows(const PadJob& j, int block) {
+  const int lanes = pad_lanes(j), groups = kPadThreads / lanes;
+  const int c0 = (threadIdx.x % lanes) * (int)sizeof(U);
+  const long r0 = (long)block * groups * kPadRowsPerLaneGroup + threadIdx.x / lanes;
+#pragma unroll
+  for (int q = 0; q < kPadRowsPerLaneGroup; ++q) {
+    const long r = r0 + (long)q * groups;
+    if (r >= j.rows) return;
+    const int t = (int)r / j.h_dst, h = (int)r - t * j.h_dst;
+    const char* s = j.src + t * j.ld_src + (long)h * j.w_src;
+    char* d = j.dst + t * j.ld_dst + (long)h * j.w_dst;
+    for (int c = c0; c < j.w_dst; c += lanes * (int)sizeof(U))
+      *(U*)(d + c) = h < j.h_src && c < j.w_src ? *(const U*)(s + c) : U{};
   }
 }
 
-template <typename T>
-static int pad_rows(long nrows, int H, int w_src, long ld_src, int w_dst, long ld_dst, const void* src, void* dst,
-                    hipStream_t stream) {
-  if (nrows <= 0) return KDA_OK;
-  KDA_REQUIRE(nrows < (1L << 31), "padded KDA: too many rows");
-  const long blocks = (nrows + 3) / 4;
-  hipLaunchKernelGGL(pad_rows_kernel<T>, dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(256), 0, stream,
-                     (int)nrows, H, w_src, ld_src, w_dst, ld_dst, (const T*)src, (T*)dst);
-  KDA_LAUNCH_CHECK("padded KDA copy");
+__global__ __launch_bounds__(kPadThreads) void pad_rows_kernel(PadJobs js) {
+  int n = 0;
+  while (n + 1 < js.n && (int)blockIdx.x >= js.job[n + 1].first_block) ++n;
+  const PadJob& j = js.job[n];
+  const int block = blockIdx.x - j.first_block;
+  if (j.unit == 16)
+    pad_rows<uint4>(j, block);
+  else if (j.unit == 8)
+    pad_rows<uint2>(j, block);
+  else if (j.unit == 4)
+    pad_rows<unsigned>(j, block);
+  else
+    pad_rows<unsigned short>(j, block);
+}
+
+// Adds the copy of `tokens` x h_dst rows; strides in elements of `size` bytes.
+static int add_pad(PadJobs& js, long tokens, int h_src, int h_dst, int size, int w_src, long ld_src, int w_dst,
+                   long ld_dst, const void* src, void* dst) {
+  if (tokens * h_dst <= 0) return KDA_OK;
+  KDA_REQUIRE(tokens * h_dst < (1L << 31), "padded KDA: too many rows");
+  PadJob j;
+  j.src = (const char*)src;
+  j.dst = (char*)dst;
+  j.ld_src = ld_src * size;
+  j.ld_dst = ld_dst * size;
+  j.rows = (int)(tokens * h_dst);
+  j.h_src = h_src;
+  j.h_dst = h_dst;
+  j.w_src = w_src * size;
+  j.w_dst = w_dst * size;
+  const uintptr_t all = (uintptr_t)src | (uintptr_t)dst | (uintptr_t)j.ld_src | (uintptr_t)j.ld_dst |
+                        (uintptr_t)j.w_src | (uintptr_t)j.w_dst;
+  j.unit = all % 16 == 0 ? 16 : all % 8 == 0 ? 8 : all % 4 == 0 ? 4 : 2;
+  j.first_block = js.blocks;
+  const long per = (long)kPadThreads / pad_lanes(j) * kPadRowsPerLaneGroup;
+  js.blocks += (int)((j.rows + per - 1) / per);
+  js.job[js.n++] = j;
+  return KDA_OK;
+}
+
+static int launch_pads(const PadJobs& js, hipStream_t stream) {
+  if (js.n == 0) return KDA_OK;
+  hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)js.blocks), dim3(kPadThreads), 0, stream, js);
+  KDA_LAUNCH_CHECK("padded KDA copies");
   return KDA_OK;
 }
 
@@ -849,33 +915,29 @@ int padded_forward(const kda_chunk_problem* p, const void* q, const void* k, con
   padded_ws_layout(p, off);
   char* w = (char*)workspace;
   const int K = p->key_dim, V = p->value_dim, Kp = pp.key_dim, Vp = pp.value_dim, H = p->heads;
-  const long toks = (long)p->batch * p->seq_len, nst = (long)p->num_seqs * H * V;
+  const long toks = (long)p->batch * p->seq_len, nst = (long)p->num_seqs * H;
   const bool k3 = p->gate_mode == KDA_GATE_K3;
-  KDA_TRY(pad_rows<bf16>(toks * H, H, K, (long)H * K, Kp, (long)H * Kp, q, w + off[PW_Q], stream));
-  KDA_TRY(pad_rows<bf16>(toks * H, H, K, (long)H * K, Kp, (long)H * Kp, k, w + off[PW_K], stream));
-  KDA_TRY(pad_rows<bf16>(toks * H, H, V, (long)H * V, Vp, (long)H * Vp, v, w + off[PW_V], stream));
-  if (k3) {
-    KDA_TRY(pad_rows<bf16>(toks * H, H, K, (long)H * K, Kp, (long)H * Kp, gate, w + off[PW_G], stream));
-    KDA_TRY(pad_rows<float>(H, H, K, (long)H * K, Kp, (long)H * Kp, dt_bias, w + off[PW_DT], stream));
-  } else {
-    KDA_TRY(pad_rows<float>(toks * H, H, K, (long)H * K, Kp, (long)H * Kp, gate, w + off[PW_G], stream));
-  }
+  PadJobs in, out;
+  KDA_TRY(add_pad(in, toks, H, H, 2, K, (long)H * K, Kp, (long)H * Kp, q, w + off[PW_Q]));
+  KDA_TRY(add_pad(in, toks, H, H, 2, K, (long)H * K, Kp, (long)H * Kp, k, w + off[PW_K]));
+  KDA_TRY(add_pad(in, toks, H, H, 2, V, (long)H * V, Vp, (long)H * Vp, v, w + off[PW_V]));
+  KDA_TRY(add_pad(in, toks, H, H, k3 ? 2 : 4, K, (long)H * K, Kp, (long)H * Kp, gate, w + off[PW_G]));
+  if (k3) KDA_TRY(add_pad(in, 1, H, H, 4, K, (long)H * K, Kp, (long)H * Kp, dt_bias, w + off[PW_DT]));
   float* s0p = nullptr;
   if (initial_state) {
-    // [N][H][V][K] -> [N][H][Vp][Kp]: rows (n, h, v) padded to Kp, then the Vp - V zero rows
+    // [N][H][V][K] -> [N][H][Vp][Kp]
     s0p = (float*)(w + off[PW_S0]);
-    KDA_TRY(pad_rows<float>((long)p->num_seqs * H, 1, V * K, (long)V * K, Vp * Kp, (long)Vp * Kp, initial_state,
-                            s0p, stream));  // zero tail of each (n, h) block
-    KDA_TRY(pad_rows<float>(nst, V, K, (long)V * K, Kp, (long)Vp * Kp, initial_state, s0p, stream));
+    KDA_TRY(add_pad(in, nst, V, Vp, 4, K, (long)V * K, Kp, (long)Vp * Kp, initial_state, s0p));
   }
+  KDA_TRY(launch_pads(in, stream));
   float* sfp = final_state ? (float*)(w + off[PW_SFIN]) : nullptr;
   bf16* outp = (bf16*)(w + off[PW_OUT]);
   KDA_TRY(kda_chunk_forward(&pp, w + off[PW_Q], w + off[PW_K], w + off[PW_V], w + off[PW_G], beta_logits, A_log,
                             k3 ? (const float*)(w + off[PW_DT]) : dt_bias, s0p, outp, sfp, w + off[PW_FAST],
                             stream));
-  KDA_TRY(pad_rows<bf16>(toks * H, H, Vp, (long)H * Vp, V, (long)H * V, outp, output, stream));
-  if (final_state) KDA_TRY(pad_rows<float>(nst, V, Kp, (long)Vp * Kp, K, (long)V * K, sfp, final_state, stream));
-  return KDA_OK;
+  KDA_TRY(add_pad(out, toks, H, H, 2, Vp, (long)H * Vp, V, (long)H * V, outp, output));
+  if (final_state) KDA_TRY(add_pad(out, nst, Vp, V, 4, Kp, (long)Vp * Kp, K, (long)V * K, sfp, final_state));
+  return launch_pads(out, stream);
 }
 
 int padded_backward(const kda_chunk_problem* p, const void* beta_logits, const float* A_log, const void* workspace,
@@ -889,35 +951,31 @@ int padded_backward(const kda_chunk_problem* p, const void* beta_logits, const f
   const char* w = (const char*)workspace;
   char* sc = (char*)scratch;
   const int K = p->key_dim, V = p->value_dim, Kp = pp.key_dim, Vp = pp.value_dim, H = p->heads;
-  const long toks = (long)p->batch * p->seq_len, nst = (long)p->num_seqs * H * V;
+  const long toks = (long)p->batch * p->seq_len, nst = (long)p->num_seqs * H;
   const bool k3 = p->gate_mode == KDA_GATE_K3;
   const long gld_qk = p->grad_row_stride > 0 ? p->grad_row_stride : (long)H * K;
   const long gld_v = p->grad_row_stride > 0 ? p->grad_row_stride : (long)H * V;
-  KDA_TRY(pad_rows<bf16>(toks * H, H, V, (long)H * V, Vp, (long)H * Vp, grad_output, sc + so[PS_DO], stream));
+  PadJobs in, out;
+  KDA_TRY(add_pad(in, toks, H, H, 2, V, (long)H * V, Vp, (long)H * Vp, grad_output, sc + so[PS_DO]));
   float* dsfp = nullptr;
   if (grad_final_state) {
     dsfp = (float*)(sc + so[PS_DSF]);
-    KDA_TRY(pad_rows<float>((long)p->num_seqs * H, 1, V * K, (long)V * K, Vp * Kp, (long)Vp * Kp,
-                            grad_final_state, dsfp, stream));
-    KDA_TRY(pad_rows<float>(nst, V, K, (long)V * K, Kp, (long)Vp * Kp, grad_final_state, dsfp, stream));
+    KDA_TRY(add_pad(in, nst, V, Vp, 4, K, (long)V * K, Kp, (long)Vp * Kp, grad_final_state, dsfp));
   }
+  KDA_TRY(launch_pads(in, stream));
   float* ds0p = dinitial_state ? (float*)(sc + so[PS_DS0]) : nullptr;
   KDA_TRY(kda_chunk_backward(&pp, w + wo[PW_Q], w + wo[PW_K], w + wo[PW_V], w + wo[PW_G], beta_logits, A_log,
                              k3 ? (const float*)(w + wo[PW_DT]) : nullptr, nullptr, w + wo[PW_FAST],
                              sc + so[PS_DO], dsfp, sc + so[PS_DQ], sc + so[PS_DK], sc + so[PS_DV],
                              sc + so[PS_DG], dbeta_logits, dA_log, k3 ? (float*)(sc + so[PS_DDT]) : nullptr,
                              ds0p, sc + so[PS_FAST], stream));
-  KDA_TRY(pad_rows<bf16>(toks * H, H, Kp, (long)H * Kp, K, gld_qk, sc + so[PS_DQ], dq, stream));
-  KDA_TRY(pad_rows<bf16>(toks * H, H, Kp, (long)H * Kp, K, gld_qk, sc + so[PS_DK], dk, stream));
-  KDA_TRY(pad_rows<bf16>(toks * H, H, Vp, (long)H * Vp, V, gld_v, sc + so[PS_DV], dv, stream));
-  if (k3) {
-    KDA_TRY(pad_rows<bf16>(toks * H, H, Kp, (long)H * Kp, K, (long)H * K, sc + so[PS_DG], dgate, stream));
-    KDA_TRY(pad_rows<float>(H, H, Kp, (long)H * Kp, K, (long)H * K, sc + so[PS_DDT], ddt_bias, stream));
-  } else {
-    KDA_TRY(pad_rows<float>(toks * H, H, Kp, (long)H * Kp, K, (long)H * K, sc + so[PS_DG], dgate, stream));
-  }
-  if (dinitial_state) KDA_TRY(pad_rows<float>(nst, V, Kp, (long)Vp * Kp, K, (long)V * K, ds0p, dinitial_state, stream));
-  return KDA_OK;
+  KDA_TRY(add_pad(out, toks, H, H, 2, Kp, (long)H * Kp, K, gld_qk, sc + so[PS_DQ], dq));
+  KDA_TRY(add_pad(out, toks, H, H, 2, Kp, (long)H * Kp, K, gld_qk, sc + so[PS_DK], dk));
+  KDA_TRY(add_pad(out, toks, H, H, 2, Vp, (long)H * Vp, V, gld_v, sc + so[PS_DV], dv));
+  KDA_TRY(add_pad(out, toks, H, H, k3 ? 2 : 4, Kp, (long)H * Kp, K, (long)H * K, sc + so[PS_DG], dgate));
+  if (k3) KDA_TRY(add_pad(out, 1, H, H, 4, Kp, (long)H * Kp, K, (long)H * K, sc + so[PS_DDT], ddt_bias));
+  if (dinitial_state) KDA_TRY(add_pad(out, nst, Vp, V, 4, Kp, (long)Vp * Kp, K, (long)V * K, ds0p, dinitial_state));
+  return launch_pads(out, stream);
 }
 
 int padded_status(const kda_chunk_problem* p, const void* scratch, hipStream_t stream) {

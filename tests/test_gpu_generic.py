@@ -227,3 +227,33 @@ def test_generic_kv_cache_decode_matches_full_forward():
         for t in range(P, T):
             step = model(idx[:, t:t + 1], kv_cache=cache)
             assert rel_err(step[:, 0], full[:, t]) < 2e-2, t
+
+
+@pytest.mark.parametrize("T,KV", [(1, (96, 96)), (63, (40, 72)), (517, (96, 96)), (130, (7, 5)), (64, (100, 33))])
+@pytest.mark.parametrize("gate", ["k3", "precomputed"])
+def test_padded_copies_equal_padded_inputs(T, KV, gate):
+    """The zero-padded route's copies (16-, 8-, 4- and 2-byte accesses by divisibility; rows of
+    every job's last block; states with padded rows) against the same call on inputs padded by
+    hand to 64 / 128: the same kernels on the same values, so outputs, states and gradients are
+    equal bit for bit."""
+    K, V = KV
+    Kp, Vp = (64 if K <= 64 else 128), (64 if V <= 64 else 128)
+    d = make_kda_inputs(2, T, 3, K, V, seed=T + K + V, gate=gate, state=True, dist="baseline")
+    pad = lambda t, w: torch.nn.functional.pad(t, (0, w - t.shape[-1]))  # noqa: E731
+    p = dict(d, q=pad(d["q"], Kp), k=pad(d["k"], Kp), v=pad(d["v"], Vp), g=pad(d["g"], Kp),
+             dt_bias=pad(d["dt_bias"].view(3, K), Kp).reshape(-1),
+             s0=torch.nn.functional.pad(d["s0"], (0, Kp - K, 0, Vp - V)))
+    do, dsT = cotangents(d, 4)
+    res = []
+    for x, xo, xs in ((d, do, dsT), (p, pad(do, Vp), torch.nn.functional.pad(dsT, (0, Kp - K, 0, Vp - V)))):
+        a = (x["q"], x["k"], x["v"], x["g"], x["beta"], x["A_log"], x["dt_bias"], x["s0"])
+        out, fin, ws = ops.chunk_forward(*a, True, -5.0, K ** -0.5, gate=gate)
+        res.append((out, fin, *ops.chunk_backward(*a, ws, xo.contiguous(), xs.contiguous(), -5.0, K ** -0.5, gate=gate)))
+    for i, (x, y) in enumerate(zip(*res)):
+        if x is None:
+            continue
+        if i == 8:  # ddt_bias [H K]
+            y = y.view(3, Kp)[:, :K].reshape(-1)
+        elif x.shape != y.shape:
+            y = y[tuple(slice(0, n) for n in x.shape)]
+        assert torch.equal(x, y), i
