@@ -159,6 +159,10 @@ def kernel_times(torch, t, do, gate, reps=20):
             call = lambda: lib.kda_chunk_backward_stage(stage, ctypes.byref(p), *bargs)  # noqa: E731
         _lib.check(call(), name)
         torch.cuda.synchronize()
+        if stage is None:  # as a captured step runs it (an eager call uses separate launches)
+            res[name] = graph_time_us(torch, lambda: lib.kda_chunk_backward(
+                ctypes.byref(p), *bargs[:-1], torch.cuda.current_stream().cuda_stream), n=reps) / 1e3
+            continue
         s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         s.record()
         for _ in range(reps):

@@ -282,6 +282,8 @@ __device__ __forceinline__ void bwd_prep_body(const BwdArgs& a, int cidx, int h)
 template <int K, int V>
 __global__ __launch_bounds__(kPrepThreads) void chunk_bwd_prep_kernel(BwdArgs a, int sched_words) {
   const int cidx = blockIdx.x, h = blockIdx.y;
+  // no wait of this call can fail: kda_chunk_backward_status finds a clear flag
+  if (cidx == 0 && h == 0 && threadIdx.x == 0) ((int*)a.sc.p[S_SYNC])[1] = 0;
   if (sched_words > 0 && cidx == (int)gridDim.x - 1) {
     // one extra column of workgroups: (x = last, y = 0) does the fused launch's scheduling
     // (sync words, tile order), saving a launch of its own
@@ -2083,12 +2085,29 @@ static bool fused_backward_enabled() {
 // launches cannot fail in a wait, so their callers need not read the failure flag.  With
 // K V <= 64^2 a tile is half as long and the lines lie lower: 70 / 73 us at 384 tiles x 24
 // strips, but 50 / 41 at 128 x 16, 83 / 77 at 512 x 32, 192 / 182 at 1,536 x 96.
-static bool fused_backward(const ChunkGeom& g) {
+static bool fused_eligible(const ChunkGeom& g) {
   if (!fused_backward_enabled()) return false;
   const int cus = device_cu_count();
   const long tiles = (long)g.max_chunks * g.heads, strips = (long)g.num_seqs * g.heads * (g.V / 16);
   if (bwd_segments(g).len > 0) return false;
   return g.K * g.V > 64 * 64 ? tiles > cus / 4 && 8 * strips <= 3L * cus : tiles > cus && 8 * strips <= cus;
+}
+
+// A wait of the fused launch that gives up has to be reported, so its caller reads a flag back
+// and drains the stream after every call.  Only a captured call, which cannot (the NaN gradients
+// are its report), gets the fused launch; an eager one runs the separate launches, which cannot
+// fail, and the host goes on: 299 -> 199 us per eager forward + backward at B2 T4096 H3, K = V =
+// 128, although its kernels take 24 us more.  A wait limit set through
+// kda_debug_set_wait_limit asks for the launch that it bounds.
+static bool fused_backward(const ChunkGeom& g, hipStream_t stream) {
+  if (!fused_eligible(g)) return false;
+  if (g_wait_limit.load(std::memory_order_relaxed) >= 0) return true;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return st == hipStreamCaptureStatusActive;
 }
 
 template <int K, int V>
@@ -2138,7 +2157,7 @@ static int launch_backward(const kda_chunk_problem* p, const ChunkGeom& g, BwdAr
     KDA_LAUNCH_CHECK("chunk_backward prep");
     return KDA_OK;
   };
-  if ((stages & all) == all && p->num_seqs > 0 && g.max_chunks > 0 && fused_backward(g)) {
+  if ((stages & all) == all && p->num_seqs > 0 && g.max_chunks > 0 && fused_backward(g, stream)) {
     // one launch: scan members + prep workgroups + dense / decay tiles (see chunk_bwd_fused_kernel)
     constexpr size_t smem =
         cmax_sz(kFusedSPW * BwdScanLds<K, V>::bytes + 2048, TileSmem<K, V>::bytes);
@@ -2341,6 +2360,13 @@ extern "C" int kda_debug_set_wait_limit(int64_t ticks) {
   return KDA_OK;
 }
 
+extern "C" int kda_chunk_backward_waits(const kda_chunk_problem* p, hipStream_t stream) {
+  using namespace kda;
+  if (validate_problem(p, "chunk_backward_waits") != KDA_OK) return 0;
+  if (padded_route(p)) return padded_waits(p, stream);
+  return !generic_dims(p) && fused_backward(make_geom(p), stream);
+}
+
 extern "C" int kda_chunk_backward_status(const kda_chunk_problem* p, const void* scratch,
                                          hipStream_t stream) {
   using namespace kda;
@@ -2351,7 +2377,7 @@ extern "C" int kda_chunk_backward_status(const kda_chunk_problem* p, const void*
   if (padded_route(p)) return padded_status(p, scratch, stream);
   if (generic_dims(p)) return KDA_OK;  // the token-serial backward has no waits
   const ChunkGeom g = make_geom(p);
-  if (!fused_backward(g)) return KDA_OK;  // the separate launches wait on nothing inside a kernel
+  if (!fused_eligible(g)) return KDA_OK;  // the separate launches wait on nothing inside a kernel
   const Regions sc = sc_regions(g, const_cast<void*>(scratch));
   int word = 0;
   hipError_t e = hipMemcpyAsync(&word, sc.p[S_SYNC] + sizeof(int), sizeof(int), hipMemcpyDeviceToHost, stream);

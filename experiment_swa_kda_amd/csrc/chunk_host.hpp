@@ -37,6 +37,7 @@ int padded_backward(const kda_chunk_problem* p, const void* beta_logits, const f
                     void* dgate, void* dbeta_logits, float* dA_log, float* ddt_bias, float* dinitial_state,
                     void* scratch, hipStream_t stream);
 int padded_status(const kda_chunk_problem* p, const void* scratch, hipStream_t stream);
+int padded_waits(const kda_chunk_problem* p, hipStream_t stream);
 
 constexpr size_t cmax_sz(size_t x, size_t y) { return x > y ? x : y; }
 

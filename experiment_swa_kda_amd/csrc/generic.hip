@@ -983,4 +983,9 @@ int padded_status(const kda_chunk_problem* p, const void* scratch, hipStream_t s
   return kda_chunk_backward_status(&pp, scratch, stream);
 }
 
+int padded_waits(const kda_chunk_problem* p, hipStream_t stream) {
+  const kda_chunk_problem pp = padded_problem(p);
+  return kda_chunk_backward_waits(&pp, stream);
+}
+
 }  // namespace kda

@@ -272,14 +272,17 @@ def chunk_backward(q, k, v, gate_values, beta_logits, A_log, dt_bias, initial_st
     ``dbeta_out`` [B, T, H] (a column slice of wider per-token rows) receives dbeta_logits,
     and the ``dbeta_pad`` elements after each token's H values are set to zero.
 
-    Outside graph capture the call then reads the launch's failure flag (a synchronisation
-    of the stream) and raises RuntimeError if an in-kernel wait gave up; under capture the
-    NaN that such a failure writes into the gradients is the report."""
+    A launch with in-kernel waits (under graph capture, or while a wait limit is set) can
+    report that one gave up: outside capture the call reads its failure flag (a
+    synchronisation of the stream) and raises RuntimeError; under capture the NaN that such
+    a failure writes into the gradients is the report.  Other launches cannot fail this way
+    and the call does not synchronise."""
     grads, p, scratch = chunk_backward_launch(
         q, k, v, gate_values, beta_logits, A_log, dt_bias, initial_state, workspace, grad_output,
         grad_final_state, lower_bound, scale, cu_seqlens=cu_seqlens, gate=gate,
         packed_qkv_grad=packed_qkv_grad, dbeta_out=dbeta_out, dbeta_pad=dbeta_pad)
-    if not torch.cuda.is_current_stream_capturing():
+    if _lib.load().kda_chunk_backward_waits(ctypes.byref(p), _stream(scratch.device)) \
+            and not torch.cuda.is_current_stream_capturing():
         chunk_backward_status(p, scratch)
     return grads
 

@@ -166,7 +166,7 @@ int kda_chunk_backward(const kda_chunk_problem* p,
 
 /*
  * Failure report of the last kda_chunk_backward on `scratch` (the same problem and scratch
- * buffer).  The fused backward launch runs the reverse scan and the per-chunk VJP tiles in
+ * buffer).  Calls that kda_chunk_backward_waits names run one fused launch, which runs the reverse scan and the per-chunk VJP tiles in
  * one grid; a tile waits, with a bound, for the scan to finish its chunk.  A wait that gives
  * up makes the tile overwrite all of its gradients with NaN (and dA_log / ddt_bias become NaN)
  * and leaves a flag in the scratch, which this call reads: it synchronises `stream` and
@@ -178,10 +178,19 @@ int kda_chunk_backward(const kda_chunk_problem* p,
 int kda_chunk_backward_status(const kda_chunk_problem* p, const void* scratch, hipStream_t stream);
 
 /*
+ * 1 if kda_chunk_backward on `stream` would now use the fused launch with in-kernel waits:
+ * for problems it gains on, while the stream is being captured or a wait limit is set; 0 if it
+ * would use separate launches, which wait on nothing and need no failure report.  No
+ * counterpart in the reference.
+ */
+int kda_chunk_backward_waits(const kda_chunk_problem* p, hipStream_t stream);
+
+/*
  * Sets the bound of every in-kernel wait of later kda_chunk_backward launches, in ticks of
  * the 100 MHz wall clock (process-wide; negative restores the 2 s default).  For tests of
  * the failure path: a bound of 0 makes every wait that is not already satisfied give up at
- * once, and every kernel still exits normally.  No counterpart in the reference.
+ * once, and every kernel still exits normally.  While a bound is set, calls outside graph
+ * capture use the fused launch too.  No counterpart in the reference.
  */
 int kda_debug_set_wait_limit(int64_t ticks);
 

@@ -447,3 +447,43 @@ def test_segmented_reverse_scan(lens, H, KV, gate):
         d["s0"] = torch.randn(n, H, V, K, generator=torch.Generator().manual_seed(3)).cuda() * 0.05
     do, dsT = cotangents(d, 11, n_states=n)
     check(gpu_grads(d, gate, do, dsT, cu), oracle_grads(d, gate, do, dsT, cu))
+
+
+def test_captured_call_equals_eager_call():
+    """A problem of more than a round of tiles uses the fused launch under capture and the
+    separate launches outside it (kda_chunk_backward_waits); the gradients of every replay
+    equal the eager call's bit for bit, with eager work and new inputs in between."""
+    import ctypes
+    from experiment_swa_kda_amd import _lib
+    lib = _lib.load()
+    K = 128
+    d = make_kda_inputs(2, 3000, 3, K, K, seed=31, dist="baseline")  # 282 tiles
+    do, dsT = cotangents(d, 32)
+    args = lambda ws: (d["q"], d["k"], d["v"], d["g"], d["beta"], d["A_log"], d["dt_bias"], None, ws, do, dsT, -5.0,  # noqa: E731
+                       K ** -0.5)
+    fwd = lambda: ops.chunk_forward(*args(None)[:8], True, -5.0, K ** -0.5)[2]  # noqa: E731
+    p = ops._problem(d["q"], d["v"], None, ops.GATE_MODES["k3"], -5.0, K ** -0.5)
+    waits = lambda: lib.kda_chunk_backward_waits(ctypes.byref(p), torch.cuda.current_stream().cuda_stream)  # noqa: E731
+    ws = fwd()
+    eager = ops.chunk_backward(*args(ws))
+    assert waits() == 0
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ops.chunk_backward(*args(fwd()))
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert waits() == 1
+        captured, _, scratch = ops.chunk_backward_launch(*args(fwd()))
+    for i in range(3):
+        if i:
+            with torch.no_grad():
+                d["v"].copy_(torch.randn(d["v"].shape, generator=torch.Generator().manual_seed(i)).bfloat16())
+            ws = fwd()
+            eager = ops.chunk_backward(*args(ws))
+        graph.replay()
+        torch.cuda.synchronize()
+        ops.chunk_backward_status(p, scratch)
+        for j, (x, y) in enumerate(zip(eager, captured)):
+            assert x is None or torch.equal(x, y), (i, j)
