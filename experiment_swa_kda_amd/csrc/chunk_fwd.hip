@@ -53,6 +53,11 @@ struct FwdArgs {
   bf16* out;
   float* sfin;
   Regions ws;
+  // Inference: the workspace regions that only a backward reads (Kd, T, M', G and the f32 state
+  // history, 136 of the 240 KB a 64-token tile writes at K = V = 128) are not written.  The
+  // kernels are bound by that traffic on a large prompt batch: at B64 T1024 H3 intra / scan /
+  // output went 170 / 172 / 68 -> 151 / 115 / 57 us.
+  bool infer;
   // optional output RMSNorm * weight * sigmoid(gate) epilogue (all null / unused if ng_out is null)
   const bf16* ng_gate;
   long ng_gate_ld;  // elements between tokens' rows of ng_gate
@@ -528,11 +533,17 @@ __global__ __launch_bounds__(kIntraThreads, 2 * kIntraNH) void chunk_fwd_intra_k
     }
   }
   float* Gout = (float*)a.ws.p[R_G] + tile * 64 * K;
+  auto store_g = [&] {
+#pragma unroll
+    for (int s = 0; s < NSH; ++s) {
+      float* o = Gout + i * K + 32 * S(s) + 8 * kg;
+      *(float4*)o = make_float4(g[s][0], g[s][1], g[s][2], g[s][3]);
+      *(float4*)(o + 4) = make_float4(g[s][4], g[s][5], g[s][6], g[s][7]);
+    }
+  };
+  if (!a.infer) store_g();
 #pragma unroll
   for (int s = 0; s < NSH; ++s) {
-    float* o = Gout + i * K + 32 * S(s) + 8 * kg;
-    *(float4*)o = make_float4(g[s][0], g[s][1], g[s][2], g[s][3]);
-    *(float4*)(o + 4) = make_float4(g[s][4], g[s][5], g[s][6], g[s][7]);
     if (lr == 0 || i == 63) {
       float* r = sGref + (lr == 0 ? rb : 4) * K + 32 * S(s) + 8 * kg;
       *(float4*)r = make_float4(g[s][0], g[s][1], g[s][2], g[s][3]);
@@ -571,6 +582,7 @@ __global__ __launch_bounds__(kIntraThreads, 2 * kIntraNH) void chunk_fwd_intra_k
   }
   __syncthreads();  // also drains the G, RQ, RK stores: the exact diagonal path reads them back
   if (NH > 1) wide = (sWide[rb] | sWide[4 + rb]) != 0;
+  if (a.infer && wide) store_g();  // the exact diagonal block reads its rows (after more barriers)
   // wave (rb, hh) computes the pairs (ba, rb) for ba >= rb over its channel part, one pair
   // per round: part 0 stores its partial products, part 1 adds its own after the round's
   // barrier (fixed order; one pair's accumulators held at a time)
@@ -634,7 +646,7 @@ __global__ __launch_bounds__(kIntraThreads, 2 * kIntraNH) void chunk_fwd_intra_k
   for (int s = 0; s < NVH; ++s) vr2[s] = *(const bf16x8*)(a.v + rbase * V + 32 * SV(s) + 8 * kg);
   emit_frags<64, 64, kIntraThreads, true>((bf16*)a.ws.p[R_AF] + tile * 64 * 64, tid,
                                           [&](int r, int c) { return (bf16)sA[r * 65 + c]; });
-  {
+  if (!a.infer) {
     float* MPout = (float*)a.ws.p[R_MP] + tile * 64 * 64;
     for (int idx = tid; idx < 64 * 64; idx += kIntraThreads) MPout[idx] = sM[(idx / 64) * 65 + idx % 64];
   }
@@ -667,7 +679,7 @@ __global__ __launch_bounds__(kIntraThreads, 2 * kIntraNH) void chunk_fwd_intra_k
         xq[s][e] = (bf16)(qh(s, e) * __expf(g[s][e]));
         xk[s][e] = (bf16)(kh(s, e) * __expf(gl[e] - g[s][e]));
       }
-      *(bf16x8*)(KDF + frag_off(K, rb, S(s), lane)) = xk[s];
+      if (!a.infer) *(bf16x8*)(KDF + frag_off(K, rb, S(s), lane)) = xk[s];
     }
   }
   __syncthreads();
@@ -752,7 +764,7 @@ __global__ __launch_bounds__(kIntraThreads, 2 * kIntraNH) void chunk_fwd_intra_k
     }
     __syncthreads();
   }
-  {
+  if (!a.infer) {
     bf16* Tout = (bf16*)a.ws.p[R_T] + tile * 64 * 64;
     for (int idx = 4 * tid; idx < 64 * 64; idx += 4 * kIntraThreads) {
       const float* t = sT + (idx / 64) * 65 + idx % 64;
@@ -1026,7 +1038,8 @@ __global__ __launch_bounds__(kScanThreads) void chunk_fwd_scan_kernel(FwdArgs a)
     for (int j = 0; j < KPW; ++j) {
       const int kt = cw * KPW + j;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) SH[(size_t)(16 * kt + 4 * kg + r) * V] = S[j][r];
+      for (int r = 0; r < 4; ++r)
+        if (!a.infer) SH[(size_t)(16 * kt + 4 * kg + r) * V] = S[j][r];
       kf[j][0] = *(const bf16x8*)(slot + L::off_kdt + ((kt * 2) * 64 + lane) * 16);
       kf[j][1] = *(const bf16x8*)(slot + L::off_kdt + ((kt * 2 + 1) * 64 + lane) * 16);
       lamf[j] = *(const float4*)(slot + L::off_lam + (16 * kt + 4 * kg) * 4);
@@ -1250,7 +1263,8 @@ __global__ __launch_bounds__(kSegThreads) void chunk_fwd_seg_kernel(FwdArgs a, i
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) SH[(size_t)(16 * kt + 4 * kg + r) * V] = S[j][kt][r];
+          for (int r = 0; r < 4; ++r)
+            if (!a.infer) SH[(size_t)(16 * kt + 4 * kg + r) * V] = S[j][kt][r];
         bf16* SHBF = (bf16*)a.ws.p[R_SHBF] + tile * V * K + (size_t)strip[j] * 16 * K;
 #pragma unroll
         for (int s = 0; s < NB; ++s) *(bf16x8*)(SHBF + ((size_t)s * 64 + lane) * 8) = Bs[j][s];
@@ -1602,7 +1616,8 @@ static int chunk_forward_impl(int stages, const kda_chunk_problem* p, const void
                                  const void* norm_gate = nullptr, const float* norm_weight = nullptr,
                                  float norm_eps = 0.f, void* norm_output = nullptr,
                                  float* norm_inv_rms = nullptr, const void* conv_x = nullptr,
-                                 long conv_ld = 0, const void* conv_w = nullptr, int conv_W = 0) {
+                                 long conv_ld = 0, const void* conv_w = nullptr, int conv_W = 0,
+                                 bool infer = false) {
   using namespace kda;
   int rc = validate_problem(p, "chunk_forward");
   if (rc != KDA_OK) return rc;
@@ -1620,7 +1635,7 @@ static int chunk_forward_impl(int stages, const kda_chunk_problem* p, const void
                 "chunk_forward: stage entry points and fused epilogues need head dims 64 or 128");
     if (padded_route(p))
       return padded_forward(p, q, k, v, gate, beta_logits, A_log, dt_bias, initial_state, output, final_state,
-                            workspace, stream);
+                            workspace, stream, infer);
     return generic_forward(p, q, k, v, gate, beta_logits, A_log, dt_bias, initial_state, output, final_state,
                            workspace, stream);
   }
@@ -1642,6 +1657,7 @@ static int chunk_forward_impl(int stages, const kda_chunk_problem* p, const void
   a.out = (bf16*)output;
   a.sfin = final_state;
   a.ws = ws_regions(g, workspace);
+  a.infer = infer;
   a.ng_gate = (const bf16*)norm_gate;
   a.ng_gate_ld = p->norm_gate_row_stride > 0 ? p->norm_gate_row_stride : (long)p->heads * p->value_dim;
   a.beta_ld = p->beta_row_stride > 0 ? p->beta_row_stride : p->heads;
@@ -1672,6 +1688,16 @@ extern "C" int kda_chunk_forward(const kda_chunk_problem* p, const void* q, cons
                                  void* workspace, hipStream_t stream) {
   return chunk_forward_impl(~0, p, q, k, v, gate, beta_logits, A_log, dt_bias, initial_state,
                             output, final_state, workspace, stream);
+}
+
+extern "C" int kda_chunk_forward_infer(const kda_chunk_problem* p, const void* q, const void* k,
+                                       const void* v, const void* gate, const void* beta_logits,
+                                       const float* A_log, const float* dt_bias,
+                                       const float* initial_state, void* output, float* final_state,
+                                       void* workspace, hipStream_t stream) {
+  return chunk_forward_impl(~0, p, q, k, v, gate, beta_logits, A_log, dt_bias, initial_state,
+                            output, final_state, workspace, stream, nullptr, nullptr, 0.f, nullptr,
+                            nullptr, nullptr, 0, nullptr, 0, true);
 }
 
 extern "C" int kda_chunk_forward_norm_gate(const kda_chunk_problem* p, const void* q, const void* k,

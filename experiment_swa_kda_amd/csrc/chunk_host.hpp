@@ -31,7 +31,7 @@ size_t padded_ws_bytes(const kda_chunk_problem* p);
 size_t padded_sc_bytes(const kda_chunk_problem* p);
 int padded_forward(const kda_chunk_problem* p, const void* q, const void* k, const void* v, const void* gate,
                    const void* beta_logits, const float* A_log, const float* dt_bias, const float* initial_state,
-                   void* output, float* final_state, void* workspace, hipStream_t stream);
+                   void* output, float* final_state, void* workspace, hipStream_t stream, bool infer);
 int padded_backward(const kda_chunk_problem* p, const void* beta_logits, const float* A_log, const void* workspace,
                     const void* grad_output, const float* grad_final_state, void* dq, void* dk, void* dv,
                     void* dgate, void* dbeta_logits, float* dA_log, float* ddt_bias, float* dinitial_state,

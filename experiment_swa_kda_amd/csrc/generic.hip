@@ -909,7 +909,7 @@ size_t padded_sc_bytes(const kda_chunk_problem* p) {
 
 int padded_forward(const kda_chunk_problem* p, const void* q, const void* k, const void* v, const void* gate,
                    const void* beta_logits, const float* A_log, const float* dt_bias, const float* initial_state,
-                   void* output, float* final_state, void* workspace, hipStream_t stream) {
+                   void* output, float* final_state, void* workspace, hipStream_t stream, bool infer) {
   const kda_chunk_problem pp = padded_problem(p);
   size_t off[PW_END + 1];
   padded_ws_layout(p, off);
@@ -932,9 +932,9 @@ int padded_forward(const kda_chunk_problem* p, const void* q, const void* k, con
   KDA_TRY(launch_pads(in, stream));
   float* sfp = final_state ? (float*)(w + off[PW_SFIN]) : nullptr;
   bf16* outp = (bf16*)(w + off[PW_OUT]);
-  KDA_TRY(kda_chunk_forward(&pp, w + off[PW_Q], w + off[PW_K], w + off[PW_V], w + off[PW_G], beta_logits, A_log,
-                            k3 ? (const float*)(w + off[PW_DT]) : dt_bias, s0p, outp, sfp, w + off[PW_FAST],
-                            stream));
+  const auto forward = infer ? kda_chunk_forward_infer : kda_chunk_forward;
+  KDA_TRY(forward(&pp, w + off[PW_Q], w + off[PW_K], w + off[PW_V], w + off[PW_G], beta_logits, A_log,
+                  k3 ? (const float*)(w + off[PW_DT]) : dt_bias, s0p, outp, sfp, w + off[PW_FAST], stream));
   KDA_TRY(add_pad(out, toks, H, H, 2, Vp, (long)H * Vp, V, (long)H * V, outp, output));
   if (final_state) KDA_TRY(add_pad(out, nst, Vp, V, 4, Kp, (long)Vp * Kp, K, (long)V * K, sfp, final_state));
   return launch_pads(out, stream);

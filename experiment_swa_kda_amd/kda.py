@@ -344,16 +344,21 @@ def _backend_reason(q, k, v, raw_gate, beta_logits, A_log, dt_bias, initial_stat
 # autograd boundaries (reference kda.py:383-466)
 # ---------------------------------------------------------------------------
 
+def _needs_grad(*tensors):
+    """Whether autograd will record a call on these tensors (so its residuals are wanted)."""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
 class _ProjectKDAAutograd(torch.autograd.Function):
     """Chunked KDA: forward saves the residual workspace, backward runs the HIP VJP."""
 
     @staticmethod
     def forward(ctx, forward_component, backward_component, q, k, v, raw_gate, beta_logits, A_log,
                 dt_bias, initial_state, output_final_state, lower_bound, scale, cu_seqlens=None,
-                gate="k3"):
+                gate="k3", residuals=True):
         output, final_state, workspace = ops.chunk_forward(
             q, k, v, raw_gate, beta_logits, A_log, dt_bias, initial_state, output_final_state,
-            lower_bound, scale, cu_seqlens=cu_seqlens, gate=gate)
+            lower_bound, scale, cu_seqlens=cu_seqlens, gate=gate, residuals=residuals)
         ctx.backward_component = backward_component
         ctx.has_initial = initial_state is not None
         ctx.lower_bound = lower_bound
@@ -377,7 +382,7 @@ class _ProjectKDAAutograd(torch.autograd.Function):
         if not ctx.has_initial:
             dinitial = None
         return (None, None, dq, dk, dv, draw_gate, dbeta, dA, ddt, dinitial, None, None, None,
-                None, None)
+                None, None, None)
 
 
 class _ProjectRMSNormGateAutograd(torch.autograd.Function):
@@ -579,8 +584,7 @@ def kda(q, k, v, raw_gate, beta_logits, A_log, dt_bias, *, initial_state=None,
     reason = _backend_reason(q, k, v, raw_gate, beta_logits, A_log, dt_bias, initial_state,
                              lower_bound=lower_bound, gate=gate)
     requested = mode.removeprefix("project_")
-    if requested == "recurrent" and torch.is_grad_enabled() and any(
-            t is not None and t.requires_grad for t in (q, k, v, raw_gate, beta_logits, A_log, dt_bias)):
+    if requested == "recurrent" and _needs_grad(q, k, v, raw_gate, beta_logits, A_log, dt_bias):
         reason = f"{'project ' if mode.startswith('project_') else ''}recurrent KDA is inference-only"
     if reason is None and mode == "project_recurrent" and q.shape[1] != 1:
         reason = "project recurrent KDA decodes exactly one token per call"
@@ -600,7 +604,8 @@ def kda(q, k, v, raw_gate, beta_logits, A_log, dt_bias, *, initial_state=None,
     if requested == "chunk":
         output, final_state = _ProjectKDAAutograd.apply(
             "chunk_forward", "chunk_backward", q, k, v, raw_gate, beta_logits, A_log, dt_bias,
-            initial_state, output_final_state, float(lower_bound), resolved_scale, cu_seqlens, gate)
+            initial_state, output_final_state, float(lower_bound), resolved_scale, cu_seqlens, gate,
+            _needs_grad(q, k, v, raw_gate, beta_logits, A_log, dt_bias, initial_state))
         _record("chunk_forward")
         return _record_backward(output, "chunk_backward"), final_state
     if q.shape[1] == 1 and cu_seqlens is None:
@@ -613,7 +618,8 @@ def kda(q, k, v, raw_gate, beta_logits, A_log, dt_bias, *, initial_state=None,
         return output, final_state
     output, final_state, _ = ops.chunk_forward(q, k, v, raw_gate, beta_logits, A_log, dt_bias,
                                                initial_state, output_final_state, float(lower_bound),
-                                               resolved_scale, cu_seqlens=cu_seqlens, gate=gate)
+                                               resolved_scale, cu_seqlens=cu_seqlens, gate=gate,
+                                               residuals=False)
     _record("chunk_forward")
     return output, final_state
 

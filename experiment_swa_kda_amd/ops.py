@@ -119,7 +119,7 @@ def _output_bytes(B, T, H, V):
 
 def chunk_forward(q, k, v, gate_values, beta_logits, A_log, dt_bias, initial_state,
                   output_final_state, lower_bound, scale, *, cu_seqlens=None, gate="k3",
-                  residuals_behind_output=False):
+                  residuals_behind_output=False, residuals=True):
     """Chunked forward.  Returns (output, final_state or None, workspace).
 
     ``gate_values`` is the bf16 raw gate (``gate="k3"``) or the f32 log decay
@@ -128,6 +128,8 @@ def chunk_forward(q, k, v, gate_values, beta_logits, A_log, dt_bias, initial_sta
     the workspace share one allocation (output first, the workspace at the next 256-byte
     boundary), so a caller that keeps only the output keeps the residuals too: the
     ``torch.ops.nanochat_kda`` schemas pass no workspace between forward and backward.
+    Without ``residuals`` (inference) the parts of the workspace that only the backward reads
+    are left unwritten.
     """
     gm = GATE_MODES[gate]
     dev = _check_chunk_inputs("chunk_forward", q, k, v, gate_values, beta_logits, A_log, dt_bias,
@@ -152,7 +154,7 @@ def chunk_forward(q, k, v, gate_values, beta_logits, A_log, dt_bias, initial_sta
         output = torch.empty(B, T, H, V, dtype=torch.bfloat16, device=dev)
     final_state = torch.empty(n, H, V, K, dtype=torch.float32, device=dev) if output_final_state else None
     with torch.cuda.device(dev):
-        rc = lib.kda_chunk_forward(
+        rc = (lib.kda_chunk_forward if residuals else lib.kda_chunk_forward_infer)(
             ctypes.byref(p), ptr(q), ptr(k), ptr(v), ptr(gate_values), ptr(beta_logits),
             ptr(A_log), ptr(dt_bias), ptr(initial_state), ptr(output), ptr(final_state),
             ptr(workspace), _stream(dev))

@@ -98,6 +98,17 @@ int kda_chunk_forward(const kda_chunk_problem* p,
                       void* workspace, hipStream_t stream);
 
 /*
+ * kda_chunk_forward for inference: the same arguments, output and final state (bit for bit), but
+ * the workspace regions that only kda_chunk_backward reads are left unwritten.  No counterpart in
+ * the reference, whose forward always stores its residuals.
+ */
+int kda_chunk_forward_infer(const kda_chunk_problem* p,
+                            const void* q, const void* k, const void* v, const void* gate,
+                            const void* beta_logits, const float* A_log, const float* dt_bias,
+                            const float* initial_state, void* output, float* final_state,
+                            void* workspace, hipStream_t stream);
+
+/*
  * kda_chunk_forward with the mixer's output RMSNorm * weight * sigmoid(gate) fused into the
  * output kernel's epilogue (a producer/consumer fusion: the norm takes o from registers instead
  * of a second kernel reading it back from HBM).  No single counterpart in

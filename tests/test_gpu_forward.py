@@ -312,3 +312,26 @@ def test_mixer_fused_conv_equals_separate_conv():
         res.append([y, x.grad] + [p.grad.clone() for p in layer.parameters()])
     for a, b in zip(*res):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,T,H,KV,gate,scale_g", [
+    (2, 200, 3, (128, 128), "k3", 1.0), (1, 65, 2, (64, 128), "precomputed", 1.0), (3, 1, 2, (128, 64), "k3", 1.0),
+    (1, 130, 2, (64, 64), "precomputed", 40.0),      # diagonal blocks of more than 80 nats (exact path)
+    (1, 6200, 1, (128, 128), "precomputed", 1.0),    # segmented scan
+    (2, 70, 2, (96, 40), "k3", 1.0)])                # zero-padded copies
+def test_forward_without_residuals(B, T, H, KV, gate, scale_g):
+    """kda() without gradients leaves the backward's residuals unwritten: output and final
+    state equal those of the recording call bit for bit, and the gradient of a recording call
+    is not disturbed by it."""
+    from experiment_swa_kda_amd import kda
+    K, V = KV
+    d = make_kda_inputs(B, T, H, K, V, seed=T + K, gate=gate, state=True, dist="baseline")
+    d["g"] = d["g"] * scale_g
+    a = (d["q"], d["k"], d["v"], d["g"], d["beta"], d["A_log"], d["dt_bias"])
+    run = lambda *x: kda(*x, initial_state=d["s0"], output_final_state=True, mode="project_chunk", gate=gate)  # noqa: E731
+    with torch.no_grad():
+        out, fin = run(*a)
+    v = d["v"].clone().requires_grad_()
+    out2, fin2 = run(*a[:2], v, *a[3:])
+    assert torch.equal(out, out2) and torch.equal(fin, fin2) and out2.requires_grad and not out.requires_grad
+    assert torch.isfinite(torch.autograd.grad(out2.float().sum(), v)[0].float()).all()
