@@ -75,6 +75,7 @@ struct FwdArgs {
   long conv_ld;
   const bf16* conv_w;
   int conv_W;
+  bf16* conv_fin;  // [3][B][HK][W] the last W inputs of every channel (zeros before the start), or null
 };
 
 // Chunk table entry {row0, len, sequence, index}: arithmetic for sequences of one length.
@@ -422,6 +423,17 @@ __global__ __launch_bounds__(kIntraThreads, 2 * kIntraNH) void chunk_fwd_intra_k
       if (!has_halo)
 #pragma unroll
         for (int e = 0; e < 8; ++e) ho[0][s][e] = ho[1][s][e] = ho[2][s][e] = to_bf16(0.f);
+    }
+    // the convolution windows a decode continues from: the sequence's last chunk copies the
+    // last W rows of this head's q, k, v inputs
+    if (a.conv_fin != nullptr && a.fixed_T > 0 && ch.w * kChunk + len == a.fixed_T) {
+      for (int idx = tid; idx < 3 * K * W; idx += kIntraThreads) {
+        const int j = idx % W, c = (idx / W) % K, t = idx / (W * K);
+        const int p = a.fixed_T - W + j;  // token of the sequence
+        bf16 x = to_bf16(0.f);
+        if (p >= 0) x = a.conv_x[(size_t)(ch.z * a.fixed_T + p) * a.conv_ld + t * HK + h * K + c];
+        a.conv_fin[(((size_t)t * a.num_seqs + ch.z) * HK + h * K + c) * W + j] = x;
+      }
     }
     __syncthreads();  // taps staged
     bf16* qo = (bf16*)a.q + rbase * K + 8 * kg;
@@ -1435,7 +1447,7 @@ __global__ __launch_bounds__(256) void chunk_fwd_output_kernel(FwdArgs a) {
     }
   };
   __builtin_amdgcn_wave_barrier();
-  store_tile(a.out);
+  if (!ng || !a.infer) store_tile(a.out);  // (o itself is only for the norm's backward)
   if (!ng) return;
   // fused RMSNorm * weight * sigmoid(gate) over each token's V values of this head, from the
   // bf16-rounded o exactly as the standalone norm kernel reads it: a row's V values live in
@@ -1456,7 +1468,7 @@ __global__ __launch_bounds__(256) void chunk_fwd_output_kernel(FwdArgs a) {
 #pragma unroll
     for (int ct = 0; ct < V / 16; ++ct)
       so[(4 * kg + r) * OP + 16 * ct + lr] = to_bf16(ov[ct][r] * inv * w[ct] * sigmoid_fast(gv[ct][r]));
-    if (lr == 0 && t < len) a.ng_inv_rms[(size_t)(ch.x + t) * H + h] = inv;
+    if (!a.infer && lr == 0 && t < len) a.ng_inv_rms[(size_t)(ch.x + t) * H + h] = inv;
   }
   __builtin_amdgcn_wave_barrier();
   store_tile(a.ng_out);
@@ -1617,12 +1629,12 @@ static int chunk_forward_impl(int stages, const kda_chunk_problem* p, const void
                                  float norm_eps = 0.f, void* norm_output = nullptr,
                                  float* norm_inv_rms = nullptr, const void* conv_x = nullptr,
                                  long conv_ld = 0, const void* conv_w = nullptr, int conv_W = 0,
-                                 bool infer = false) {
+                                 bool infer = false, void* conv_fin = nullptr) {
   using namespace kda;
   int rc = validate_problem(p, "chunk_forward");
   if (rc != KDA_OK) return rc;
   const bool empty = (size_t)p->batch * p->seq_len == 0;
-  KDA_REQUIRE(empty || (q && k && v && gate && beta_logits && output),
+  KDA_REQUIRE(empty || (q && k && v && gate && beta_logits && (output || (infer && norm_output))),
               "chunk_forward: null input/output pointer");
   KDA_REQUIRE(aligned16(q, k, v, gate, output, initial_state, final_state),
               "chunk_forward: q, k, v, gate, output and the states must be 16-byte aligned");
@@ -1669,6 +1681,7 @@ static int chunk_forward_impl(int stages, const kda_chunk_problem* p, const void
   a.conv_ld = conv_ld;
   a.conv_w = (const bf16*)conv_w;
   a.conv_W = conv_W;
+  a.conv_fin = (bf16*)conv_fin;
   // fixed-length problems with at least one chunk get their tables from the intra kernel
   a.fixed_T = (p->cu_seqlens == nullptr && g.max_chunks > 0) ? p->seq_len : 0;
   if ((stages & (1 << KDA_STAGE_PREP)) && a.fixed_T == 0) {
@@ -1721,15 +1734,13 @@ extern "C" int kda_chunk_forward_norm_gate(const kda_chunk_problem* p, const voi
                             norm_output, inverse_rms);
 }
 
-extern "C" int kda_chunk_forward_conv_norm_gate(const kda_chunk_problem* p, const void* conv_x,
-                                                int64_t conv_ld, const void* conv_weight,
-                                                int32_t conv_width, void* q, void* k, void* v,
-                                                const void* gate, const void* beta_logits,
-                                                const float* A_log, const float* dt_bias,
-                                                void* output, void* workspace,
-                                                const void* norm_gate, const float* norm_weight,
-                                                float epsilon, void* norm_output, float* inverse_rms,
-                                                hipStream_t stream) {
+static int conv_norm_gate_impl(const kda_chunk_problem* p, const void* conv_x, int64_t conv_ld,
+                               const void* conv_weight, int32_t conv_width, void* q, void* k, void* v,
+                               const void* gate, const void* beta_logits, const float* A_log,
+                               const float* dt_bias, void* output, float* final_state, void* workspace,
+                               const void* norm_gate, const float* norm_weight, float epsilon,
+                               void* norm_output, float* inverse_rms, hipStream_t stream, bool infer,
+                               void* conv_windows) {
   using namespace kda;
   KDA_REQUIRE(p != nullptr, "chunk_forward_conv_norm_gate: null problem");
   const bool empty = (size_t)p->batch * p->seq_len == 0;
@@ -1742,12 +1753,41 @@ extern "C" int kda_chunk_forward_conv_norm_gate(const kda_chunk_problem* p, cons
   KDA_REQUIRE(conv_ld >= 3 * (int64_t)p->heads * p->key_dim && conv_ld % 8 == 0,
               "chunk_forward_conv_norm_gate: conv_ld must be a multiple of 8 and >= 3 * heads * key_dim");
   KDA_REQUIRE(aligned16(conv_x), "chunk_forward_conv_norm_gate: conv_x must be 16-byte aligned");
-  KDA_REQUIRE(empty || (norm_gate && norm_weight && norm_output && inverse_rms),
+  KDA_REQUIRE(empty || (norm_gate && norm_weight && norm_output && (inverse_rms || infer)),
               "chunk_forward_conv_norm_gate: null norm pointer");
   KDA_REQUIRE(epsilon >= 0.f, "chunk_forward_conv_norm_gate: epsilon must be non-negative");
   return chunk_forward_impl(~0, p, q, k, v, gate, beta_logits, A_log, dt_bias, nullptr, output,
-                            nullptr, workspace, stream, norm_gate, norm_weight, epsilon, norm_output,
-                            inverse_rms, empty ? nullptr : conv_x, conv_ld, conv_weight, conv_width);
+                            final_state, workspace, stream, norm_gate, norm_weight, epsilon, norm_output,
+                            inverse_rms, empty ? nullptr : conv_x, conv_ld, conv_weight, conv_width, infer,
+                            conv_windows);
+}
+
+extern "C" int kda_chunk_forward_conv_norm_gate(const kda_chunk_problem* p, const void* conv_x,
+                                                int64_t conv_ld, const void* conv_weight,
+                                                int32_t conv_width, void* q, void* k, void* v,
+                                                const void* gate, const void* beta_logits,
+                                                const float* A_log, const float* dt_bias,
+                                                void* output, void* workspace,
+                                                const void* norm_gate, const float* norm_weight,
+                                                float epsilon, void* norm_output, float* inverse_rms,
+                                                hipStream_t stream) {
+  return conv_norm_gate_impl(p, conv_x, conv_ld, conv_weight, conv_width, q, k, v, gate, beta_logits, A_log, dt_bias,
+                             output, nullptr, workspace, norm_gate, norm_weight, epsilon, norm_output, inverse_rms,
+                             stream, false, nullptr);
+}
+
+extern "C" int kda_chunk_forward_conv_norm_gate_infer(const kda_chunk_problem* p, const void* conv_x,
+                                                      int64_t conv_ld, const void* conv_weight,
+                                                      int32_t conv_width, void* q, void* k, void* v,
+                                                      const void* gate, const void* beta_logits,
+                                                      const float* A_log, const float* dt_bias,
+                                                      void* workspace, const void* norm_gate,
+                                                      const float* norm_weight, float epsilon,
+                                                      void* norm_output, float* final_state,
+                                                      void* conv_windows, hipStream_t stream) {
+  return conv_norm_gate_impl(p, conv_x, conv_ld, conv_weight, conv_width, q, k, v, gate, beta_logits, A_log, dt_bias,
+                             nullptr, final_state, workspace, norm_gate, norm_weight, epsilon, norm_output, nullptr,
+                             stream, true, conv_windows);
 }
 
 extern "C" int kda_chunk_forward_stage(int32_t stage, const kda_chunk_problem* p, const void* q,

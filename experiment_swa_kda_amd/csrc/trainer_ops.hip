@@ -288,6 +288,27 @@ __global__ __launch_bounds__(256) void rms_norm_bwd_kernel(long rows, const bf16
   }
 }
 
+// f32 weights as bf16, several of them end to end in one pass (a source of null: zeros).  A
+// mixer's call casts its ten weights; as a concatenation and a cast per matrix they were up to
+// 11 launches of 2-6 us for a few megabytes.
+constexpr int kMaxCasts = 16;
+struct CastArgs {
+  const float* src[kMaxCasts];
+  long end[kMaxCasts];  // running element counts, multiples of 8
+  int n;
+};
+
+__global__ __launch_bounds__(kGlueThreads) void cast_weights_kernel(CastArgs a, bf16* __restrict__ dst) {
+  const long i = ((long)blockIdx.x * kGlueThreads + threadIdx.x) * 8;
+  if (i >= a.end[a.n - 1]) return;
+  int s = 0;
+  while (i >= a.end[s]) ++s;
+  const float* src = a.src[s];
+  float f[8] = {};
+  if (src) load8f(src + (i - (s ? a.end[s - 1] : 0)), f);
+  *reinterpret_cast<bf16x8*>(dst + i) = pack8(f);
+}
+
 }  // namespace kda
 
 #define KDA_GLUE_CHECK(n, ...)                                                              \
@@ -567,3 +588,24 @@ extern "C" int kda_embedding_backward(int64_t n_tokens, int32_t vocab, int32_t d
   return KDA_OK;
 }
 
+extern "C" int kda_cast_weights_bf16(int32_t n, const float* const* src, const int64_t* counts, void* dst,
+                                     hipStream_t stream) {
+  using namespace kda;
+  KDA_REQUIRE(n >= 1 && n <= kMaxCasts && src && counts, "cast_weights_bf16: 1 to %d weights", kMaxCasts);
+  CastArgs a;
+  a.n = n;
+  long total = 0;
+  for (int s = 0; s < n; ++s) {
+    KDA_REQUIRE(counts[s] >= 0 && counts[s] % 8 == 0, "cast_weights_bf16: counts must be multiples of 8");
+    KDA_REQUIRE(aligned16(src[s]), "cast_weights_bf16: weights must be 16-byte aligned");
+    a.src[s] = src[s];
+    a.end[s] = total += counts[s];
+  }
+  if (total == 0) return KDA_OK;
+  KDA_REQUIRE(dst && aligned16(dst), "cast_weights_bf16: dst must be non-null and 16-byte aligned");
+  const long blocks = (total / 8 + kGlueThreads - 1) / kGlueThreads;
+  KDA_REQUIRE(blocks < (1L << 31), "cast_weights_bf16: too many elements");
+  hipLaunchKernelGGL(cast_weights_kernel, dim3((unsigned)blocks), dim3(kGlueThreads), 0, stream, a, (bf16*)dst);
+  KDA_LAUNCH_CHECK("cast_weights_bf16");
+  return KDA_OK;
+}

@@ -142,9 +142,10 @@ class Linear(nn.Linear):
     """nn.Linear whose parameters stay f32 while the product runs in the input's dtype
     (bf16 on the GPU: the weight is cast per call and its gradient comes back in f32)."""
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, w16: torch.Tensor | None = None) -> torch.Tensor:
+        """``w16``: the weight already cast to bf16 by the caller, for a bf16 input."""
         if x.is_cuda and x.dtype == torch.bfloat16 and self.weight.dtype == torch.float32:
-            return _LinearBF16.apply(x, self.weight, self.bias, getattr(self, "_w16", None))
+            return _LinearBF16.apply(x, self.weight, self.bias, getattr(self, "_w16", None) if w16 is None else w16)
         bias = None if self.bias is None else self.bias.to(dtype=x.dtype)
         return F.linear(x, self.weight.to(dtype=x.dtype), bias)
 
@@ -200,6 +201,7 @@ _COMPONENTS = {
     "chunk_forward_norm_gate": ("kda_chunk_forward_norm_gate", "chunk_fwd.hip"),
     "chunk_forward_conv_norm_gate": ("kda_chunk_forward_conv_norm_gate", "chunk_fwd.hip"),
     "recurrent_decode": ("kda_recurrent_decode", "decode.hip"),
+    "mixer_step": ("kda_mixer_step", "decode.hip"),
     "causal_convolution_forward": ("kda_causal_conv_forward", "conv.hip"),
     "causal_convolution_backward": ("kda_causal_conv_backward", "conv.hip"),
     "rmsnorm_gate_forward": ("kda_rmsnorm_gate_forward", "norm_gate.hip"),
@@ -742,6 +744,8 @@ class KimiDeltaAttention(nn.Module):
         fallback = self.allow_fallback if allow_fallback is None else allow_fallback
         if state is None and not output_final_state and self._batched_ok(hidden_states, mode):
             return self._forward_batched(hidden_states, mode, fallback), None
+        if self._inference_ok(hidden_states, state, mode):
+            return self._forward_inference(hidden_states, state, output_final_state, state_in_place)
         return self._forward_stepwise(hidden_states, state, output_final_state, mode, fallback,
                                       state_in_place)
 
@@ -775,6 +779,92 @@ class KimiDeltaAttention(nn.Module):
         if not keep_state:
             return y, None
         return y, KDAState(memory, branches["q"][1], branches["k"][1], branches["v"][1])
+
+    def _inference_ok(self, x, state, mode):
+        """Whether a call runs the fused inference path: a prompt without a carried state
+        (chunk modes) or one token with one (recurrent modes), nothing for autograd or a
+        transform to record, and the layouts the kernels take.  Everything else, errors
+        included, is the general path's."""
+        n_b, n_t, C = x.shape
+        H, D = self.num_heads, self.head_dim
+        prompt = state is None and mode in ("project_chunk", "chunk") and n_t > 0
+        token = isinstance(state, KDAState) and mode in ("project_recurrent", "recurrent") and n_t == 1
+        if not (prompt or token) or n_b == 0 or not x.is_cuda or x.dtype != torch.bfloat16:
+            return False
+        if D not in (64, 128) or self.conv_size != 4 or not -5.0 <= self.lower_bound < 0.0:
+            return False
+        linears = (self.q_proj, self.k_proj, self.v_proj, self.g_proj, self.f_a_proj, self.b_proj, self.f_b_proj,
+                   self.o_proj)
+        if any(type(m) is not Linear or m.bias is not None for m in linears):
+            return False
+        params = [m.weight for m in (*linears, self.q_conv1d, self.k_conv1d, self.v_conv1d, self.o_norm)]
+        params += [self.A_log, self.dt_bias]
+        if any(p.dtype != torch.float32 or p.device != x.device or not p.is_contiguous() or p.data_ptr() % 16
+               for p in params):
+            return False
+        carried = () if prompt else (state.memory, state.q_conv, state.k_conv, state.v_conv)
+        for t, shape, dtype in zip(carried, ((n_b, H, D, D),) + ((n_b, C, 4),) * 3,
+                                   (torch.float32,) + (torch.bfloat16,) * 3):
+            if t.shape != shape or t.dtype != dtype or t.device != x.device or not t.is_contiguous() \
+                    or t.data_ptr() % 16:
+                return False
+        if _needs_grad(x, *params, *carried):
+            return False
+        # forward-mode tangents and functorch transforms: the general path's autograd functions
+        # are what accepts or refuses them
+        return torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+
+    def _weights16(self):
+        """(stacked input projection, stacked convolution taps, f_b, o_proj) in bf16: the copies
+        GPT.cache_bf16_weights keeps, or one cast of the current f32 weights."""
+        cached = (getattr(self, "_w16_in", None), getattr(self, "_conv_w16", None),
+                  getattr(self.f_b_proj, "_w16", None), getattr(self.o_proj, "_w16", None))
+        if all(w is not None for w in cached):
+            return cached
+        w_in = self._in_weights()
+        d = self.hidden_size
+        rows = 4 * d + self.head_dim + self.num_heads + self._in_pad()
+        groups = ((*w_in, None), (self.q_conv1d.weight, self.k_conv1d.weight, self.v_conv1d.weight),
+                  (self.f_b_proj.weight,), (self.o_proj.weight,))
+        weights = [w for g in groups for w in g]
+        counts = [self._in_pad() * d if w is None else w.numel() for w in weights]
+        arena = ops.cast_weights_bf16(weights, counts)
+        parts = torch.split(arena, [rows * d, 3 * d * self.conv_size, d * self.head_dim, d * d])
+        return (parts[0].view(rows, d), parts[1].view(3 * d, self.conv_size), parts[2].view(d, self.head_dim),
+                parts[3].view(d, d))
+
+    def _cast_ok(self):
+        """Whether _weights16 can cast: f32 weights of multiples of 8 elements, as laid out."""
+        ws = (*self._in_weights(), self.q_conv1d.weight, self.k_conv1d.weight, self.v_conv1d.weight,
+              self.f_b_proj.weight, self.o_proj.weight)
+        return type(self.o_proj) is Linear and self.hidden_size % 8 == 0 and all(
+            w.dtype == torch.float32 and w.is_contiguous() and w.numel() % 8 == 0 and w.data_ptr() % 16 == 0 for w in ws)
+
+    def _forward_inference(self, x, state, keep_state, state_in_place):
+        """A prompt (state None) or one token: the six projections of x as one GEMM, f_b, and one
+        call for everything up to the output projection (for a prompt the convolution, the chunk
+        forward and the gated norm; for a token all of them and f_b in one kernel)."""
+        n_b, n_t, C = x.shape
+        H, D = self.num_heads, self.head_dim
+        w_in, conv16, fb16, o16 = self._weights16()
+        y = F.linear(x, w_in)
+        if state is None:
+            raw_gate = F.linear(y[..., 4 * C:4 * C + D], fb16).view(n_b, n_t, H, D)
+            out, memory, windows = ops.chunk_forward_conv_norm_gate(
+                y[..., :3 * C], conv16, raw_gate, y[..., 4 * C + D:4 * C + D + H], self.A_log, self.dt_bias,
+                float(self.lower_bound), float(D ** -0.5), y[..., 3 * C:4 * C].view(n_b, n_t, H, D),
+                self.o_norm.weight, float(self.o_norm.eps), H, infer=True)
+            _record("chunk_forward_conv_norm_gate")
+        else:
+            out, memory, windows = ops.mixer_step(
+                y.view(n_b, -1), conv16, (state.q_conv, state.k_conv, state.v_conv), fb16, self.A_log, self.dt_bias,
+                self.o_norm.weight, state.memory, H, float(self.lower_bound), float(D ** -0.5),
+                float(self.o_norm.eps), out_memory=state.memory if state_in_place and keep_state else None)
+            _record("mixer_step")
+        out = self.o_proj(out.view(n_b, n_t, C), w16=o16)
+        if not keep_state:
+            return out, None
+        return out, KDAState(memory, windows[0], windows[1], windows[2])
 
     def _gated_norm(self, o, gate, mode):
         """RMSNorm(o)·sigmoid(gate): the HIP kernel pair whenever its dtypes and head size fit,
@@ -811,7 +901,9 @@ class KimiDeltaAttention(nn.Module):
         H, D = self.num_heads, self.head_dim
         # zero rows pad the output width to a multiple of 8 (16-byte rows for the kernels)
         pad = self._in_pad()
-        y = _StackedLinearBF16.apply(hidden_states, getattr(self, "_w16_in", None), pad, *self._in_weights())
+        w_in, conv16, fb16, o16 = self._weights16() if self._cast_ok() else \
+            (getattr(self, "_w16_in", None), getattr(self, "_conv_w16", None), getattr(self.f_b_proj, "_w16", None), None)
+        y = _StackedLinearBF16.apply(hidden_states, w_in, pad, *self._in_weights())
         convs = (self.q_conv1d.weight, self.k_conv1d.weight, self.v_conv1d.weight)
         if D in (64, 128) and convs[0].shape[-1] <= 4 and self.o_norm.weight.dtype == torch.float32 \
                 and self.fuse_conv and self.f_b_proj.weight.dtype == torch.float32 \
@@ -819,12 +911,11 @@ class KimiDeltaAttention(nn.Module):
             # the column blocks of y read in place; convolution in the chunk forward's first
             # kernel, output norm in its last
             mixed = _ProjectMixerCore.apply(
-                y, getattr(self, "_conv_w16", None), self.f_b_proj.weight, getattr(self.f_b_proj, "_w16", None),
-                self.A_log, self.dt_bias, self.o_norm.weight, float(self.o_norm.eps), float(self.lower_bound),
-                float(D ** -0.5), H, *convs)
+                y, conv16, self.f_b_proj.weight, fb16, self.A_log, self.dt_bias, self.o_norm.weight,
+                float(self.o_norm.eps), float(self.lower_bound), float(D ** -0.5), H, *convs)
             _record("chunk_forward_conv_norm_gate")
-            mixed = _record_backward(mixed, "chunk_backward")
-            return self.o_proj(mixed.reshape(batch, length, C))
+            mixed = _record_backward(mixed, "chunk_backward").reshape(batch, length, C)
+            return self.o_proj(mixed) if o16 is None else self.o_proj(mixed, w16=o16)
         conv_w = torch.cat(convs, dim=0).squeeze(1).to(torch.bfloat16)
         qkv_in, gate_lin, fa, beta_logits, _ = _SplitColumns.apply(y, (3 * C, C, D, H, pad))
         raw_gate = self.f_b_proj(fa).view(batch, length, H, D)

@@ -375,24 +375,25 @@ class Block(nn.Module):
     def forward(self, x, kv_cache=None):
         """nanochat/gpt.py:180-205 for a KDA layer: with a cache, the layer's state is read
         from and written back to it, and a one-token step runs the recurrent decode kernel."""
+        x = x + self._mix(norm(x), kv_cache)
+        return x + self.mlp(norm(x))
+
+    def _mix(self, h, kv_cache):
         state = None if kv_cache is None else kv_cache.get_kda_state(self.attn.layer_idx)
         mode = None
-        if x.is_cuda and self.attn.mode.startswith("project_"):
-            mode = "project_recurrent" if kv_cache is not None and x.shape[1] == 1 else "project_chunk"
-        mixed, state = self.attn(norm(x), state=state, output_final_state=kv_cache is not None, mode=mode,
+        if h.is_cuda and self.attn.mode.startswith("project_"):
+            mode = "project_recurrent" if kv_cache is not None and h.shape[1] == 1 else "project_chunk"
+        mixed, state = self.attn(h, state=state, output_final_state=kv_cache is not None, mode=mode,
                                  state_in_place=kv_cache is not None and kv_cache.inplace_state)
         if kv_cache is not None:
             kv_cache.set_kda_state(self.attn.layer_idx, state)
-        x = x + mixed
-        return x + self.mlp(norm(x))
+        return mixed
 
-    def forward_mixed(self, x, x0, lam_r, lam_0, i):
-        """The training path of ``block(resid_mix(x, x0, lam_r, lam_0, i))`` (no cache) with
-        the residual mix fused into the first norm and the residual add into the second;
-        the same values."""
+    def forward_mixed(self, x, x0, lam_r, lam_0, i, kv_cache=None):
+        """``block(resid_mix(x, x0, lam_r, lam_0, i), kv_cache)`` with the residual mix fused
+        into the first norm and the residual add into the second; the same values."""
         xin, h = _ResidMixNorm.apply(x, x0, lam_r, lam_0, i, _RMS_EPS)
-        mode = "project_chunk" if self.attn.mode.startswith("project_") else None
-        mixed, _ = self.attn(h, state=None, output_final_state=False, mode=mode)
+        mixed = self._mix(h, kv_cache)
         y, h2 = _AddNorm.apply(xin, mixed, _RMS_EPS)
         return y + self.mlp(h2)
 
@@ -507,10 +508,10 @@ class GPT(nn.Module):
         x = x0 = self._smear(x, before)
         mid = self.config.n_layer // 2
         mid_out = None
-        fused = kv_cache is None and _norm_fusable(x) and x0.shape == x.shape
+        fused = _norm_fusable(x) and x0.shape == x.shape
         for i, block in enumerate(self.transformer.h):
             if fused:
-                x = block.forward_mixed(x, x0, self.resid_lambdas, self.x0_lambdas, i)
+                x = block.forward_mixed(x, x0, self.resid_lambdas, self.x0_lambdas, i, kv_cache)
             else:
                 x = block(resid_mix(x, x0, self.resid_lambdas, self.x0_lambdas, i).to(torch.bfloat16), kv_cache)
             mid_out = x if i == mid else mid_out

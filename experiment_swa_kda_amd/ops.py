@@ -202,14 +202,16 @@ def chunk_forward_norm_gate(q, k, v, gate_values, beta_logits, A_log, dt_bias, i
 
 
 def chunk_forward_conv_norm_gate(qkv_in, conv_weight, gate_values, beta_logits, A_log, dt_bias,
-                                 lower_bound, scale, norm_gate, norm_weight, eps, heads, *, gate="k3"):
+                                 lower_bound, scale, norm_gate, norm_weight, eps, heads, *, gate="k3",
+                                 infer=False):
     """:func:`chunk_forward_norm_gate` with the short convolution + SiLU of q, k, v computed
     by the chunk forward's first kernel (stateless path: no convolution or recurrent state).
     ``qkv_in`` [B,T,3HK] bf16 holds the pre-convolution q, k, v projections side by side; it
     may be a column slice of a wider row (unit channel stride, row stride a multiple of 8).
     ``conv_weight`` [3HK, W] bf16, W <= 4.  Returns (q, k, v, o, normed, inverse_rms,
     workspace) with q, k, v the post-SiLU activations [B,T,H,K], bit-identical to
-    :func:`causal_conv_forward`'s."""
+    :func:`causal_conv_forward`'s; with ``infer`` (a prompt at inference) (normed, final state
+    [B,H,V,K], convolution windows [3,B,HK,W]) and nothing for a backward."""
     gm = GATE_MODES[gate]
     what = "chunk_forward_conv_norm_gate"
     dev = _require_cuda(what, qkv_in, conv_weight, gate_values, beta_logits, A_log, dt_bias, norm_gate,
@@ -251,8 +253,19 @@ def chunk_forward_conv_norm_gate(qkv_in, conv_weight, gate_values, beta_logits, 
     if ws_bytes == 0 and B * T > 0:
         check(1, "chunk_workspace_bytes")
     workspace = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
-    output = torch.empty(B, T, H, D, dtype=torch.bfloat16, device=dev)
-    normed = torch.empty_like(output)
+    normed = torch.empty(B, T, H, D, dtype=torch.bfloat16, device=dev)
+    if infer:
+        W = int(conv_weight.shape[1])
+        final_state = torch.empty(B, H, D, D, dtype=torch.float32, device=dev)
+        windows = torch.empty(3, B, H * D, W, dtype=torch.bfloat16, device=dev)
+        with torch.cuda.device(dev):
+            rc = lib.kda_chunk_forward_conv_norm_gate_infer(
+                ctypes.byref(p), ptr(qkv_in), int(ld), ptr(conv_weight), W, ptr(q), ptr(k), ptr(v),
+                ptr(gate_values), ptr(beta_logits), ptr(A_log), ptr(dt_bias), ptr(workspace), ptr(norm_gate),
+                ptr(norm_weight), float(eps), ptr(normed), ptr(final_state), ptr(windows), _stream(dev))
+        check(rc, "kda_chunk_forward_conv_norm_gate_infer")
+        return normed, final_state, windows
+    output = torch.empty_like(normed)
     inv = torch.empty(B * T * H, dtype=torch.float32, device=dev)
     with torch.cuda.device(dev):
         rc = lib.kda_chunk_forward_conv_norm_gate(
@@ -399,6 +412,58 @@ def recurrent_decode(q, k, v, gate_values, beta_logits, A_log, dt_bias, initial_
                                       ptr(final_state), _stream(dev))
     check(rc, "kda_recurrent_decode")
     return output, final_state
+
+
+def mixer_step(y, conv_weight, windows, fb_weight, A_log, dt_bias, norm_weight, memory, heads, lower_bound, scale,
+               eps, *, out_memory=None):
+    """One token of the mixer between its input and output projections: ``y`` [B, N] the
+    stacked input projection's rows [q | k | v | output gate | f_a | beta | ...], ``windows``
+    the three convolution windows [B, HD, 4] (not written), ``memory`` [B,H,D,D] f32.  Returns
+    (normed output [B, HD], new memory, new windows [3, B, HD, 4]); ``out_memory`` receives the
+    new memory (it may be ``memory``)."""
+    what = "mixer_step"
+    dev = _require_cuda(what, y, conv_weight, fb_weight, A_log, dt_bias, norm_weight, memory, out_memory, *windows)
+    B, H, D = y.shape[0], int(heads), memory.shape[-1]
+    C = H * D
+    for name, t, shape in (("conv_weight", conv_weight, (3 * C, 4)), ("fb_weight", fb_weight, (C, D)),
+                           *((f"window {i}", w, (B, C, 4)) for i, w in enumerate(windows))):
+        _check_dtype(what, t, torch.bfloat16, name)
+        if tuple(t.shape) != shape or not t.is_contiguous():
+            raise RuntimeError(f"{what}: {name} must be a contiguous {shape} tensor")
+    out_memory = torch.empty_like(memory) if out_memory is None else out_memory
+    for name, t, shape in (("A_log", A_log, (H,)), ("dt_bias", dt_bias, (C,)), ("norm_weight", norm_weight, (D,)),
+                           ("memory", memory, (B, H, D, D)), ("out_memory", out_memory, (B, H, D, D))):
+        _check_dtype(what, t, torch.float32, name)
+        if tuple(t.shape) != shape or not t.is_contiguous():
+            raise RuntimeError(f"{what}: {name} must be a contiguous {shape} tensor")
+    _check_dtype(what, y, torch.bfloat16, "y")
+    if y.ndim != 2 or y.stride(1) != 1 or y.shape[1] < 4 * C + D + H:
+        raise RuntimeError(f"{what}: y must be [B, 4HD + D + H or more] rows")
+    out = torch.empty(B, C, dtype=torch.bfloat16, device=dev)
+    new_windows = torch.empty(3, B, C, 4, dtype=torch.bfloat16, device=dev)
+    with torch.cuda.device(dev):
+        rc = _lib.load().kda_mixer_step(
+            B, H, D, float(lower_bound), float(scale), float(eps), ptr(y), y.stride(0) if B > 1 else y.shape[1],
+            ptr(conv_weight), ptr(windows[0]), ptr(windows[1]), ptr(windows[2]), ptr(new_windows), ptr(fb_weight),
+            ptr(A_log), ptr(dt_bias), ptr(norm_weight), ptr(memory), ptr(out_memory), ptr(out), _stream(dev))
+    check(rc, "kda_mixer_step")
+    return out, out_memory, new_windows
+
+
+def cast_weights_bf16(weights, counts):
+    """f32 weights rounded to bf16 end to end in one tensor, one launch; ``counts[i]`` elements
+    each (a weight of None: that many zeros).  Multiples of 8, contiguous, 16-byte aligned."""
+    dev = _require_cuda("cast_weights_bf16", *weights)
+    for w, n in zip(weights, counts):
+        if w is not None and (w.dtype != torch.float32 or w.numel() != n or not w.is_contiguous()):
+            raise RuntimeError("cast_weights_bf16: contiguous f32 weights of the given counts expected")
+    out = torch.empty(sum(counts), dtype=torch.bfloat16, device=dev)
+    n = len(weights)
+    with torch.cuda.device(dev):
+        rc = _lib.load().kda_cast_weights_bf16(n, (ctypes.c_void_p * n)(*(ptr(w) for w in weights)),
+                                               (ctypes.c_int64 * n)(*counts), ptr(out), _stream(dev))
+    check(rc, "kda_cast_weights_bf16")
+    return out
 
 
 def causal_conv_forward(x, weight, initial_state, output_final_state):

@@ -226,6 +226,42 @@ int kda_chunk_backward_noalloc(const kda_chunk_problem* p,
 size_t kda_chunk_backward_noalloc_max_scratch_bytes(void);
 
 /*
+ * kda_chunk_forward_conv_norm_gate for a prompt at inference: output o, its inverse RMS and the
+ * backward's residuals are not stored; the final state (f32 [B,H,V,K] or NULL) and the
+ * convolution windows (bf16 [3][B][H*K][W]: the last W inputs of the q, k, v channels, newest
+ * last, zeros before the start; or NULL) are, as kda_mixer_step continues from them.
+ */
+int kda_chunk_forward_conv_norm_gate_infer(const kda_chunk_problem* p, const void* conv_x, int64_t conv_ld,
+                                           const void* conv_weight, int32_t conv_width, void* q, void* k, void* v,
+                                           const void* gate, const void* beta_logits, const float* A_log,
+                                           const float* dt_bias, void* workspace, const void* norm_gate,
+                                           const float* norm_weight, float epsilon, void* norm_output,
+                                           float* final_state, void* conv_windows, hipStream_t stream);
+
+/*
+ * One token of the mixer between its stacked input projection and its output projection
+ * (nanochat/mixers/kda.py:744-798 for T = 1 with a carried state): short convolutions + SiLU with
+ * their windows moved on, gate projection f_b, recurrent step, RMSNorm * weight * sigmoid(gate).
+ *   y: bf16 [B] rows of y_row_stride elements: [q | k | v | output gate | f_a | beta logits], the
+ *      pre-convolution projections (H*D each), then D and H columns
+ *   conv_weight: bf16 [3*H*D][4]; q/k/v_window: bf16 [B][H*D][4]; windows_out: bf16 [3][B][H*D][4]
+ *   fb_weight: bf16 [H*D][D]; A_log f32 [H]; dt_bias f32 [H*D]; norm_weight f32 [D]
+ *   state, state_out: f32 [B,H,D,D] V-first (may be the same); output: bf16 [B][H*D]
+ * D (head_dim) 64 or 128.
+ */
+int kda_mixer_step(int32_t batch, int32_t heads, int32_t head_dim, float lower_bound, float scale, float epsilon,
+                   const void* y, int64_t y_row_stride, const void* conv_weight, const void* q_window,
+                   const void* k_window, const void* v_window, void* windows_out, const void* fb_weight,
+                   const float* A_log, const float* dt_bias, const float* norm_weight, const float* state,
+                   float* state_out, void* output, hipStream_t stream);
+
+/*
+ * n (at most 16) f32 weights rounded to bf16 end to end into dst; a NULL source writes zeros.
+ * counts[i] elements each, multiples of 8; src and counts are host arrays, read during the call.
+ */
+int kda_cast_weights_bf16(int32_t n, const float* const* src, const int64_t* counts, void* dst, hipStream_t stream);
+
+/*
  * Runs one kernel of the chunked forward or backward on buffers that a full
  * kda_chunk_forward / kda_chunk_backward call with the same arguments has prepared, so a
  * benchmark can time that kernel alone.  No counterpart in the reference (it exists for

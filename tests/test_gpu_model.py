@@ -286,3 +286,72 @@ def test_kv_cache_prefill_expands_batch_one():
         assert torch.equal(b[r], a[0])
     with pytest.raises(ValueError):
         KVCache(1, 2, 64, 128, 2, "cuda", torch.bfloat16, mixer_types="KL")
+
+
+@pytest.mark.parametrize("B,H,D", [(1, 1, 64), (3, 2, 128), (5, 3, 64), (33, 4, 128)])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_mixer_inference_path_matches_general_path(B, H, D, in_place):
+    """The fused inference path (a prompt, then one-token steps in one kernel each) against the
+    general path, which the same calls take when autograd records them or, for the recurrent
+    steps, when a convolution window is not in the layout the kernel takes: outputs and memory
+    agree to bf16 rounding of the intermediate projections (2^-8 through three of them), the
+    windows to one bf16 rounding of a differently summed projection; a prompt shorter than the
+    window leaves zeros before its start."""
+    from experiment_swa_kda_amd import KDAState
+    torch.manual_seed(B + D)
+    C = H * D
+    layer = KimiDeltaAttention(C, H, D, mode="project_chunk", allow_fallback=False).cuda()
+    with torch.no_grad():
+        for n, p in layer.named_parameters():
+            p.copy_(torch.randn(p.shape, device="cuda") * (0.3 if p.ndim < 2 or "conv" in n else C ** -0.5))
+        layer.o_norm.weight.add_(1.0)
+    strided = lambda st: KDAState(st.memory.clone(), *(torch.stack([w, w], -1)[..., 0]  # noqa: E731
+                                                       for w in (st.q_conv, st.k_conv, st.v_conv)))
+    for T in (2, 70):
+        x = torch.randn(B, T + 3, C, device="cuda").bfloat16()
+        reset_project_runtime_events()
+        with torch.no_grad():
+            y, st = layer(x[:, :T], output_final_state=True)
+        assert {e["component"] for e in project_runtime_events()} == {"chunk_forward_conv_norm_gate"}
+        y2, st2 = layer(x[:, :T].clone().requires_grad_(), output_final_state=True)
+        assert rel_err(y, y2) < 1.2e-2 and rel_err(st.memory, st2.memory) < 1.2e-2
+        for name in ("q_conv", "k_conv", "v_conv"):
+            assert rel_err(getattr(st, name), getattr(st2, name)) < 4e-3
+            assert T > 2 or not getattr(st, name)[..., :2].any()
+        for t in range(T, T + 3):
+            ref = strided(st)
+            before = st.memory.clone()
+            kept = st
+            reset_project_runtime_events()
+            with torch.no_grad():
+                y, st = layer(x[:, t:t + 1], state=st, output_final_state=True, mode="project_recurrent",
+                              state_in_place=in_place)
+                assert {e["component"] for e in project_runtime_events()} == {"mixer_step"}
+                y2, ref = layer(x[:, t:t + 1], state=ref, output_final_state=True, mode="project_recurrent")
+            assert (st.memory.data_ptr() == kept.memory.data_ptr()) == in_place
+            assert in_place or torch.equal(kept.memory, before)
+            assert rel_err(y, y2) < 1.2e-2 and rel_err(st.memory, ref.memory) < 1.2e-2
+            for name in ("q_conv", "k_conv", "v_conv"):
+                assert rel_err(getattr(st, name), getattr(ref, name)) < 4e-3
+                assert torch.equal(getattr(st, name)[..., :3], getattr(kept, name)[..., 1:])
+
+
+def test_recurrent_mode_with_gradients_is_still_refused():
+    layer = KimiDeltaAttention(128, 2, 64, mode="project_chunk", allow_fallback=False).cuda()
+    x = torch.randn(1, 3, 128, device="cuda").bfloat16()
+    with torch.no_grad():
+        _, st = layer(x, output_final_state=True)
+    with pytest.raises(RuntimeError, match="inference-only"):
+        layer(x[:, :1], state=st, mode="project_recurrent")
+    layer.lower_bound = -6.0
+    with torch.no_grad(), pytest.raises(RuntimeError, match="lower_bound"):
+        layer(x[:, :1], state=st, mode="project_recurrent")
+
+
+@pytest.mark.parametrize("counts", [(8,), (8, 16, 2048, 8), (24, 4096, 8 * 777)])
+def test_cast_weights(counts):
+    from experiment_swa_kda_amd import ops
+    g = torch.Generator().manual_seed(sum(counts))
+    ws = [torch.randn(n, generator=g).cuda() if i != 1 else None for i, n in enumerate(counts)]
+    out = ops.cast_weights_bf16(ws, list(counts))
+    assert torch.equal(out, torch.cat([torch.zeros(n).cuda() if w is None else w for w, n in zip(ws, counts)]).bfloat16())
