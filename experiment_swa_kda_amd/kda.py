@@ -67,6 +67,17 @@ def _mm_f32(a, b):
         return (a @ b).float()
 
 
+def _needs_grad(*tensors):
+    """Whether autograd will record a call on these tensors (so its residuals are wanted)."""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
+def _untransformed():
+    """No forward-mode level and no functorch transform is active: the autograd functions are
+    what accepts or refuses those, so paths without one ask first."""
+    return torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+
+
 class _LinearBF16(torch.autograd.Function):
     """y = x W^T with an f32 master weight cast to bf16; the weight gradient comes from the
     split-contraction HIP kernel straight in f32 (nanochat/gpt.py:52-57)."""
@@ -145,9 +156,29 @@ class Linear(nn.Linear):
     def forward(self, x: torch.Tensor, w16: torch.Tensor | None = None) -> torch.Tensor:
         """``w16``: the weight already cast to bf16 by the caller, for a bf16 input."""
         if x.is_cuda and x.dtype == torch.bfloat16 and self.weight.dtype == torch.float32:
-            return _LinearBF16.apply(x, self.weight, self.bias, getattr(self, "_w16", None) if w16 is None else w16)
+            w16 = getattr(self, "_w16", None) if w16 is None else w16
+            if self._few_rows_ok(x):
+                w16 = self.weight.to(torch.bfloat16) if w16 is None else w16
+                if ops.linear_rows_gains(x, w16):
+                    return ops.linear_rows(x, w16)
+            return _LinearBF16.apply(x, self.weight, self.bias, w16)
         bias = None if self.bias is None else self.bias.to(dtype=x.dtype)
         return F.linear(x, self.weight.to(dtype=x.dtype), bias)
+
+    def _few_rows_ok(self, x):
+        return (x.numel() <= 64 * self.in_features and self.bias is None and not _needs_grad(x, self.weight)
+                and _untransformed() and self.weight.device == x.device)
+
+    def few_rows(self, x, *, relu2=False, residual=None):
+        """``relu(y)^2`` or ``residual + y`` of y = self(x) in one kernel, for the few rows of a
+        decode step; None where that kernel does not apply (or a hook wants to see y)."""
+        w16 = getattr(self, "_w16", None)
+        if (w16 is None or not x.is_cuda or x.dtype != torch.bfloat16 or self._forward_hooks or self._forward_pre_hooks
+                or not self._few_rows_ok(x) or not ops.linear_rows_gains(x, w16)):
+            return None
+        if residual is not None and (residual.dtype != x.dtype or _needs_grad(residual)):
+            return None
+        return ops.linear_rows(x, w16, relu2=relu2, residual=residual)
 
 
 def _norm_gate_eager(x, gate, weight, eps):
@@ -345,11 +376,6 @@ def _backend_reason(q, k, v, raw_gate, beta_logits, A_log, dt_bias, initial_stat
 # ---------------------------------------------------------------------------
 # autograd boundaries (reference kda.py:383-466)
 # ---------------------------------------------------------------------------
-
-def _needs_grad(*tensors):
-    """Whether autograd will record a call on these tensors (so its residuals are wanted)."""
-    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
-
 
 class _ProjectKDAAutograd(torch.autograd.Function):
     """Chunked KDA: forward saves the residual workspace, backward runs the HIP VJP."""
@@ -797,8 +823,12 @@ class KimiDeltaAttention(nn.Module):
                    self.o_proj)
         if any(type(m) is not Linear or m.bias is not None for m in linears):
             return False
-        params = [m.weight for m in (*linears, self.q_conv1d, self.k_conv1d, self.v_conv1d, self.o_norm)]
-        params += [self.A_log, self.dt_bias]
+        params = [self.o_norm.weight, self.A_log, self.dt_bias]
+        cached = self._cached16()
+        if cached is None or torch.is_grad_enabled():
+            params += [m.weight for m in (*linears, self.q_conv1d, self.k_conv1d, self.v_conv1d)]
+        elif any(w.device != x.device for w in cached):
+            return False
         if any(p.dtype != torch.float32 or p.device != x.device or not p.is_contiguous() or p.data_ptr() % 16
                for p in params):
             return False
@@ -810,16 +840,18 @@ class KimiDeltaAttention(nn.Module):
                 return False
         if _needs_grad(x, *params, *carried):
             return False
-        # forward-mode tangents and functorch transforms: the general path's autograd functions
-        # are what accepts or refuses them
-        return torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+        return _untransformed()
+
+    def _cached16(self):
+        cached = (getattr(self, "_w16_in", None), getattr(self, "_conv_w16", None),
+                  getattr(self.f_b_proj, "_w16", None), getattr(self.o_proj, "_w16", None))
+        return cached if all(w is not None for w in cached) else None
 
     def _weights16(self):
         """(stacked input projection, stacked convolution taps, f_b, o_proj) in bf16: the copies
         GPT.cache_bf16_weights keeps, or one cast of the current f32 weights."""
-        cached = (getattr(self, "_w16_in", None), getattr(self, "_conv_w16", None),
-                  getattr(self.f_b_proj, "_w16", None), getattr(self.o_proj, "_w16", None))
-        if all(w is not None for w in cached):
+        cached = self._cached16()
+        if cached is not None:
             return cached
         w_in = self._in_weights()
         d = self.hidden_size
@@ -847,7 +879,7 @@ class KimiDeltaAttention(nn.Module):
         n_b, n_t, C = x.shape
         H, D = self.num_heads, self.head_dim
         w_in, conv16, fb16, o16 = self._weights16()
-        y = F.linear(x, w_in)
+        y = ops.linear_rows(x, w_in) if ops.linear_rows_gains(x, w_in) else F.linear(x, w_in)
         if state is None:
             raw_gate = F.linear(y[..., 4 * C:4 * C + D], fb16).view(n_b, n_t, H, D)
             out, memory, windows = ops.chunk_forward_conv_norm_gate(

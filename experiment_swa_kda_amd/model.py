@@ -361,8 +361,15 @@ class MLP(nn.Module):
         self.c_fc = Linear(d, 4 * d, bias=False)
         self.c_proj = Linear(4 * d, d, bias=False)
 
-    def forward(self, x):
-        return self.c_proj(relu2(self.c_fc(x)))
+    def forward(self, x, residual=None):
+        """The block's MLP, plus ``residual`` if given (for a decode step's few rows the
+        activation and the add run in the projections' epilogues; the same values)."""
+        h = self.c_fc.few_rows(x, relu2=True)
+        h = relu2(self.c_fc(x)) if h is None else h
+        if residual is None:
+            return self.c_proj(h)
+        y = self.c_proj.few_rows(h, residual=residual)
+        return residual + self.c_proj(h) if y is None else y
 
 
 class Block(nn.Module):
@@ -395,7 +402,7 @@ class Block(nn.Module):
         xin, h = _ResidMixNorm.apply(x, x0, lam_r, lam_0, i, _RMS_EPS)
         mixed = self._mix(h, kv_cache)
         y, h2 = _AddNorm.apply(xin, mixed, _RMS_EPS)
-        return y + self.mlp(h2)
+        return self.mlp(h2, y)
 
 
 class GPT(nn.Module):

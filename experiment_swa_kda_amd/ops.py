@@ -23,7 +23,23 @@ GATE_MODES = {"k3": KDA_GATE_K3, "precomputed": KDA_GATE_LOGDECAY}
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+class _Here:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE = _Here()
+
+
+def _on(device: torch.device):
+    """Makes ``device`` current for a launch; nothing to do (or to undo) when it already is."""
+    return _HERE if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 def _require_cuda(what: str, *tensors) -> torch.device:
@@ -153,7 +169,7 @@ def chunk_forward(q, k, v, gate_values, beta_logits, A_log, dt_bias, initial_sta
         workspace = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=dev)
         output = torch.empty(B, T, H, V, dtype=torch.bfloat16, device=dev)
     final_state = torch.empty(n, H, V, K, dtype=torch.float32, device=dev) if output_final_state else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = (lib.kda_chunk_forward if residuals else lib.kda_chunk_forward_infer)(
             ctypes.byref(p), ptr(q), ptr(k), ptr(v), ptr(gate_values), ptr(beta_logits),
             ptr(A_log), ptr(dt_bias), ptr(initial_state), ptr(output), ptr(final_state),
@@ -191,7 +207,7 @@ def chunk_forward_norm_gate(q, k, v, gate_values, beta_logits, A_log, dt_bias, i
     normed = torch.empty(B, T, H, V, dtype=torch.bfloat16, device=dev)
     inv = torch.empty(B * T * H, dtype=torch.float32, device=dev)
     final_state = torch.empty(n, H, V, K, dtype=torch.float32, device=dev) if output_final_state else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.kda_chunk_forward_norm_gate(
             ctypes.byref(p), ptr(q), ptr(k), ptr(v), ptr(gate_values), ptr(beta_logits),
             ptr(A_log), ptr(dt_bias), ptr(initial_state), ptr(output), ptr(final_state),
@@ -258,7 +274,7 @@ def chunk_forward_conv_norm_gate(qkv_in, conv_weight, gate_values, beta_logits, 
         W = int(conv_weight.shape[1])
         final_state = torch.empty(B, H, D, D, dtype=torch.float32, device=dev)
         windows = torch.empty(3, B, H * D, W, dtype=torch.bfloat16, device=dev)
-        with torch.cuda.device(dev):
+        with _on(dev):
             rc = lib.kda_chunk_forward_conv_norm_gate_infer(
                 ctypes.byref(p), ptr(qkv_in), int(ld), ptr(conv_weight), W, ptr(q), ptr(k), ptr(v),
                 ptr(gate_values), ptr(beta_logits), ptr(A_log), ptr(dt_bias), ptr(workspace), ptr(norm_gate),
@@ -267,7 +283,7 @@ def chunk_forward_conv_norm_gate(qkv_in, conv_weight, gate_values, beta_logits, 
         return normed, final_state, windows
     output = torch.empty_like(normed)
     inv = torch.empty(B * T * H, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.kda_chunk_forward_conv_norm_gate(
             ctypes.byref(p), ptr(qkv_in), int(ld), ptr(conv_weight), int(conv_weight.shape[1]),
             ptr(q), ptr(k), ptr(v), ptr(gate_values), ptr(beta_logits), ptr(A_log), ptr(dt_bias),
@@ -306,7 +322,7 @@ def chunk_backward_status(p, scratch):
     """Raise RuntimeError if the last backward on ``scratch`` (problem ``p``) reported a
     wait that gave up (kda_chunk_backward_status; synchronises the stream)."""
     lib = _lib.load()
-    with torch.cuda.device(scratch.device):
+    with _on(scratch.device):
         check(lib.kda_chunk_backward_status(ctypes.byref(p), ptr(scratch), _stream(scratch.device)),
               "kda_chunk_backward")
 
@@ -365,7 +381,7 @@ def chunk_backward_launch(q, k, v, gate_values, beta_logits, A_log, dt_bias, ini
     else:
         dA = ddt = None
     dinit = torch.empty_like(initial_state) if initial_state is not None else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.kda_chunk_backward(
             ctypes.byref(p), ptr(q), ptr(k), ptr(v), ptr(gate_values), ptr(beta_logits),
             ptr(A_log), ptr(dt_bias), ptr(initial_state), ptr(workspace), ptr(grad_output),
@@ -405,7 +421,7 @@ def recurrent_decode(q, k, v, gate_values, beta_logits, A_log, dt_bias, initial_
     elif output_final_state:
         final_state = torch.empty(B, H, V, K, dtype=torch.float32, device=dev)
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.kda_recurrent_decode(B, H, K, V, gm, float(lower_bound), float(scale), ptr(q),
                                       ptr(k), ptr(v), ptr(gate_values), ptr(beta_logits),
                                       ptr(A_log), ptr(dt_bias), ptr(initial_state), ptr(output),
@@ -441,13 +457,55 @@ def mixer_step(y, conv_weight, windows, fb_weight, A_log, dt_bias, norm_weight, 
         raise RuntimeError(f"{what}: y must be [B, 4HD + D + H or more] rows")
     out = torch.empty(B, C, dtype=torch.bfloat16, device=dev)
     new_windows = torch.empty(3, B, C, 4, dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_mixer_step(
             B, H, D, float(lower_bound), float(scale), float(eps), ptr(y), y.stride(0) if B > 1 else y.shape[1],
             ptr(conv_weight), ptr(windows[0]), ptr(windows[1]), ptr(windows[2]), ptr(new_windows), ptr(fb_weight),
             ptr(A_log), ptr(dt_bias), ptr(norm_weight), ptr(memory), ptr(out_memory), ptr(out), _stream(dev))
     check(rc, "kda_mixer_step")
     return out, out_memory, new_windows
+
+
+_LINEAR_ROWS = 64  # the most rows kda_linear_rows takes
+
+
+def linear_rows_fits(x, w16):
+    """Whether :func:`linear_rows` takes these operands (the last dimension of x against the
+    rows of w16)."""
+    K = x.shape[-1]
+    return (0 < x.numel() <= _LINEAR_ROWS * K and K % 32 == 0 and w16.shape[0] % 4 == 0 and x.is_contiguous()
+            and w16.is_contiguous() and x.data_ptr() % 16 == 0 and w16.data_ptr() % 16 == 0)
+
+
+def linear_rows_gains(x, w16):
+    """Whether :func:`linear_rows` takes these operands and beats the library GEMM on them: at 8
+    rows 2.4 / 3.9 / 6.8 us against 3.5 / 4.7 / 9.1 for weights of 2312 x 384, 384 x 1536 and
+    32768 x 384, at 64 rows 3.9 / 8.5 / 17 against 5.0 / 4.6 / 8.2 (each wave reads all rows of x
+    for its 16 outputs, so more rows only pay for short contractions of few outputs)."""
+    N, K = w16.shape
+    return linear_rows_fits(x, w16) and (x.numel() <= 16 * K or (K <= 512 and N <= 4096))
+
+
+def linear_rows(x, w16, *, relu2=False, residual=None):
+    """``x W^T`` for a few rows (bf16, f32 sums), then ``relu(.)^2`` or ``residual + .``, each
+    rounded to bf16 as the separate operations round; operands as linear_rows_fits accepts."""
+    dev = _require_cuda("linear_rows", x, w16, residual)
+    _check_dtype("linear_rows", x, torch.bfloat16, "x")
+    _check_dtype("linear_rows", w16, torch.bfloat16, "w16")
+    N, K = w16.shape
+    if x.shape[-1] != K or not linear_rows_fits(x, w16):
+        raise RuntimeError("linear_rows: x [..., K] of at most 64 rows and w16 [N, K] expected")
+    y = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=dev)
+    if residual is not None:
+        _check_dtype("linear_rows", residual, torch.bfloat16, "residual")
+        if residual.shape != y.shape or relu2:
+            raise RuntimeError("linear_rows: residual must be shaped like the result, without relu2")
+        residual = _c(residual)
+    with _on(dev):
+        rc = _lib.load().kda_linear_rows(x.numel() // K, N, K, ptr(x), K, ptr(w16), 1 if relu2 else 2 if residual is not None
+                                         else 0, ptr(residual), N, ptr(y), _stream(dev))
+    check(rc, "kda_linear_rows")
+    return y
 
 
 def cast_weights_bf16(weights, counts):
@@ -459,7 +517,7 @@ def cast_weights_bf16(weights, counts):
             raise RuntimeError("cast_weights_bf16: contiguous f32 weights of the given counts expected")
     out = torch.empty(sum(counts), dtype=torch.bfloat16, device=dev)
     n = len(weights)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_cast_weights_bf16(n, (ctypes.c_void_p * n)(*(ptr(w) for w in weights)),
                                                (ctypes.c_int64 * n)(*counts), ptr(out), _stream(dev))
     check(rc, "kda_cast_weights_bf16")
@@ -480,7 +538,7 @@ def causal_conv_forward(x, weight, initial_state, output_final_state):
         raise RuntimeError("causal_convolution_forward: initial_state must have shape [B, C, W]")
     y = torch.empty_like(x)
     fin = torch.empty(B, C, W, dtype=x.dtype, device=dev) if output_final_state else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_causal_conv_forward(B, T, C, W, ptr(x), ptr(weight), ptr(initial_state),
                                                  ptr(y), ptr(fin), _stream(dev))
     check(rc, "kda_causal_conv_forward")
@@ -548,7 +606,7 @@ def causal_conv_backward(x, weight, initial_state, grad_output, grad_final_state
     dw = torch.empty_like(weight)
     dst = torch.empty_like(initial_state) if initial_state is not None else None
     ldx, ldd = _row_stride(x), _row_stride(dx)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.kda_causal_conv_backward_strided(B, T, C, W, ptr(x), ldx, ptr(weight), ptr(initial_state),
                                                   ptr(grad_output), ptr(grad_final_state), ptr(dx), ldd,
                                                   ptr(dw), ptr(dst), ptr(scratch), _stream(dev))
@@ -569,7 +627,7 @@ def rmsnorm_gate_forward(x, gate, weight, eps):
     rows = x.numel() // D if D else 0
     y = torch.empty_like(x)
     inv = torch.empty(rows, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_rmsnorm_gate_forward(rows, D, ptr(x), ptr(gate), ptr(weight),
                                                   float(eps), ptr(y), ptr(inv), _stream(dev))
     check(rc, "kda_rmsnorm_gate_forward")
@@ -608,7 +666,7 @@ def rmsnorm_gate_backward(x, gate, weight, inv_rms, grad_output, eps, *, dgate_o
                           device=dev)
     dx = torch.empty_like(x)
     dw = torch.empty_like(weight)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.kda_rmsnorm_gate_backward_strided(rows, D, heads, ptr(x), ptr(gate), int(gld), ptr(weight),
                                                    ptr(inv_rms), ptr(grad_output), float(eps), ptr(dx),
                                                    ptr(dg), int(dgld), ptr(dw), ptr(scratch), _stream(dev))
@@ -635,7 +693,7 @@ def softcap_cross_entropy_forward(logits, targets, vocab, softcap, ignore_index=
     rows, stride = logits.shape
     loss = torch.empty(rows, dtype=torch.float32, device=dev)
     lse = torch.empty(rows, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_softcap_cross_entropy_forward(rows, int(vocab), stride, float(softcap),
                                                            ptr(logits), ptr(targets), int(ignore_index),
                                                            ptr(loss), ptr(lse), _stream(dev))
@@ -650,7 +708,7 @@ def softcap_cross_entropy_mean(loss_rows, targets, ignore_index=-1):
     _check_dtype("softcap_cross_entropy_mean", targets, torch.int64, "targets")
     loss_rows, targets = _c(loss_rows), _c(targets)
     out = torch.empty(2, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_softcap_cross_entropy_mean(loss_rows.numel(), ptr(loss_rows), ptr(targets),
                                                         int(ignore_index), ptr(out), out.data_ptr() + 4,
                                                         _stream(dev))
@@ -681,7 +739,7 @@ def softcap_cross_entropy_fused(logits, targets, vocab, softcap, ignore_index=-1
     grad = torch.empty_like(logits)
     sc = torch.empty(2, dtype=torch.float32, device=dev)  # count, grad scale
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.kda_softcap_cross_entropy_count(rows, ptr(targets), int(ignore_index), float(expected_grad),
                                                  ptr(sc), sc.data_ptr() + 4, _stream(dev))
         check(rc, "kda_softcap_cross_entropy_count")
@@ -700,7 +758,7 @@ def rescale_bf16_if_changed(data, actual, expected):
     if not data.is_contiguous():
         raise RuntimeError("rescale_bf16_if_changed: data must be contiguous")
     actual = actual.to(torch.float32).reshape(1).contiguous()
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_bf16_rescale_if_changed(data.numel(), ptr(data), ptr(actual), float(expected),
                                                      _stream(dev))
     check(rc, "kda_bf16_rescale_if_changed")
@@ -718,7 +776,7 @@ def embedding_backward(idx, grad_output, vocab):
         raise RuntimeError("embedding_backward: grad_output must be idx.shape + [dim]")
     idx, grad_output = _c(idx), _c(grad_output)
     dw = torch.empty(vocab, dim, dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_embedding_backward(idx.numel(), int(vocab), int(dim), ptr(idx), ptr(grad_output),
                                                 ptr(dw), _stream(dev))
     check(rc, "kda_embedding_backward")
@@ -732,7 +790,7 @@ def softcap_cross_entropy_backward(logits, targets, lse, grad_scale, vocab, soft
     grad_scale = grad_scale.to(torch.float32).reshape(1).contiguous()
     rows, stride = logits.shape
     grad = torch.empty_like(logits)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_softcap_cross_entropy_backward(rows, int(vocab), stride, float(softcap),
                                                             ptr(logits), ptr(targets), int(ignore_index),
                                                             ptr(lse), ptr(grad_scale), ptr(grad),
@@ -756,7 +814,7 @@ def weight_grad(grad_output, x):
     lib = _lib.load()
     scratch = torch.empty(lib.kda_weight_grad_scratch_bytes(M, N, K), dtype=torch.uint8, device=dev)
     dw = torch.empty(N, K, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.kda_weight_grad(M, N, K, ptr(grad_output), max(grad_output.stride(0), N), ptr(x),
                                  max(x.stride(0), K), ptr(dw), ptr(scratch), _stream(dev))
     check(rc, "kda_weight_grad")
@@ -778,7 +836,7 @@ def resid_mix_forward(x, x0, a, b):
     dev = _glue_check("resid_mix_forward", x, x0)
     x, x0, a, b = _c(x), _c(x0), _c(a), _c(b)
     y = torch.empty_like(x)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_resid_mix_forward(x.numel(), ptr(a), ptr(b), ptr(x), ptr(x0), ptr(y),
                                                _stream(dev))
     check(rc, "kda_resid_mix_forward")
@@ -798,7 +856,7 @@ def resid_mix_backward(x, x0, lam_a, lam_b, slot, grad):
     dx, dx0 = torch.empty_like(x), torch.empty_like(x0)
     da = torch.empty(n, dtype=torch.float32, device=dev)
     db = torch.empty(n, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.kda_resid_mix_backward(x.numel(), ptr(lam_a) + 4 * slot, ptr(lam_b) + 4 * slot, ptr(x), ptr(x0),
                                         ptr(grad), ptr(dx), ptr(dx0), ptr(da), ptr(db), slot, n, ptr(scratch),
                                         _stream(dev))
@@ -810,7 +868,7 @@ def relu2_forward(x):
     dev = _glue_check("relu2_forward", x)
     x = _c(x)
     y = torch.empty_like(x)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_relu2_forward(x.numel(), ptr(x), ptr(y), _stream(dev))
     check(rc, "kda_relu2_forward")
     return y
@@ -820,7 +878,7 @@ def relu2_backward(x, grad):
     dev = _glue_check("relu2_backward", x, grad)
     x, grad = _c(x), _c(grad)
     dx = torch.empty_like(x)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_relu2_backward(x.numel(), ptr(x), ptr(grad), ptr(dx), _stream(dev))
     check(rc, "kda_relu2_backward")
     return dx
@@ -834,7 +892,7 @@ def rms_norm_forward(x, eps):
     rows = x.numel() // D if D else 0
     y = torch.empty_like(x)
     rinv = torch.empty(rows, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_rms_norm_forward(rows, D, float(eps), ptr(x), ptr(y), ptr(rinv), _stream(dev))
     check(rc, "kda_rms_norm_forward")
     return y, rinv
@@ -851,7 +909,7 @@ def rms_norm_backward(x, rinv, grad, grad_add=None):
     D = x.shape[-1]
     rows = x.numel() // D if D else 0
     dx = torch.empty_like(x)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_rms_norm_backward_add(rows, D, ptr(x), ptr(rinv), ptr(grad), ptr(grad_add), ptr(dx),
                                                    _stream(dev))
     check(rc, "kda_rms_norm_backward")
@@ -874,7 +932,7 @@ def mix_rms_norm_forward(x, x2, eps, a=None, b=None):
     rows = x.numel() // D if D else 0
     s, y = torch.empty_like(x), torch.empty_like(x)
     rinv = torch.empty(rows, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib.load().kda_mix_rms_norm_forward(rows, D, float(eps), ptr(a), ptr(b), ptr(x), ptr(x2), ptr(s),
                                                   ptr(y), ptr(rinv), _stream(dev))
     check(rc, "kda_mix_rms_norm_forward")

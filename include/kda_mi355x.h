@@ -256,6 +256,16 @@ int kda_mixer_step(int32_t batch, int32_t heads, int32_t head_dim, float lower_b
                    float* state_out, void* output, hipStream_t stream);
 
 /*
+ * y = x W^T for at most 64 rows of x (a decode step's projections), f32 sums rounded to bf16, then
+ * epilogue 0: nothing; 1: relu(y)^2; 2: residual + y.  x bf16 [rows] of x_row_stride elements
+ * (a multiple of 8), weight bf16 [out_dim][in_dim], residual bf16 [rows] of residual_row_stride,
+ * y bf16 [rows][out_dim].  out_dim a multiple of 4, in_dim of 32.
+ */
+int kda_linear_rows(int32_t rows, int32_t out_dim, int32_t in_dim, const void* x, int64_t x_row_stride,
+                    const void* weight, int32_t epilogue, const void* residual, int64_t residual_row_stride,
+                    void* y, hipStream_t stream);
+
+/*
  * n (at most 16) f32 weights rounded to bf16 end to end into dst; a NULL source writes zeros.
  * counts[i] elements each, multiples of 8; src and counts are host arrays, read during the call.
  */

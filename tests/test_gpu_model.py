@@ -355,3 +355,28 @@ def test_cast_weights(counts):
     ws = [torch.randn(n, generator=g).cuda() if i != 1 else None for i, n in enumerate(counts)]
     out = ops.cast_weights_bf16(ws, list(counts))
     assert torch.equal(out, torch.cat([torch.zeros(n).cuda() if w is None else w for w, n in zip(ws, counts)]).bfloat16())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 4, 32), (3, 20, 96), (16, 2312, 384), (17, 384, 1536), (32, 16, 64),
+                                    (33, 1000, 1024), (64, 40, 2080)])
+def test_linear_rows(M, N, K):
+    """Rows up to every tile count, a partial tile of outputs, contractions shorter than one
+    round of a workgroup's waves and not a multiple of it, both wave counts: against float64
+    products of the same bf16 values.  One bf16 rounding (2^-9) plus f32 sums of K terms; with
+    an epilogue a second rounding, and relu^2 doubles a relative error."""
+    from experiment_swa_kda_amd import ops
+    g = torch.Generator().manual_seed(M + N + K)
+    x, w = (torch.randn(*s, generator=g).bfloat16().cuda() for s in ((M, K), (N, K)))
+    r = torch.randn(M, N, generator=g).bfloat16().cuda()
+    e = x.double() @ w.double().t()
+    tol = lambda v, n: n * 2.0 ** -8 * v.abs() + 1e-4 * K ** 0.5  # noqa: E731
+    y = ops.linear_rows(x, w)
+    assert ((y.double() - e).abs() <= tol(e, 1)).all()
+    assert torch.equal(ops.linear_rows(x, w, residual=r), r + y)
+    assert torch.equal(ops.linear_rows(x, w, relu2=True), ops.relu2_forward(y) if y.numel() % 8 == 0
+                       else torch.relu(y.float()).square().bfloat16())
+    assert torch.equal(ops.linear_rows(x[:1], w), y[:1])  # a row does not depend on the others
+    big = torch.zeros(65, K, dtype=torch.bfloat16, device="cuda")
+    assert not ops.linear_rows_fits(big, w)
+    with pytest.raises(RuntimeError):
+        ops.linear_rows(big, w)
