@@ -93,6 +93,7 @@ SIGNATURES = {
     "kda_softcap_cross_entropy_mean": (ctypes.c_int, [_L, _P, _P, _L, _P, _P, _P]),
     "kda_mfma_probe": (ctypes.c_int, [_I, _I, _I, _P, ctypes.POINTER(ctypes.c_double), _P]),
     "kda_linear_rows": (ctypes.c_int, [_I, _I, _I, _P, _L, _P, _I, _P, _L, _P, _P]),
+    "kda_norm_linear_rows": (ctypes.c_int, [_I, _I, _I, _F, _P, _P, _P, _P, _P, _I, _P, _P, _P]),
     "kda_mixer_step": (ctypes.c_int, [_I, _I, _I, _F, _F, _F, _P, _L] + [_P] * 13),
     "kda_cast_weights_bf16": (ctypes.c_int, [_I, ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_int64), _P, _P]),
     "kda_chunk_forward_conv_norm_gate_infer": (ctypes.c_int, [_PP, _P, _L, _P, _I] + [_P] * 10 + [_F] + [_P] * 4),

@@ -78,7 +78,126 @@ __global__ __launch_bounds__(WAVES * kWave) void linear_rows_kernel(int M, int N
   }
 }
 
+// The projection of a normed row with the norm in front of it: s = a x + b x2 (a = wa[0], b =
+// wb[0], 1 where null) rounded to bf16, h = rms_norm(s), y = h W^T with linear_rows' epilogues.
+// Every workgroup norms the (at most 16) rows for itself, 16 lanes a row as rms_norm_fwd_kernel
+// does, while its first fragments of W are in flight, and keeps them in LDS; workgroup 0 also
+// writes s.  At 8 rows of 384 the mix + norm launch and the projection's cost 2.3 + 2.4 us and
+// two calls of the host; this one takes 4.0 us and one call (decoder step B8: 1011 -> 814 us).
+template <int J>
+__global__ __launch_bounds__(256) void norm_linear_rows_kernel(int M, int N, float eps, int epilogue,
+                                                               const float* __restrict__ wa,
+                                                               const float* __restrict__ wb,
+                                                               const bf16* __restrict__ x,
+                                                               const bf16* __restrict__ x2,
+                                                               const bf16* __restrict__ w, bf16* __restrict__ s,
+                                                               bf16* __restrict__ y) {
+  constexpr int K = 128 * J, HP = K + 8, WAVES = 4, STEPS = K / 32, PER = STEPS / WAVES;
+  constexpr int AHEAD = PER <= 4 ? PER : PER % 4 == 0 ? 4 : 3;
+  static_assert(PER % AHEAD == 0, "whole rounds");
+  __shared__ __attribute__((aligned(16))) bf16 sh[16 * HP];
+  __shared__ f32x4 part[WAVES][kWave];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, lr = lane % 16, kg = lane / 16;
+  const int n0 = 16 * blockIdx.x;
+  const bf16* wr = w + (size_t)min(n0 + lr, N - 1) * K + 8 * kg;
+  bf16x8 fw[AHEAD];
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) fw[u] = *(const bf16x8*)(wr + 32 * (wave + u * WAVES));
+  {
+    const int row = threadIdx.x / 16, l = threadIdx.x % 16, rc = min(row, M - 1);
+    bf16x8 xv[J], zv[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      xv[j] = *(const bf16x8*)(x + (size_t)rc * K + 128 * j + 8 * l);
+      zv[j] = *(const bf16x8*)(x2 + (size_t)rc * K + 128 * j + 8 * l);
+    }
+    const float a = wa ? wa[0] : 1.f, b = wb ? wb[0] : 1.f;
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        xv[j][e] = to_bf16(fmaf(a, (float)xv[j][e], b * (float)zv[j][e]));
+        ss = fmaf((float)xv[j][e], (float)xv[j][e], ss);
+      }
+      if (blockIdx.x == 0 && row < M) *(bf16x8*)(s + (size_t)row * K + 128 * j + 8 * l) = xv[j];
+    }
+    const float r = rsqrtf(group_sum<16>(ss) / K + eps);
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      bf16x8 h;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) h[e] = to_bf16((float)xv[j][e] * r);
+      *(bf16x8*)(sh + row * HP + 128 * j + 8 * l) = h;
+    }
+  }
+  wait_lgkm0();
+  ring_barrier();  // LDS only: the loads of W stay in flight
+  f32x4 acc = zero4();
+#pragma unroll
+  for (int s0 = 0; s0 < PER; s0 += AHEAD) {
+    bf16x8 nx[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (s0 + AHEAD < PER) nx[u] = *(const bf16x8*)(wr + 32 * (wave + (s0 + AHEAD + u) * WAVES));
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      acc = mfma16(fw[u], *(const bf16x8*)(sh + lr * HP + 32 * (wave + (s0 + u) * WAVES) + 8 * kg), acc);
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (s0 + AHEAD < PER) fw[u] = nx[u];
+  }
+  part[wave][lane] = acc;
+  __syncthreads();
+  if (wave != 0) return;
+  f32x4 v = part[0][lane];
+#pragma unroll
+  for (int q = 1; q < WAVES; ++q) v += part[q][lane];
+  const int n = n0 + 4 * kg;
+  if (lr >= M || n >= N) return;
+  bf16x4 o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    o[r] = to_bf16(v[r]);
+    if (epilogue == kLinRelu2) {
+      const float p = fmaxf((float)o[r], 0.f);
+      o[r] = to_bf16(p * p);
+    }
+  }
+  *(bf16x4*)(y + (size_t)lr * N + n) = o;
+}
+
 }  // namespace kda
+
+extern "C" int kda_norm_linear_rows(int32_t rows, int32_t out_dim, int32_t in_dim, float eps, const float* a,
+                                    const float* b, const void* x, const void* x2, const void* weight,
+                                    int32_t epilogue, void* sum, void* y, hipStream_t stream) {
+  using namespace kda;
+  const int J = in_dim / 128;
+  KDA_REQUIRE(rows >= 0 && rows <= 16, "norm_linear_rows: at most 16 rows");
+  KDA_REQUIRE(in_dim > 0 && in_dim % 128 == 0 && (J <= 4 || J == 6 || J == 8),
+              "norm_linear_rows: in_dim must be 128 x {1,2,3,4,6,8}");
+  KDA_REQUIRE(out_dim > 0 && out_dim % 4 == 0, "norm_linear_rows: out_dim must be a multiple of 4");
+  KDA_REQUIRE(epilogue == kLinNone || epilogue == kLinRelu2, "norm_linear_rows: unknown epilogue");
+  if (rows == 0) return KDA_OK;
+  KDA_REQUIRE(x && x2 && weight && sum && y && aligned16(x, x2, weight, sum, y),
+              "norm_linear_rows: null or unaligned pointer");
+  const dim3 grid((unsigned)((out_dim + 15) / 16));
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, rows, out_dim, eps, epilogue, a, b, (const bf16*)x,
+                       (const bf16*)x2, (const bf16*)weight, (bf16*)sum, (bf16*)y);
+  };
+  switch (J) {
+    case 1: go(norm_linear_rows_kernel<1>); break;
+    case 2: go(norm_linear_rows_kernel<2>); break;
+    case 3: go(norm_linear_rows_kernel<3>); break;
+    case 4: go(norm_linear_rows_kernel<4>); break;
+    case 6: go(norm_linear_rows_kernel<6>); break;
+    default: go(norm_linear_rows_kernel<8>); break;
+  }
+  KDA_LAUNCH_CHECK("norm_linear_rows");
+  return KDA_OK;
+}
 
 extern "C" int kda_linear_rows(int32_t rows, int32_t out_dim, int32_t in_dim, const void* x, int64_t x_row_stride,
                                const void* weight, int32_t epilogue, const void* residual,

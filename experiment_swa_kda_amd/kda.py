@@ -887,15 +887,20 @@ class KimiDeltaAttention(nn.Module):
                 float(self.lower_bound), float(D ** -0.5), y[..., 3 * C:4 * C].view(n_b, n_t, H, D),
                 self.o_norm.weight, float(self.o_norm.eps), H, infer=True)
             _record("chunk_forward_conv_norm_gate")
+            state = KDAState(memory, windows[0], windows[1], windows[2])
         else:
-            out, memory, windows = ops.mixer_step(
-                y.view(n_b, -1), conv16, (state.q_conv, state.k_conv, state.v_conv), fb16, self.A_log, self.dt_bias,
-                self.o_norm.weight, state.memory, H, float(self.lower_bound), float(D ** -0.5),
-                float(self.o_norm.eps), out_memory=state.memory if state_in_place and keep_state else None)
-            _record("mixer_step")
-        out = self.o_proj(out.view(n_b, n_t, C), w16=o16)
-        if not keep_state:
-            return out, None
+            out, state = self._token_core(y.view(n_b, -1), state, state_in_place and keep_state)
+        return self.o_proj(out.view(n_b, n_t, C), w16=o16), state if keep_state else None
+
+    def _token_core(self, y, state, state_in_place):
+        """One token between the projections: the stacked projection's rows y [B, N] and the
+        carried state -> (normed output [B, C], new state)."""
+        _, conv16, fb16, _ = self._weights16()
+        out, memory, windows = ops.mixer_step(
+            y, conv16, (state.q_conv, state.k_conv, state.v_conv), fb16, self.A_log, self.dt_bias, self.o_norm.weight,
+            state.memory, self.num_heads, float(self.lower_bound), float(self.head_dim ** -0.5),
+            float(self.o_norm.eps), out_memory=state.memory if state_in_place else None)
+        _record("mixer_step")
         return out, KDAState(memory, windows[0], windows[1], windows[2])
 
     def _gated_norm(self, o, gate, mode):

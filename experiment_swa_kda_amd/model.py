@@ -399,10 +399,44 @@ class Block(nn.Module):
     def forward_mixed(self, x, x0, lam_r, lam_0, i, kv_cache=None):
         """``block(resid_mix(x, x0, lam_r, lam_0, i), kv_cache)`` with the residual mix fused
         into the first norm and the residual add into the second; the same values."""
+        if kv_cache is not None and self._token_ok(x, x0, lam_r, lam_0, kv_cache):
+            return self._token(x, x0, lam_r, lam_0, i, kv_cache)
         xin, h = _ResidMixNorm.apply(x, x0, lam_r, lam_0, i, _RMS_EPS)
         mixed = self._mix(h, kv_cache)
         y, h2 = _AddNorm.apply(xin, mixed, _RMS_EPS)
         return self.mlp(h2, y)
+
+
+    def _token_ok(self, x, x0, lam_r, lam_0, kv_cache):
+        """Whether a one-token step of a few sequences runs as _token: the mixer's own
+        conditions for its one-token kernel, bf16 weights cached, no module hooks."""
+        attn, mlp = self.attn, self.mlp
+        if x.shape[1] != 1 or x.shape[0] > 16 or not attn.mode.startswith("project_") or attn._cached16() is None:
+            return False
+        if type(mlp.c_fc) is not Linear or mlp.c_fc.bias is not None or type(mlp.c_proj) is not Linear \
+                or mlp.c_proj.bias is not None:
+            return False
+        w1, w2 = getattr(mlp.c_fc, "_w16", None), getattr(mlp.c_proj, "_w16", None)
+        if w1 is None or w2 is None or any(m._forward_hooks or m._forward_pre_hooks for m in (
+                attn, mlp, mlp.c_fc, mlp.c_proj, attn.o_proj)):
+            return False
+        if torch.is_grad_enabled() and any(t.requires_grad for t in (
+                x, x0, lam_r, lam_0, mlp.c_fc.weight, mlp.c_proj.weight)):
+            return False
+        return w1.device == x.device and attn._inference_ok(
+            x, kv_cache.get_kda_state(attn.layer_idx), "project_recurrent")
+
+    def _token(self, x, x0, lam_r, lam_0, i, kv_cache):
+        """forward_mixed for one token in five launches: mix + norm + input projection, mixer
+        step, output projection, add + norm + c_fc + relu^2, c_proj + add."""
+        attn, layer = self.attn, self.attn.layer_idx
+        w_in, _, _, o16 = attn._weights16()
+        s, y = ops.norm_linear_rows(x, x0, w_in, _RMS_EPS, a=lam_r, b=lam_0, slot=i)
+        out, state = attn._token_core(y.view(x.shape[0], -1), kv_cache.get_kda_state(layer), kv_cache.inplace_state)
+        kv_cache.set_kda_state(layer, state)
+        mixed = ops.linear_rows(out.view(x.shape), o16)
+        s, h = ops.norm_linear_rows(s, mixed, self.mlp.c_fc._w16, _RMS_EPS, relu2=True)
+        return ops.linear_rows(h, self.mlp.c_proj._w16, residual=s)
 
 
 class GPT(nn.Module):

@@ -508,6 +508,31 @@ def linear_rows(x, w16, *, relu2=False, residual=None):
     return y
 
 
+def norm_linear_rows(x, x2, w16, eps, *, a=None, b=None, slot=0, relu2=False):
+    """(s, rms_norm(s) W^T) of at most 16 rows, s = a[slot] x + b[slot] x2 (f32 vectors; None
+    means 1) rounded to bf16; ``relu2`` as in :func:`linear_rows`."""
+    dev = _require_cuda("norm_linear_rows", x, x2, w16, a, b)
+    for t in (x, x2, w16):
+        _check_dtype("norm_linear_rows", t, torch.bfloat16, "operand")
+    N, K = w16.shape
+    if x.shape != x2.shape or x.shape[-1] != K or x.numel() > 16 * K or not w16.is_contiguous():
+        raise RuntimeError("norm_linear_rows: x and x2 [..., K] of at most 16 rows and w16 [N, K] expected")
+    for t in (a, b):
+        if t is not None and (t.dtype != torch.float32 or t.ndim != 1 or not t.is_contiguous()
+                              or not 0 <= slot < t.numel()):
+            raise RuntimeError("norm_linear_rows: a and b must be contiguous f32 vectors with the slot inside")
+    x, x2 = _c(x), _c(x2)
+    s = torch.empty_like(x)
+    y = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=dev)
+    with _on(dev):
+        rc = _lib.load().kda_norm_linear_rows(
+            x.numel() // K, N, K, float(eps), None if a is None else a.data_ptr() + 4 * slot,
+            None if b is None else b.data_ptr() + 4 * slot, ptr(x), ptr(x2), ptr(w16), 1 if relu2 else 0, ptr(s),
+            ptr(y), _stream(dev))
+    check(rc, "kda_norm_linear_rows")
+    return s, y
+
+
 def cast_weights_bf16(weights, counts):
     """f32 weights rounded to bf16 end to end in one tensor, one launch; ``counts[i]`` elements
     each (a weight of None: that many zeros).  Multiples of 8, contiguous, 16-byte aligned."""

@@ -266,6 +266,15 @@ int kda_linear_rows(int32_t rows, int32_t out_dim, int32_t in_dim, const void* x
                     void* y, hipStream_t stream);
 
 /*
+ * kda_linear_rows of a normed residual mix, for at most 16 rows: sum = a x + b x2 (one-element f32
+ * a and b; NULL means 1) rounded to bf16, y = rms_norm(sum, eps) W^T with epilogue 0 or 1.  x, x2,
+ * sum bf16 [rows][in_dim], in_dim 128 x {1,2,3,4,6,8}; weight bf16 [out_dim][in_dim].
+ */
+int kda_norm_linear_rows(int32_t rows, int32_t out_dim, int32_t in_dim, float eps, const float* a, const float* b,
+                         const void* x, const void* x2, const void* weight, int32_t epilogue, void* sum, void* y,
+                         hipStream_t stream);
+
+/*
  * n (at most 16) f32 weights rounded to bf16 end to end into dst; a NULL source writes zeros.
  * counts[i] elements each, multiples of 8; src and counts are host arrays, read during the call.
  */

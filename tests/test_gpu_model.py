@@ -380,3 +380,49 @@ def test_linear_rows(M, N, K):
     assert not ops.linear_rows_fits(big, w)
     with pytest.raises(RuntimeError):
         ops.linear_rows(big, w)
+
+
+@pytest.mark.parametrize("M,N,J", [(1, 4, 1), (3, 20, 2), (16, 2312, 3), (5, 1536, 4), (7, 36, 6), (16, 8, 8)])
+@pytest.mark.parametrize("scalars", [False, True])
+def test_norm_linear_rows_equals_separate_kernels(M, N, J, scalars):
+    """The norm in front of a projection: the mix and the normed rows are those of the separate
+    norm kernel bit for bit, and the product differs from linear_rows' only by the order of its
+    f32 sums (one bf16 rounding, 2^-8, of a value that K terms sum to)."""
+    from experiment_swa_kda_amd import ops
+    K = 128 * J
+    g = torch.Generator().manual_seed(M + N + K)
+    x, x2, w = (torch.randn(*s, generator=g).bfloat16().cuda() for s in ((M, K), (M, K), (N, K)))
+    a, b = (torch.randn(3, generator=g).cuda() for _ in range(2)) if scalars else (None, None)
+    es, eh, _ = ops.mix_rms_norm_forward(x, x2, 1e-6, a[1:2] if scalars else None, b[1:2] if scalars else None)
+    s, y = ops.norm_linear_rows(x, x2, w, 1e-6, a=a, b=b, slot=1 if scalars else 0)
+    assert torch.equal(s, es)
+    e = eh.double() @ w.double().t()
+    assert ((y.double() - e).abs() <= 2.0 ** -8 * e.abs() + 1e-4 * K ** 0.5).all()
+    _, y2 = ops.norm_linear_rows(x, x2, w, 1e-6, a=a, b=b, slot=1 if scalars else 0, relu2=True)
+    assert torch.equal(y2, torch.relu(y.float()).square().bfloat16())
+
+
+@pytest.mark.parametrize("B", [1, 16, 17])
+def test_decode_step_with_cached_weights_matches_full_forward(B):
+    """Cached bf16 weights and at most 16 sequences: five launches per layer (17: the general
+    decode path); every step's logits equal the full-sequence forward at that position."""
+    from experiment_swa_kda_amd.model import KVCache
+    cfg = GPTConfig(sequence_len=64, vocab_size=512, n_layer=3, n_head=3, n_embd=384)
+    torch.manual_seed(0)
+    model = GPT(cfg).cuda()
+    model.init_weights()
+    with torch.no_grad():
+        for b in model.transformer.h:
+            b.attn.o_proj.weight.normal_(0, 0.02)
+            b.mlp.c_proj.weight.normal_(0, 0.02)
+        model.smear_lambda.fill_(0.4)
+    model.cache_bf16_weights()
+    g = torch.Generator(device="cuda").manual_seed(2)
+    T, P = 20, 14
+    idx = torch.randint(0, 512, (B, T), device="cuda", generator=g)
+    with torch.no_grad():
+        full = model(idx)
+        cache = KVCache(B, 3, T, 128, 3, "cuda", torch.bfloat16, inplace_state=True)
+        assert rel_err(model(idx[:, :P], kv_cache=cache), full[:, :P]) < 2e-2
+        for t in range(P, T):
+            assert rel_err(model(idx[:, t:t + 1], kv_cache=cache)[:, 0], full[:, t]) < 2e-2, t
