@@ -806,6 +806,9 @@ struct HandSmem {
 template <int K, int V, bool CHIP, class Gate = NoGate>
 __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx, int4 ch, DenseCarry<K>& cy,
                                            size_t hand = 0, const Gate& gate = Gate()) {
+  // multiply-adds only where written (fmaf): the same arithmetic in every kernel this is inlined
+  // into, so the fused launch, the tile launch and the separate parts agree bit for bit
+#pragma clang fp contract(off)
   using L = DenseSmem<K, V>;
   constexpr int MP = L::TP, KP = L::KP, VP = L::VP;
   constexpr int kVjpThreads = kDenseThreads, kVjpWaves = kDenseWaves;
@@ -829,7 +832,8 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
   const int H = a.H, h = hidx;
   const size_t tile = (size_t)cidx * H + h;
   const int row0 = ch.x;
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // uniform: scalar branches and bases
   const int lr = lane % 16, kg = lane / 16;
 
   const bf16* Tg = (const bf16*)a.ws.p[R_T] + tile * 64 * 64;
@@ -907,6 +911,29 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
   // round trip of its own after the gate): beta rows and lam of PA's key column
   const float beta_row = ((const float*)a.ws.p[R_BETA])[tile * 64 + (tid & 63)];
   const float lam_pa = ((const float*)a.ws.p[R_LAM])[tile * K + pa_c];
+  // X_c from the strip-major history [V/16][K][16]: 16-byte piece p = (strip, key, half)
+  // -> row key, columns 16 strip + 8 half of the staged [key][VP] matrix.  After a scan launch
+  // it is requested and staged with the rest, in the fused launch after the gate
+  constexpr int NP = K * V / 8, NPT = (NP + kDenseThreads - 1) / kDenseThreads;
+  bf16x8 xp[NPT];
+  auto load_x = [&] {
+#pragma unroll
+    for (int q = 0; q < NPT; ++q) {
+      const int p = min(q * kDenseThreads + tid, NP - 1);
+      xp[q] = Gate::kCoherent ? load16_coherent_bf16(DSH, p * 16) : *(const bf16x8*)(DSH + (size_t)p * 8);
+    }
+  };
+  auto x_row = [&](int key) { return key < 64 ? sX0 + key * VP : sX1 + (key - 64) * VP; };
+  auto stage_x = [&] {
+#pragma unroll
+    for (int q = 0; q < NPT; ++q) {
+      const int p = q * kDenseThreads + tid;
+      if (p >= NP) break;
+      const int st = p / (K * 2), key = (p / 2) % K, half = p % 2;
+      *(bf16x8*)(x_row(key) + 16 * st + 8 * half) = xp[q];
+    }
+  };
+  if constexpr (!Gate::kCoherent) load_x();
   // ---- P0 (scan-independent, before the gate): stage dO, v, beta kh e^G, delta, beta;
   // dQg = dO S^T and dA = tril(dO delta^T) need nothing from the scan ----
   {
@@ -935,6 +962,7 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
 #pragma unroll
     for (int e = 0; e < 8; ++e) sDL[(t0 + 16 * (e / 4) + e % 4) * VP + vv] = dlf[q][e];
   }
+  if constexpr (!Gate::kCoherent) stage_x();
   if (tid < 64) sB[tid] = beta_row;
   if (tid < 512) stage_permuted_piece((bf16*)(smem + L::off_a), L::TP, 64, tid, xa);
   for (int idx = tid; idx < 4 * 64; idx += kVjpThreads) sPM[idx] = 0.f;
@@ -1005,38 +1033,14 @@ __device__ __forceinline__ void dense_tile(const BwdArgs& a, int cidx, int hidx,
     for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(xs[sv][e]));
 
   gate();
-  // ---- the scan's histories (bf16, strip-major as the scan's strips wrote them): dS'
-  // rows of PA's key tile from [V/16][K][16], dU = dDelta from [V/16][4][16 v][16 t] ----
-#pragma unroll
-  for (int sv = 0; sv < NVS; ++sv) {
-    const int col = 32 * sv + 8 * kg;  // 8 columns inside strip col / 16
-    const size_t off = (size_t)(col / 16) * K * 16 + (size_t)pa_c * 16 + col % 16;
-    if (Gate::kCoherent) {
-      xd[sv] = load16_coherent_bf16(DSH, (int)off * 2);
-    } else {
-      xd[sv] = *(const bf16x8*)(DSH + off);
-    }
+  if constexpr (Gate::kCoherent) {
+    load_x();
+    stage_x();
+    __syncthreads();
   }
-  // X_c from the strip-major history [V/16][K][16]: 16-byte piece p = (strip, key, half)
-  // -> row key, columns 16 strip + 8 half of the staged [key][VP] matrix
-  {
-    constexpr int NP = K * V / 8, NPT = (NP + kDenseThreads - 1) / kDenseThreads;
-    bf16x8 xp[NPT];
+  // dS' rows of PA's key tile, from the staged X_c (PA overwrites it with dW)
 #pragma unroll
-    for (int q = 0; q < NPT; ++q) {
-      const int p = min(q * kDenseThreads + tid, NP - 1);
-      xp[q] = Gate::kCoherent ? load16_coherent_bf16(DSH, p * 16) : *(const bf16x8*)(DSH + (size_t)p * 8);
-    }
-#pragma unroll
-    for (int q = 0; q < NPT; ++q) {
-      const int p = q * kDenseThreads + tid;
-      if (p >= NP) break;
-      const int st = p / (K * 2), key = (p / 2) % K, half = p % 2;
-      bf16* row = key < 64 ? sX0 + key * VP : sX1 + (key - 64) * VP;
-      *(bf16x8*)(row + 16 * st + 8 * half) = xp[q];
-    }
-  }
-  __syncthreads();
+  for (int sv = 0; sv < NVS; ++sv) xd[sv] = *(const bf16x8*)(x_row(pa_c) + 32 * sv + 8 * kg);
   // dU = A^T dO + Kd X_c (bf16, the operand of PA and PB)
 #pragma unroll
   for (int j = 0; j < NDU; ++j) {
@@ -1297,6 +1301,9 @@ struct TileSmem {
 template <int K, bool CHIP>
 __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx, int4 ch, const DenseCarry<K>& cy,
                                            size_t hand) {
+  // multiply-adds only where written (fmaf): the same arithmetic in every kernel this is inlined
+  // into, so the fused launch, the tile launch and the separate parts agree bit for bit
+#pragma clang fp contract(off)
   using L = DecaySmem<K>;
   constexpr int QP = L::QP, GP = L::GP, AP = L::AP, HALF = L::HALF, OP = L::OP, NSEG = L::NSEG;
   constexpr int NKT = 4 * (K / 16);
@@ -1332,7 +1339,8 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
   const int H = a.H, h = hidx;
   const size_t tile = (size_t)cidx * H + h;
   const int row0 = ch.x;
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // uniform: scalar branches and bases
   const int lr = lane % 16, kg = lane / 16;
 
   const float* Gg = (const float*)a.ws.p[R_G] + tile * 64 * K;
@@ -1407,8 +1415,8 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
           kr[e] = to_bf16(0.f);
         }
         const float qv = to_f32(qr[e]), kv = to_f32(kr[e]);
-        sq += qv * qv;
-        sk += kv * kv;
+        sq = fmaf(qv, qv, sq);
+        sk = fmaf(kv, kv, sk);
       }
       *(bf16x8*)(sQ + t * QP + c0) = qr;
       *(bf16x8*)(sK + t * QP + c0) = kr;
@@ -1507,7 +1515,9 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
       if (!unsafe) {
         const float gf_rt = sG[(16 * rt) * GP + c], gl_rt = sG[(16 * rt + 15) * GP + c];
         // row side: blocks b <= rt, A = dA / dM' rows of tile rt, B = KR rows of block b
-        for (int b = 0; b <= rt; ++b) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          if (b > rt) break;
           const bf16x4 fa = *(const bf16x4*)(sDA + (16 * rt + lr) * AP + 16 * b + 4 * kg);
           const bf16x4 fm = *(const bf16x4*)(sDM + (16 * rt + lr) * AP + 16 * b + 4 * kg);
           const bf16x4 bh = lds_col_frag4(sKRh, OP, 16 * b, 16 * ctl, plane);
@@ -1530,7 +1540,9 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
           rk[r] *= f;
         }
         // column side: blocks b >= rt, A = dA^T / dM'^T (columns of tile rt), B = QC / KC
-        for (int b = rt; b < 4; ++b) {
+#pragma unroll
+        for (int b = 3; b >= 0; --b) {
+          if (b < rt) break;
           const bf16x4 fa = lds_col_frag4(sDA, AP, 16 * b, 16 * rt, plane);
           const bf16x4 fm = lds_col_frag4(sDM, AP, 16 * b, 16 * rt, plane);
           const bf16x4 qh = lds_col_frag4(sQCh, OP, 16 * b, 16 * ctl, plane);
@@ -1579,33 +1591,35 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
         }
       }
       const float GL = sG[63 * GP + c];
+      const int i0 = 16 * rt + 4 * kg;  // this lane's rows
+      const f32x4 rq4 = *(const f32x4*)(sRq + i0), rk4 = *(const f32x4*)(sRk + i0), bt4 = *(const f32x4*)(sBeta + i0);
       float glp = 0.f;
-      f32x4 dqs, dks, dgs;
+      f32x4 dqs, dks, dgs, pb4, pq4, pk4;
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
-        const int ii = 16 * rt + 4 * kg + rr;
-        const float qh = to_f32(sQ[ii * QP + c]) * sRq[ii], kh = to_f32(sK[ii * QP + c]) * sRk[ii];
+        const int ii = i0 + rr;
+        const float qh = to_f32(sQ[ii * QP + c]) * rq4[rr], kh = to_f32(sK[ii * QP + c]) * rk4[rr];
         const float G = sG[ii * GP + c];
-        const float bt = sBeta[ii];
+        const float bt = bt4[rr];
         const float eG = __expf(G), eKd = __expf(GL - G);
         const float dQg = rdQ[rr], dKd = rdK[rr], dKb = rdB[rr];
         const float cc = cq[rr] + ck[rr];
         const float dqh = fmaf(dQg, eG, rq[rr]);
-        const float dkh = dKd * eKd + bt * eG * dKb + rk[rr] + cc;
+        const float dkh = fmaf(dKd, eKd, fmaf(bt * eG, dKb, rk[rr] + cc));
         const float kdd = dKd * kh * eKd;
         const float kbb = dKb * kh * eG;  // dbeta partial (the beta factor of Kb removed)
-        dgs[rr] = dQg * qh * eG - kdd + bt * kbb + qh * rq[rr] + kh * rk[rr] - kh * cc;
+        dgs[rr] = fmaf(dQg * qh, eG, fmaf(bt, kbb, fmaf(qh, rq[rr], fmaf(kh, rk[rr] - cc, -kdd))));
         dqs[rr] = dqh;
         dks[rr] = dkh;
         glp += kdd;
-        const float pb = group_sum<16>(kbb);
-        const float pq = group_sum<16>(qh * dqh);
-        const float pk = group_sum<16>(kh * dkh);
-        if (lr == 0) {
-          sPB[ct * 64 + ii] = pb;
-          sPQ[ct * 64 + ii] = pq;
-          sPK[ct * 64 + ii] = pk;
-        }
+        pb4[rr] = group_sum<16>(kbb);
+        pq4[rr] = group_sum<16>(qh * dqh);
+        pk4[rr] = group_sum<16>(kh * dkh);
+      }
+      if (lr == 0) {
+        *(f32x4*)(sPB + ct * 64 + i0) = pb4;
+        *(f32x4*)(sPQ + ct * 64 + i0) = pq4;
+        *(f32x4*)(sPK + ct * 64 + i0) = pk4;
       }
       if (pass == 0) {
         keep_q[0] = dqs; keep_k[0] = dks; keep_g[0] = dgs;
@@ -1652,8 +1666,8 @@ __device__ __forceinline__ void decay_tile(const BwdArgs& a, int cidx, int hidx,
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) {
       const int ii = 16 * rt + 4 * kg + rr;
-      dqv[rr] = sRq[ii] * dqs[rr] - to_f32(sQ[ii * QP + c]) * sRq[ii] * sPQ[ii];
-      dkv[rr] = sRk[ii] * dks[rr] - to_f32(sK[ii * QP + c]) * sRk[ii] * sPK[ii];
+      dqv[rr] = sRq[ii] * fmaf(-to_f32(sQ[ii * QP + c]), sPQ[ii], dqs[rr]);
+      dkv[rr] = sRk[ii] * fmaf(-to_f32(sK[ii * QP + c]), sPK[ii], dks[rr]);
     }
     // every read of this element's q / k happened in this lane; write back in place
 #pragma unroll
@@ -1774,9 +1788,25 @@ __global__ __launch_bounds__(kVjpThreads) void chunk_bwd_part_kernel(BwdArgs a, 
 
 // Both parts of tile blockIdx.x in one workgroup, after a scan launch.  At 3,072 tiles (B4
 // T8192 H6, K = V = 128) the dense and decay parts as 24 launches of 256 workgroups took
-// 631 us, this one launch 458 us.
+// 631 us, this one launch 460 us.
+//
+// At K = V = 128 a workgroup has a CU to itself (its LDS) and every workgroup takes the same
+// time: the chip loads 256 tiles at once at the rate of memory (12 us of the 41 us of a tile,
+// 224 KB each), then computes 256 tiles with memory idle.  So the first workgroup of each CU
+// starts late by up to 31 steps of kStagger, the same step on every XCD (consecutive workgroups
+// go to different XCDs), and from then on some CUs load while others compute.  The start costs
+// up to 20 us and each later round saves about 5.  Medians without -> with: 768 tiles 118 ->
+// 128 us, 1024 161 -> 163, 1280 200 -> 199, 1536 237 -> 230, 2048 307 -> 298, 2560 386 -> 360,
+// 3072 465 -> 442; packed documents of 2,064 tiles 318 -> 294.  Steps of 8, 15, 25, 35 and 45 at
+// 3072: 458, 447, 442, 449, 461 us.
+constexpr int kCUs = 256, kStaggerFrom = 5 * kCUs, kStagger = 25;  // kStagger: 64-clock units
+
 template <int K, int V>
 __global__ __launch_bounds__(kVjpThreads) void chunk_bwd_tile_kernel(BwdArgs a) {
+  if constexpr (K == 128 && V == 128) {
+    if (gridDim.x >= kStaggerFrom && blockIdx.x < kCUs)
+      for (int k = blockIdx.x / 8; k > 0; --k) __builtin_amdgcn_s_sleep(kStagger);
+  }
   const int cidx = blockIdx.x / a.H, h = blockIdx.x % a.H;
   const int4 ch = chunk_entry(a, cidx);
   DenseCarry<K> cy;

@@ -487,3 +487,16 @@ def test_captured_call_equals_eager_call():
         ops.chunk_backward_status(p, scratch)
         for j, (x, y) in enumerate(zip(eager, captured)):
             assert x is None or torch.equal(x, y), (i, j)
+
+
+@pytest.mark.parametrize("B", [160, 161])
+def test_many_tiles_equal_their_halves(B):
+    """1,280 tiles or more start staggered over the CUs; 640 or so do not.  Each sequence's
+    gradients are its own, so the whole batch gives bit for bit what its two parts give."""
+    d = make_kda_inputs(B, 500, 1, 128, 128, seed=51)  # 8 chunks a sequence, the last one ragged
+    do, _ = cotangents(d, 52)
+    whole = gpu_grads(d, "k3", do, None)
+    for part in (slice(0, 80), slice(80, B)):
+        half = {n: x[part].contiguous() if n in ("q", "k", "v", "g", "beta") else x for n, x in d.items()}
+        for a, b in zip(whole[:5], gpu_grads(half, "k3", do[part].contiguous(), None)[:5]):
+            assert torch.equal(a[part], b)
