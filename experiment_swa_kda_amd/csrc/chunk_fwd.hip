@@ -876,24 +876,38 @@ __global__ __launch_bounds__(kIntraThreads, 2 * kIntraNH) void chunk_fwd_intra_k
 // the f32 state history straight to HBM (nothing in their stream waits on those stores);
 // the store wave copies the bf16 state and delta histories out of the double-buffered
 // exchange one step later.
+//
+// With OUT the workgroup also forms its strips' outputs O = Qg S + A delta: two output waves
+// in the store wave's place read the staged state and delta, hold the Qg and A fragments of
+// their two row tiles kOutAhead chunks ahead in registers, and write the outputs.  The bf16
+// state history is then written and read by no one, and without a gradient to come the delta
+// history neither: 96 KB of 184 KB per chunk at K = V = 128.  The workgroup owns two strips,
+// which share -W, Kd^T, Qg and A: with one the steps of a full chip (one workgroup per CU, by
+// its LDS) were as long and twice as many.  B64 T1024 H3 at inference: scan and output
+// launches 115 + 57 us, here 95 us; with one strip 144 us.
 constexpr int kScanRing = 4;
 constexpr int kScanCompute = 4;                 // compute waves (one 16-token delta tile each)
 constexpr int kScanThreads = (kScanCompute + 3) * kWave;  // + two loader waves and a store wave
+constexpr int kScanOutThreads = (kScanCompute + 4) * kWave;  // ... or two output waves
+constexpr int kOutAhead = 3;  // chunks whose Qg and A fragments an output wave holds or has in flight
 
-template <int K, int V>
+template <int K, int V, bool OUT>
 struct ScanLds {
+  static constexpr int NST = OUT ? 2 : 1;               // strips of a workgroup
+  static constexpr int RING = OUT ? 3 : kScanRing;
   static constexpr int off_w = 0;                       // -W fragments, 64 x K bf16
   static constexpr int off_kdt = off_w + 64 * K * 2;    // Kd^T fragments, K x 64 bf16
   static constexpr int off_u = off_kdt + K * 64 * 2;    // U strip, C layout, 64 x 16 bf16
-  static constexpr int off_lam = off_u + 64 * 16 * 2;   // lam, K f32
+  static constexpr int off_lam = off_u + NST * 64 * 16 * 2;  // lam, K f32
   static constexpr int slot = off_lam + K * 4;
-  static constexpr int n_load0 = (64 * K * 2) / 1024 + 2;  // loader 0: W blocks + U strip
+  static constexpr int n_load0 = (64 * K * 2) / 1024 + 2 * NST;  // loader 0: W blocks + U strips
   static constexpr int n_load1 = (K * 64 * 2) / 1024 + 1;  // loader 1: Kd^T blocks + lam
   // staging (x2): f32 state in accumulator order, bf16 state and delta fragments
   static constexpr int st_sb = 0;
   static constexpr int st_dl = st_sb + 16 * K * 2;
-  static constexpr int stage = st_dl + 16 * 64 * 2;
-  static constexpr int off_stage = kScanRing * slot;
+  static constexpr int strip_stage = st_dl + 16 * 64 * 2;
+  static constexpr int stage = NST * strip_stage;
+  static constexpr int off_stage = RING * slot;
   static constexpr int bytes = off_stage + 2 * stage;
 };
 
@@ -907,26 +921,53 @@ __device__ __forceinline__ bf16x8 pack_tiles(const f32x4& lo, const f32x4& hi) {
   return x;
 }
 
-template <int K, int V>
-__global__ __launch_bounds__(kScanThreads) void chunk_fwd_scan_kernel(FwdArgs a) {
-  using L = ScanLds<K, V>;
-  constexpr int KT = K / 16, NB = K / 32, KPW = KT / kScanCompute;
+// One 16-token row tile of a strip's output, O = Qg S + A delta, from the operands in
+// registers: formed transposed (the strip's columns as the rows of the product), so that a lane
+// holds four consecutive columns of one token.  The sums are the output kernel's.
+template <int K>
+__device__ __forceinline__ bf16x4 out_tile(const bf16x8* fq, const bf16x8* fa, const bf16x8* sb, const bf16x8* dl) {
+  f32x4 o0 = zero4(), o1 = zero4();
+#pragma unroll
+  for (int s = 0; s < K / 32; s += 2) {
+    o0 = mfma16(sb[s], fq[s], o0);
+    o1 = mfma16(sb[s + 1], fq[s + 1], o1);
+  }
+  o0 = mfma16(dl[0], fa[0], o0);
+  o1 = mfma16(dl[1], fa[1], o1);
+  bf16x4 x;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) x[r] = to_bf16(o0[r] + o1[r]);
+  return x;
+}
+
+template <int V>
+__device__ __forceinline__ void store_out(const FwdArgs& a, int row0, int len, int h, int v0, int rt, bf16x4 x,
+                                          int lane) {
+  const int t = 16 * rt + lane % 16, kg = lane / 16;
+  if (t < len) *(bf16x4*)(a.out + ((size_t)(row0 + t) * a.H + h) * V + v0 + 4 * kg) = x;
+}
+
+template <int K, int V, bool OUT>
+__global__ __launch_bounds__(OUT ? kScanOutThreads : kScanThreads) void chunk_fwd_scan_kernel(FwdArgs a) {
+  using L = ScanLds<K, V, OUT>;
+  constexpr int KT = K / 16, NB = K / 32, KPW = KT / kScanCompute, NST = L::NST, RING = L::RING;
   static_assert(KT % kScanCompute == 0, "state tiles split evenly over the compute waves");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int H = a.H;
   int rec, strip;
-  if (!xcd_strip_coords(a.num_seqs * H, V / 16, rec, strip)) return;
-  const int seq = rec / H, h = rec % H, v0 = strip * 16;
+  if (!xcd_strip_coords(a.num_seqs * H, V / 16 / NST, rec, strip)) return;
+  const int seq = rec / H, h = rec % H, v0 = strip * (16 * NST);
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int lr = lane % 16, kg = lane / 16;
   const int2 sq = seq_entry(a, seq);  // {first chunk, chunk count}
   const int n = sq.y;
   if (n <= 0) {
     if (wave == 0 && a.sfin) {
-      for (int kt = 0; kt < KT; ++kt) {
-        const size_t o = (((size_t)seq * H + h) * V + v0 + lr) * K + 16 * kt + 4 * kg;
-        *(float4*)(a.sfin + o) = a.s0 ? *(const float4*)(a.s0 + o) : make_float4(0.f, 0.f, 0.f, 0.f);
-      }
+      for (int st = 0; st < NST; ++st)
+        for (int kt = 0; kt < KT; ++kt) {
+          const size_t o = (((size_t)seq * H + h) * V + v0 + 16 * st + lr) * K + 16 * kt + 4 * kg;
+          *(float4*)(a.sfin + o) = a.s0 ? *(const float4*)(a.s0 + o) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
     }
     return;
   }
@@ -937,15 +978,14 @@ __global__ __launch_bounds__(kScanThreads) void chunk_fwd_scan_kernel(FwdArgs a)
     auto issue = [&](int ci) {
       const int c = ci < n ? ci : n - 1;  // fixed load count per chunk (clamped index)
       const size_t tile = (size_t)(sq.x + c) * H + h;
-      char* slot = smem + (ci % kScanRing) * L::slot;
+      char* slot = smem + (ci % RING) * L::slot;
       if (lw == 0) {
         const char* w = (const char*)((const bf16*)a.ws.p[R_WF] + tile * 64 * K) + lane * 16;
 #pragma unroll
         for (int b = 0; b < (64 * K * 2) / 1024; ++b) dma16(w + b * 1024, slot + L::off_w + b * 1024);
-        const char* u = (const char*)((const bf16*)a.ws.p[R_UF] + tile * 64 * V + (size_t)strip * 64 * 16) +
-                        lane * 16;
-        dma16(u, slot + L::off_u);
-        dma16(u + 1024, slot + L::off_u + 1024);
+        const char* u = (const char*)((const bf16*)a.ws.p[R_UF] + tile * 64 * V + (size_t)v0 * 64) + lane * 16;
+#pragma unroll
+        for (int b = 0; b < 2 * NST; ++b) dma16(u + b * 1024, slot + L::off_u + b * 1024);
       } else {
         const char* kd = (const char*)((const bf16*)a.ws.p[R_KDTF] + tile * K * 64) + lane * 16;
 #pragma unroll
@@ -954,15 +994,15 @@ __global__ __launch_bounds__(kScanThreads) void chunk_fwd_scan_kernel(FwdArgs a)
       }
     };
 #pragma unroll
-    for (int d = 0; d < kScanRing - 1; ++d) issue(d);
+    for (int d = 0; d < RING - 1; ++d) issue(d);
     for (int ci = 0; ci < n; ++ci) {
       // the slot of chunk ci is complete once at most (ring - 2) chunks' loads are newer
       if (lw == 0)
-        wait_vmcnt<(kScanRing - 2) * L::n_load0>();
+        wait_vmcnt<(RING - 2) * L::n_load0>();
       else
-        wait_vmcnt<(kScanRing - 2) * L::n_load1>();
+        wait_vmcnt<(RING - 2) * L::n_load1>();
       ring_barrier();  // B1(ci): every read of slot ci - 1 finished before B2(ci - 1)
-      issue(ci + kScanRing - 1);
+      issue(ci + RING - 1);
       ring_barrier();  // B2(ci)
     }
     ring_barrier();   // B1(n)
@@ -970,7 +1010,71 @@ __global__ __launch_bounds__(kScanThreads) void chunk_fwd_scan_kernel(FwdArgs a)
     return;
   }
 
-  if (wave == kScanCompute + 2) {
+  if constexpr (OUT) {
+    if (wave >= kScanCompute + 2) {
+      // ---- output wave: row tiles 2 ow and 2 ow + 1 of chunk c, its state and delta read
+      // between B1(c + 1) and B2(c + 1) as the store wave does ----
+      const int ow = wave - (kScanCompute + 2);
+      struct Ops {
+        bf16x8 q[2][NB], a[2][2];
+      } ops[kOutAhead];
+      const int row0 = chunk_entry(a, sq.x).x;
+      const int tokens = (n - 1) * kChunk + chunk_entry(a, sq.x + n - 1).y;
+      auto fetch = [&](Ops& o, int ci) {
+        const int c = sq.x + (ci < n ? ci : n - 1);
+        const size_t tile = (size_t)c * H + h;
+        const bf16* QGF = (const bf16*)a.ws.p[R_QGF] + tile * 64 * K;
+        const bf16* AF = (const bf16*)a.ws.p[R_AF] + tile * 64 * 64;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+          for (int s = 0; s < NB; ++s) o.q[t][s] = *(const bf16x8*)(QGF + frag_off(K, 2 * ow + t, s, lane));
+#pragma unroll
+          for (int s = 0; s < 2; ++s) o.a[t][s] = *(const bf16x8*)(AF + frag_off(64, 2 * ow + t, s, lane));
+        }
+      };
+#pragma unroll
+      for (int d = 0; d < kOutAhead; ++d) fetch(ops[d], d);
+      ring_barrier();  // B1(0)
+      ring_barrier();  // B2(0)
+      for (int c0 = 0;; c0 += kOutAhead) {
+#pragma unroll
+        for (int d = 0; d < kOutAhead; ++d) {
+          const int c = c0 + d;
+          if (c >= n) return;  // (a jump to the loop's end would make every set wait for the newest loads)
+          ring_barrier();  // B1(c + 1)
+          bf16x8 sb[NST][NB], dl[NST][2];
+#pragma unroll
+          for (int j = 0; j < NST; ++j) {
+            const char* st = smem + L::off_stage + (c & 1) * L::stage + j * L::strip_stage;
+#pragma unroll
+            for (int s = 0; s < NB; ++s) sb[j][s] = *(const bf16x8*)(st + L::st_sb + (s * 64 + lane) * 16);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) dl[j][s] = *(const bf16x8*)(st + L::st_dl + (s * 64 + lane) * 16);
+          }
+          bf16x4 x[NST][2];
+#pragma unroll
+          for (int j = 0; j < NST; ++j)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) x[j][t] = out_tile<K>(ops[d].q[t], ops[d].a[t], sb[j], dl[j]);
+          wait_lgkm0();
+          if (c + 1 < n) ring_barrier();  // B2(c + 1)
+          if (!a.infer) {
+            bf16* DLF = (bf16*)a.ws.p[R_DLF] + ((size_t)(sq.x + c) * H + h) * 64 * V + (size_t)v0 * 64;
+#pragma unroll
+            for (int j = 0; j < NST; ++j)
+              *(bf16x8*)(DLF + ((size_t)(2 * j + ow) * 64 + lane) * 8) = ow == 0 ? dl[j][0] : dl[j][1];
+          }
+          const int r0 = row0 + c * kChunk, len = tokens - c * kChunk;
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int j = 0; j < NST; ++j) store_out<V>(a, r0, len, h, v0 + 16 * j, 2 * ow + t, x[j][t], lane);
+          fetch(ops[d], c + kOutAhead);
+        }
+      }
+    }
+  } else if (wave == kScanCompute + 2) {
     // ---- store wave: histories of chunk ci - 1, read between B1(ci) and B2(ci) (the
     // compute waves refill that staging buffer after B2(ci)), written to HBM after ----
     for (int ci = 0; ci <= n; ++ci) {
@@ -999,50 +1103,62 @@ __global__ __launch_bounds__(kScanThreads) void chunk_fwd_scan_kernel(FwdArgs a)
 
   // ---- compute wave c: delta row tile c, state tiles c*KPW .. c*KPW + KPW - 1 ----
   const int cw = wave;
-  f32x4 S[KPW];
+  f32x4 S[NST][KPW];
 #pragma unroll
-  for (int j = 0; j < KPW; ++j) {
-    const int k0 = 16 * (cw * KPW + j) + 4 * kg;
-    if (a.s0) {
-      const float4 s = *(const float4*)(a.s0 + (((size_t)seq * H + h) * V + v0 + lr) * K + k0);
-      S[j][0] = s.x; S[j][1] = s.y; S[j][2] = s.z; S[j][3] = s.w;
-    } else {
-      S[j] = zero4();
+  for (int i = 0; i < NST; ++i)
+#pragma unroll
+    for (int j = 0; j < KPW; ++j) {
+      const int k0 = 16 * (cw * KPW + j) + 4 * kg;
+      if (a.s0) {
+        const float4 s = *(const float4*)(a.s0 + (((size_t)seq * H + h) * V + v0 + 16 * i + lr) * K + k0);
+        S[i][j][0] = s.x; S[i][j][1] = s.y; S[i][j][2] = s.z; S[i][j][3] = s.w;
+      } else {
+        S[i][j] = zero4();
+      }
     }
-  }
   // the bf16 state (B operand of the delta product) lives in the staging buffer of the
   // chunk it enters: fragment s packs state tiles 2s (low half) and 2s + 1 (high half)
   auto put_state = [&](char* st) {
 #pragma unroll
-    for (int j = 0; j < KPW; ++j) {
-      const int kt = cw * KPW + j;
-      bf16x4 x;
+    for (int i = 0; i < NST; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) x[r] = to_bf16(S[j][r]);
-      *(bf16x4*)(st + L::st_sb + ((kt / 2) * 64 + lane) * 16 + (kt % 2) * 8) = x;
-    }
+      for (int j = 0; j < KPW; ++j) {
+        const int kt = cw * KPW + j;
+        bf16x4 x;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = to_bf16(S[i][j][r]);
+        *(bf16x4*)(st + i * L::strip_stage + L::st_sb + ((kt / 2) * 64 + lane) * 16 + (kt % 2) * 8) = x;
+      }
   };
   put_state(smem + L::off_stage);
   wait_lgkm0();
   for (int ci = 0; ci < n; ++ci) {
     ring_barrier();  // B1(ci): slot ci loaded, the state entering chunk ci staged
-    const char* slot = smem + (ci % kScanRing) * L::slot;
+    const char* slot = smem + (ci % RING) * L::slot;
     char* st = smem + L::off_stage + (ci & 1) * L::stage;
-    bf16x8 wf[NB], Bs[NB], kf[KPW][2];
+    bf16x8 wf[NB], Bs[NST][NB], kf[KPW][2];
     float4 lamf[KPW];
 #pragma unroll
     for (int s = 0; s < NB; ++s) {
       wf[s] = *(const bf16x8*)(slot + L::off_w + ((cw * NB + s) * 64 + lane) * 16);
-      Bs[s] = *(const bf16x8*)(st + L::st_sb + (s * 64 + lane) * 16);
+#pragma unroll
+      for (int i = 0; i < NST; ++i)
+        Bs[i][s] = *(const bf16x8*)(st + i * L::strip_stage + L::st_sb + (s * 64 + lane) * 16);
     }
-    const bf16x4 uf = *(const bf16x4*)(slot + L::off_u + (cw * 64 + lane) * 8);
+    bf16x4 uf[NST];
+#pragma unroll
+    for (int i = 0; i < NST; ++i) uf[i] = *(const bf16x4*)(slot + L::off_u + i * 2048 + (cw * 64 + lane) * 8);
     __builtin_amdgcn_sched_barrier(0);
     // delta tile c = U + (-W) S: one K/32-deep chain
-    f32x4 dl;
+    f32x4 dl[NST];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) dl[r] = to_f32(uf[r]);
+    for (int i = 0; i < NST; ++i)
 #pragma unroll
-    for (int s = 0; s < NB; ++s) dl = mfma16(wf[s], Bs[s], dl);
+      for (int r = 0; r < 4; ++r) dl[i][r] = to_f32(uf[i][r]);
+#pragma unroll
+    for (int s = 0; s < NB; ++s)
+#pragma unroll
+      for (int i = 0; i < NST; ++i) dl[i] = mfma16(wf[s], Bs[i][s], dl[i]);
     // meanwhile: the f32 history of the entering state (straight to HBM: nothing in this
     // wave waits on its stores), and this wave's Kd^T rows and lam
     float* SH = (float*)a.ws.p[R_SH] + ((size_t)(sq.x + ci) * H + h) * K * V + v0 + lr;
@@ -1051,46 +1167,61 @@ __global__ __launch_bounds__(kScanThreads) void chunk_fwd_scan_kernel(FwdArgs a)
       const int kt = cw * KPW + j;
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (!a.infer) SH[(size_t)(16 * kt + 4 * kg + r) * V] = S[j][r];
+        if (!a.infer)
+#pragma unroll
+          for (int i = 0; i < NST; ++i) SH[(size_t)(16 * kt + 4 * kg + r) * V + 16 * i] = S[i][j][r];
       kf[j][0] = *(const bf16x8*)(slot + L::off_kdt + ((kt * 2) * 64 + lane) * 16);
       kf[j][1] = *(const bf16x8*)(slot + L::off_kdt + ((kt * 2 + 1) * 64 + lane) * 16);
       lamf[j] = *(const float4*)(slot + L::off_lam + (16 * kt + 4 * kg) * 4);
     }
-    {
+#pragma unroll
+    for (int i = 0; i < NST; ++i) {
       bf16x4 x;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) x[r] = to_bf16(dl[r]);
+      for (int r = 0; r < 4; ++r) x[r] = to_bf16(dl[i][r]);
       // delta B fragment t packs row tiles 2t (low half) and 2t + 1 (high half)
-      *(bf16x4*)(st + L::st_dl + ((cw / 2) * 64 + lane) * 16 + (cw % 2) * 8) = x;
+      *(bf16x4*)(st + i * L::strip_stage + L::st_dl + ((cw / 2) * 64 + lane) * 16 + (cw % 2) * 8) = x;
     }
-    f32x4 acc[KPW];
+    f32x4 acc[NST][KPW];
 #pragma unroll
-    for (int j = 0; j < KPW; ++j) {
-      acc[j][0] = lamf[j].x * S[j][0];
-      acc[j][1] = lamf[j].y * S[j][1];
-      acc[j][2] = lamf[j].z * S[j][2];
-      acc[j][3] = lamf[j].w * S[j][3];
-    }
+    for (int i = 0; i < NST; ++i)
+#pragma unroll
+      for (int j = 0; j < KPW; ++j) {
+        acc[i][j][0] = lamf[j].x * S[i][j][0];
+        acc[i][j][1] = lamf[j].y * S[i][j][1];
+        acc[i][j][2] = lamf[j].z * S[i][j][2];
+        acc[i][j][3] = lamf[j].w * S[i][j][3];
+      }
     wait_lgkm0();
     ring_barrier();  // B2(ci): every delta tile staged
-    const bf16x8 D0 = *(const bf16x8*)(st + L::st_dl + lane * 16);
-    const bf16x8 D1 = *(const bf16x8*)(st + L::st_dl + (64 + lane) * 16);
+    bf16x8 D[NST][2];
+#pragma unroll
+    for (int i = 0; i < NST; ++i)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        D[i][s] = *(const bf16x8*)(st + i * L::strip_stage + L::st_dl + (s * 64 + lane) * 16);
     // S = lam S + Kd^T delta
 #pragma unroll
-    for (int j = 0; j < KPW; ++j) S[j] = mfma16(kf[j][0], D0, acc[j]);
+    for (int i = 0; i < NST; ++i)
 #pragma unroll
-    for (int j = 0; j < KPW; ++j) S[j] = mfma16(kf[j][1], D1, S[j]);
+      for (int j = 0; j < KPW; ++j) S[i][j] = mfma16(kf[j][0], D[i][0], acc[i][j]);
+#pragma unroll
+    for (int i = 0; i < NST; ++i)
+#pragma unroll
+      for (int j = 0; j < KPW; ++j) S[i][j] = mfma16(kf[j][1], D[i][1], S[i][j]);
     put_state(smem + L::off_stage + ((ci + 1) & 1) * L::stage);
     wait_lgkm0();
   }
   ring_barrier();  // B1(n)
   if (a.sfin) {
 #pragma unroll
-    for (int j = 0; j < KPW; ++j) {
-      const int k0 = 16 * (cw * KPW + j) + 4 * kg;
-      *(float4*)(a.sfin + (((size_t)seq * H + h) * V + v0 + lr) * K + k0) =
-          make_float4(S[j][0], S[j][1], S[j][2], S[j][3]);
-    }
+    for (int i = 0; i < NST; ++i)
+#pragma unroll
+      for (int j = 0; j < KPW; ++j) {
+        const int k0 = 16 * (cw * KPW + j) + 4 * kg;
+        *(float4*)(a.sfin + (((size_t)seq * H + h) * V + v0 + 16 * i + lr) * K + k0) =
+            make_float4(S[i][j][0], S[i][j][1], S[i][j][2], S[i][j][3]);
+      }
   }
 }
 
@@ -1108,18 +1239,22 @@ __global__ __launch_bounds__(kScanThreads) void chunk_fwd_scan_kernel(FwdArgs a)
 //     the segments of one recurrence, one wave per V strip (S as hi + lo bf16 operands);
 //  3. replay (chunk_fwd_seg_kernel<.., true>): every segment reruns its chunks from its true
 //     entering state and writes the state / delta histories exactly as the one-pass scan.
+//     With OUT it also forms the outputs, from Qg and A in its LDS slots: they cost a third
+//     slot, but the bf16 state is not written and read again.  B4 T8192 H6, K = V = 128:
+//     replay 100 + output 72 us, here 128 us.
 // Sequential depth: L + (segments - 1) + L steps instead of the chunk count.  In the
 // segment kernels one workgroup owns several strips and every compute wave owns whole
 // strips (its delta tiles and state tiles), so a step needs no exchange between waves:
 // a loader wave fills an LDS ring with the chunk's -W, Kd^T, U strips and lam, and the one
 // barrier per chunk only recycles ring slots.
 constexpr int kSegRing = 3;
+constexpr int kSegOutRing = 2;   // with Qg and A in the slot
 constexpr int kSegCompute = 4;   // compute waves, one strip each (every wave reads the
                                  // chunk's whole -W and Kd^T from LDS)
 constexpr int kSegSPW = 1;
 constexpr int kSegThreads = (kSegCompute + 1) * kWave;
 
-template <int K, int V, bool REPLAY>
+template <int K, int V, bool REPLAY, bool OUT = false>
 struct SegCfg {
   static constexpr int NSTRIPS = REPLAY ? V / 16 : (V + K) / 16;  // strips per (rec, segment)
   static constexpr int SPW = kSegSPW;                               // strips per compute wave
@@ -1130,14 +1265,20 @@ struct SegCfg {
   static constexpr int off_kdt = off_w + 64 * K * 2;   // Kd^T fragments, K x 64 bf16
   static constexpr int off_u = off_kdt + K * 64 * 2;   // U, C layout, SPG strips x 2 KB
   static constexpr int off_lam = off_u + SPG * 2048;   // lam, K f32
-  static constexpr int slot = off_lam + K * 4;
-  static constexpr int n_load = (64 * K * 2) / 1024 + (K * 64 * 2) / 1024 + 2 * SPG + 1;
-  static constexpr int bytes = kSegRing * slot;
+  static constexpr int off_qg = off_lam + K * 4;       // OUT: Qg fragments, 64 x K bf16
+  static constexpr int off_a = off_qg + (OUT ? 64 * K * 2 : 0);  // OUT: A fragments, 64 x 64 bf16
+  static constexpr int slot = off_a + (OUT ? 64 * 64 * 2 : 0);
+  static constexpr int RING = OUT ? kSegOutRing : kSegRing;
+  static constexpr int n_load = (64 * K * 2) / 1024 + (K * 64 * 2) / 1024 + 2 * SPG + 1 +
+                                (OUT ? (64 * K * 2) / 1024 + 8 : 0);
+  static constexpr int bytes = RING * slot;
 };
 
-template <int K, int V, bool REPLAY>
+template <int K, int V, bool REPLAY, bool OUT = false>
 __global__ __launch_bounds__(kSegThreads) void chunk_fwd_seg_kernel(FwdArgs a, int seg_len, int max_segs) {
-  using C = SegCfg<K, V, REPLAY>;
+  using C = SegCfg<K, V, REPLAY, OUT>;
+  constexpr int RING = C::RING;
+  static_assert(REPLAY || !OUT, "only the replay knows the true states");
   constexpr int KT = K / 16, NB = K / 32, VS = V / 16, SPW = C::SPW;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int H = a.H;
@@ -1177,7 +1318,7 @@ __global__ __launch_bounds__(kSegThreads) void chunk_fwd_seg_kernel(FwdArgs a, i
     auto issue = [&](int ci) {
       const int c = c_begin + (ci < steps ? ci : steps - 1);
       const size_t tile = (size_t)(sq.x + c) * H + h;
-      char* slot = smem + (ci % kSegRing) * C::slot;
+      char* slot = smem + (ci % RING) * C::slot;
       const char* w = (const char*)((const bf16*)a.ws.p[R_WF] + tile * 64 * K) + lane * 16;
 #pragma unroll
       for (int b = 0; b < (64 * K * 2) / 1024; ++b) dma16(w + b * 1024, slot + C::off_w + b * 1024);
@@ -1192,13 +1333,21 @@ __global__ __launch_bounds__(kSegThreads) void chunk_fwd_seg_kernel(FwdArgs a, i
         dma16(u0 + (size_t)us * 2048 + 1024, slot + C::off_u + j * 2048 + 1024);
       }
       if (lane < K / 4) dma16((const float*)a.ws.p[R_LAM] + tile * K + lane * 4, slot + C::off_lam);
+      if constexpr (OUT) {
+        const char* q = (const char*)((const bf16*)a.ws.p[R_QGF] + tile * 64 * K) + lane * 16;
+#pragma unroll
+        for (int b = 0; b < (64 * K * 2) / 1024; ++b) dma16(q + b * 1024, slot + C::off_qg + b * 1024);
+        const char* f = (const char*)((const bf16*)a.ws.p[R_AF] + tile * 64 * 64) + lane * 16;
+#pragma unroll
+        for (int b = 0; b < 8; ++b) dma16(f + b * 1024, slot + C::off_a + b * 1024);
+      }
     };
 #pragma unroll
-    for (int d = 0; d < kSegRing - 1; ++d) issue(d);
+    for (int d = 0; d < RING - 1; ++d) issue(d);
     for (int ci = 0; ci < steps; ++ci) {
-      wait_vmcnt<(kSegRing - 2) * C::n_load>();  // chunk ci's loads have landed
+      wait_vmcnt<(RING - 2) * C::n_load>();  // chunk ci's loads have landed
       ring_barrier();                             // B(ci); the slot of ci - 1 fully read
-      issue(ci + kSegRing - 1);
+      issue(ci + RING - 1);
     }
     ring_barrier();   // B(steps)
     wait_vmcnt<0>();  // no LDS write may land after the workgroup ends
@@ -1233,9 +1382,14 @@ __global__ __launch_bounds__(kSegThreads) void chunk_fwd_seg_kernel(FwdArgs a, i
       }
     }
   }
+  int row0 = 0, tokens = 0;  // OUT: the segment's first row, its tokens
+  if constexpr (OUT) {
+    row0 = chunk_entry(a, sq.x + c_begin).x;
+    tokens = (steps - 1) * kChunk + chunk_entry(a, sq.x + c_begin + steps - 1).y;
+  }
   for (int ci = 0; ci < steps; ++ci) {
     ring_barrier();  // B(ci): slot ci loaded
-    const char* slot = smem + (ci % kSegRing) * C::slot;
+    const char* slot = smem + (ci % RING) * C::slot;
     // every operand of the step requested before the first product
     bf16x8 wf[4][NB], kf[KT][2];
     float4 lam[KT];
@@ -1277,9 +1431,11 @@ __global__ __launch_bounds__(kSegThreads) void chunk_fwd_seg_kernel(FwdArgs a, i
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             if (!a.infer) SH[(size_t)(16 * kt + 4 * kg + r) * V] = S[j][kt][r];
-        bf16* SHBF = (bf16*)a.ws.p[R_SHBF] + tile * V * K + (size_t)strip[j] * 16 * K;
+        if constexpr (!OUT) {
+          bf16* SHBF = (bf16*)a.ws.p[R_SHBF] + tile * V * K + (size_t)strip[j] * 16 * K;
 #pragma unroll
-        for (int s = 0; s < NB; ++s) *(bf16x8*)(SHBF + ((size_t)s * 64 + lane) * 8) = Bs[j][s];
+          for (int s = 0; s < NB; ++s) *(bf16x8*)(SHBF + ((size_t)s * 64 + lane) * 8) = Bs[j][s];
+        }
       }
     }
     // delta = U + (-W) S: 4 x SPW independent row-tile chains sharing each -W fragment
@@ -1302,7 +1458,7 @@ __global__ __launch_bounds__(kSegThreads) void chunk_fwd_seg_kernel(FwdArgs a, i
     for (int j = 0; j < SPW; ++j) {
       D[j][0] = pack_tiles(dl[j][0], dl[j][1]);
       D[j][1] = pack_tiles(dl[j][2], dl[j][3]);
-      if (REPLAY) {
+      if (REPLAY && !(OUT && a.infer)) {
         bf16* DLF = (bf16*)a.ws.p[R_DLF] + tile * 64 * V + (size_t)strip[j] * 16 * 64;
         *(bf16x8*)(DLF + (size_t)lane * 8) = D[j][0];
         *(bf16x8*)(DLF + (size_t)(64 + lane) * 8) = D[j][1];
@@ -1324,6 +1480,22 @@ __global__ __launch_bounds__(kSegThreads) void chunk_fwd_seg_kernel(FwdArgs a, i
     for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
       for (int j = 0; j < SPW; ++j) S[j][kt] = mfma16(kf[kt][1], D[j][1], S[j][kt]);
+    if constexpr (OUT) {
+      __builtin_amdgcn_sched_barrier(0);  // (the step's other operands are dead by now)
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) {
+        bf16x8 fq[NB], fa[2];
+#pragma unroll
+        for (int s = 0; s < NB; ++s) fq[s] = *(const bf16x8*)(slot + C::off_qg + ((rt * NB + s) * 64 + lane) * 16);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) fa[s] = *(const bf16x8*)(slot + C::off_a + ((rt * 2 + s) * 64 + lane) * 16);
+#pragma unroll
+        for (int j = 0; j < SPW; ++j) {
+          const bf16x4 x = out_tile<K>(fq, fa, Bs[j], D[j]);
+          store_out<V>(a, row0 + ci * kChunk, tokens - ci * kChunk, h, 16 * strip[j], rt, x, lane);
+        }
+      }
+    }
   }
   ring_barrier();  // B(steps)
   // segment end
@@ -1530,6 +1702,27 @@ ChunkGeom make_geom(const kda_chunk_problem* p) {
   return g;
 }
 
+// Whether the scan (or the segment replay) forms the outputs, rather than a launch after it.
+// Where the scan leaves CUs idle its steps are a chain of latencies, which the output waves
+// lengthen, and a launch of its own has the whole chip; where it does not, the histories cost
+// more than the products.  Forward with -> without histories kept for a gradient, launches
+// apart -> here, us: one pass, K = V = 128, T1024 H3: 24 recurrences (192 strips) 48.9 -> 46.5
+// and 50.1 -> 52.1, 48 73.8 -> 59.1 and 83.3 -> 67.4, 192 301 -> 227 and 395 -> 315; K = V = 64:
+// 48 (192 strips) 46.5 -> 45.6 and 48.8 -> 49.8, 72 69.4 -> 59.3 and 73.5 -> 64.8.  Short chains
+// save the launch: 1 to 4 chunks 0.88 to 0.98 of the time, 8 chunks 0.95 to 1.06.  Segmented,
+// K = V = 128: T8192 H2 (44 workgroups) 71.3 -> 70.0 and 79.5 -> 79.0, H4 (88) 84.1 -> 79.4 and
+// 91.8 -> 88.2; T32768 H1 (46) 112 -> 112 and 124 -> 125, H4 (184) 233 -> 202 and 299 -> 282;
+// K = V = 64, T32768 H3 (69) 111 -> 107 and 128 -> 133, H4 (92) 126 -> 120 and 147 -> 143.
+constexpr int kOutChunks = 4;      // one pass: chains this short always
+constexpr int kOutStrips = 256;    // one pass: recurrences x V/16 strips from which it gains
+constexpr int kOutSegGroups = 80;  // segmented: replay workgroups from which it gains
+
+static bool scan_forms_output(const kda_chunk_problem* p, const ChunkGeom& g) {
+  const long nrec = (long)p->num_seqs * p->heads;
+  if (g.seg_len > 0) return nrec * g.max_segs * (p->value_dim / 64) >= kOutSegGroups;
+  return p->seq_len <= kOutChunks * kChunk || nrec * (p->value_dim / 16) >= kOutStrips;
+}
+
 template <int K, int V>
 static int launch_forward(const kda_chunk_problem* p, const ChunkGeom& g, FwdArgs& a,
                           hipStream_t stream, int stages) {
@@ -1544,9 +1737,12 @@ static int launch_forward(const kda_chunk_problem* p, const ChunkGeom& g, FwdArg
     hipLaunchKernelGGL(intra, dim3(g.max_chunks, p->heads), dim3(kIntraThreads), smem, stream, a);
     KDA_LAUNCH_CHECK("chunk_forward intra");
   }
-  if (p->num_seqs > 0 && (stages & (1 << KDA_STAGE_FWD_SCAN))) {
-    auto scan = chunk_fwd_scan_kernel<K, V>;
-    constexpr size_t smem = ScanLds<K, V>::bytes;
+  // the scan forms the outputs itself unless the norm needs whole rows (the output stage alone
+  // then runs that scan; the scan stage alone writes the histories the output kernel reads)
+  const bool fuse = a.ng_out == nullptr && (stages >> KDA_STAGE_FWD_OUTPUT & 1) && scan_forms_output(p, g);
+  if (p->num_seqs > 0 && (fuse || (stages & (1 << KDA_STAGE_FWD_SCAN)))) {
+    auto scan = fuse ? chunk_fwd_scan_kernel<K, V, true> : chunk_fwd_scan_kernel<K, V, false>;
+    const size_t smem = fuse ? ScanLds<K, V, true>::bytes : ScanLds<K, V, false>::bytes;
     {
       hipError_t e = ensure_lds_limit((const void*)scan, (int)smem);
       if (e != hipSuccess)
@@ -1554,16 +1750,18 @@ static int launch_forward(const kda_chunk_problem* p, const ChunkGeom& g, FwdArg
     }
     const int nrec = p->num_seqs * p->heads;
     if (g.seg_len == 0) {
-      const int grid = kXcds * (V / 16) * ((nrec + kXcds - 1) / kXcds);
-      hipLaunchKernelGGL(scan, dim3(grid), dim3(kScanThreads), smem, stream, a);
+      const int groups = V / 16 / (fuse ? ScanLds<K, V, true>::NST : 1);
+      const int grid = kXcds * groups * ((nrec + kXcds - 1) / kXcds);
+      hipLaunchKernelGGL(scan, dim3(grid), dim3(fuse ? kScanOutThreads : kScanThreads), smem, stream, a);
       KDA_LAUNCH_CHECK("chunk_forward scan");
     } else {
       auto local = chunk_fwd_seg_kernel<K, V, false>;
-      auto replay = chunk_fwd_seg_kernel<K, V, true>;
+      auto replay = fuse ? chunk_fwd_seg_kernel<K, V, true, true> : chunk_fwd_seg_kernel<K, V, true, false>;
       using CL = SegCfg<K, V, false>;
-      using CR = SegCfg<K, V, true>;
+      using CR = SegCfg<K, V, true, false>;
+      const int replay_lds = fuse ? SegCfg<K, V, true, true>::bytes : CR::bytes;
       if (ensure_lds_limit((const void*)local, (int)CL::bytes) != hipSuccess ||
-          ensure_lds_limit((const void*)replay, (int)CR::bytes) != hipSuccess)
+          ensure_lds_limit((const void*)replay, replay_lds) != hipSuccess)
         return set_error(KDA_ERR_LAUNCH, "chunk_forward: segmented scan LDS attribute failed");
       const int nrs = nrec * g.max_segs;
       hipLaunchKernelGGL(local, dim3(kXcds * CL::GROUPS * ((nrs + kXcds - 1) / kXcds)), dim3(kSegThreads),
@@ -1584,11 +1782,11 @@ static int launch_forward(const kda_chunk_problem* p, const ChunkGeom& g, FwdArg
       hipLaunchKernelGGL(comb, dim3(kXcds * (V / 16) * ((nrec + kXcds - 1) / kXcds)), dim3(kCombThreads), 0, stream, c);
       KDA_LAUNCH_CHECK("chunk_forward segment combine");
       hipLaunchKernelGGL(replay, dim3(kXcds * CR::GROUPS * ((nrs + kXcds - 1) / kXcds)), dim3(kSegThreads),
-                         CR::bytes, stream, a, g.seg_len, g.max_segs);
+                         replay_lds, stream, a, g.seg_len, g.max_segs);
       KDA_LAUNCH_CHECK("chunk_forward segment replay");
     }
   }
-  if (g.max_chunks > 0 && (stages & (1 << KDA_STAGE_FWD_OUTPUT))) {
+  if (g.max_chunks > 0 && !fuse && (stages & (1 << KDA_STAGE_FWD_OUTPUT))) {
     auto outk = chunk_fwd_output_kernel<K, V>;
     hipLaunchKernelGGL(outk, dim3(g.max_chunks, p->heads), dim3(256), 0, stream, a);
     KDA_LAUNCH_CHECK("chunk_forward output");

@@ -287,6 +287,7 @@ int kda_cast_weights_bf16(int32_t n, const float* const* src, const int64_t* cou
  * measurement only).  Forward stages: KDA_STAGE_PREP, KDA_STAGE_FWD_INTRA,
  * KDA_STAGE_FWD_SCAN, KDA_STAGE_FWD_OUTPUT; backward stages: KDA_STAGE_BWD_SCAN, KDA_STAGE_BWD_DENSE,
  * KDA_STAGE_BWD_DECAY, KDA_STAGE_BWD_PARAMS.  Arguments are those of the full calls.
+ * Where the full call's scan forms the outputs itself, KDA_STAGE_FWD_OUTPUT runs that scan.
  */
 #define KDA_STAGE_PREP 0
 #define KDA_STAGE_FWD_INTRA 1

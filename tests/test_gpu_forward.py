@@ -335,3 +335,34 @@ def test_forward_without_residuals(B, T, H, KV, gate, scale_g):
     out2, fin2 = run(*a[:2], v, *a[3:])
     assert torch.equal(out, out2) and torch.equal(fin, fin2) and out2.requires_grad and not out.requires_grad
     assert torch.isfinite(torch.autograd.grad(out2.float().sum(), v)[0].float()).all()
+
+
+@pytest.mark.parametrize("infer", [False, True])
+@pytest.mark.parametrize("lens,H,KV", [([1], 1, (128, 128)),                   # one chunk of one token
+                                       ([256, 3, 65, 0, 130], 2, (64, 128)),   # packed, 4 chunks at most but by total
+                                       ([256], 2, (64, 64)),                   # 4 chunks, the longest short chain
+                                       ([449] * 32, 1, (128, 128)),            # 256 strips, 8 chunks, the last one token
+                                       ([200, 64, 321, 77] * 16, 1, (128, 64)),
+                                       ([6400, 6143], 4, (128, 128)),          # segmented replay, ragged ends
+                                       ([6145] * 20, 1, (64, 64))])
+def test_outputs_from_the_scan_equal_the_output_kernel(lens, H, KV, infer):
+    """Where the scan forms the outputs, they are bit for bit those of the output kernel, which
+    the call with the fused norm still launches (the same products, the same order of sums),
+    and the histories give bit for bit the same gradients."""
+    K, V = KV
+    fixed = len(set(lens)) == 1
+    B, T, n = (len(lens), lens[0], len(lens)) if fixed else (1, sum(lens), len(lens))
+    d = make_kda_inputs(B, T, H, K, V, seed=61)
+    cu = None if fixed else torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda")
+    g = torch.Generator().manual_seed(62)
+    s0 = 0.1 * torch.randn(n, H, V, K, generator=g).cuda()
+    args = (d["q"], d["k"], d["v"], d["g"], d["beta"], d["A_log"], d["dt_bias"], s0)
+    out, fin, ws = ops.chunk_forward(*args, True, -5.0, K ** -0.5, cu_seqlens=cu, gate="k3", residuals=not infer)
+    o2, _, _, f2, ws2 = ops.chunk_forward_norm_gate(*args, True, -5.0, K ** -0.5, torch.ones_like(d["v"]),
+                                                    torch.ones(V, device="cuda"), 1e-5, cu_seqlens=cu, gate="k3")
+    assert torch.equal(out, o2) and torch.equal(fin, f2)
+    if not infer:
+        do = torch.randn(d["v"].shape, generator=g).bfloat16().cuda()
+        for a, b in zip(*(ops.chunk_backward(*args, w, do, None, -5.0, K ** -0.5, cu_seqlens=cu, gate="k3")
+                          for w in (ws, ws2))):
+            assert torch.equal(a, b)
