@@ -449,6 +449,16 @@ def pmc_workload(torch):
                  gate="precomputed", allow_fallback=False)
     out.backward(do)
     torch.cuda.synchronize()
+    # the fused launch, which captured calls run (the eager backward above ran the separate launches)
+    scale = t["q"].shape[-1] ** -0.5
+    args = [t[n].detach() for n in ("q", "k", "v", "g", "beta", "A_log", "dt_bias")]
+    _, _, ws = ops.chunk_forward(*args, None, False, -5.0, scale, gate="precomputed")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        keep = ops.chunk_backward_launch(*args, None, ws, do, None, -5.0, scale, gate="precomputed")
+    graph.replay()
+    torch.cuda.synchronize()
+    del keep
     g = torch.Generator(device="cuda").manual_seed(1)
     x, dy, gt = (torch.randn(2, 4096, 384, device="cuda", generator=g).bfloat16() for _ in range(3))
     w = torch.randn(384, 4, device="cuda", generator=g).bfloat16()
