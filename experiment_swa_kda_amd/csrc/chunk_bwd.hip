@@ -405,7 +405,7 @@ enum ScanMode { kScanWhole, kScanLocal, kScanReplay };
 
 // Hand-off of the segmented scan, in the scratch regions that only the separate dense and
 // decay launches use (no scratch of its own; bwd_segmented checks that it fits):
-//   P     bf16 [rec][segment][hi, lo] K x K A fragments, permuted      (S_DQG)
+//   P     f32  [rec][segment] K x K in f32_frag_elem order             (S_DQG)
 //   sigma f32  [rec][segment][V][K]                                    (S_DKD)
 //   xin   f32  [rec][segment][V][K], segments >= 1                     (S_DKB)
 struct SegArgs {
@@ -692,16 +692,12 @@ __device__ __forceinline__ void bwd_scan_body(const BwdArgs& a, int* progress, c
       for (int kt = 0; kt < KT; ++kt)
         *(float4*)(sg_out + 16 * (cw * KT + kt) + 4 * kg) = make_float4(X[kt][0], X[kt][1], X[kt][2], X[kt][3]);
     } else {
-      bf16* hi = (bf16*)a.sc.p[S_DQG] + (size_t)rseg * 2 * K * K;
+      float* P = (float*)a.sc.p[S_DQG] + (size_t)rseg * K * K;
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const size_t o = perm_frag_elem(K, 16 * (cw * KT + kt) + 4 * kg + q, 16 * (sg - V / 16) + lr);
-          const bf16 x = to_bf16(X[kt][q]);
-          hi[o] = x;
-          hi[(size_t)K * K + o] = to_bf16(X[kt][q] - to_f32(x));
-        }
+        for (int q = 0; q < 4; ++q)
+          P[f32_frag_elem(K, 16 * (cw * KT + kt) + 4 * kg + q, 16 * (sg - V / 16) + lr)] = X[kt][q];
     }
     return;
   }
@@ -2078,11 +2074,13 @@ static long long wait_limit_ticks() {
 }
 
 // Segments of the reverse scan (len 0: whole sequences in one pass): the forward's segments,
-// where the strips are few enough that two shorter passes beat the one long chain (whole K3
-// backward, K = V = 128, without and with segments): 345 -> 168 us at 8 strips x 512 chunks
-// (B1 T32768 H1), 122 -> 95 at 16 x 128, 432 -> 395 at 24 x 512 and 132 -> 133 at 24 x 128; at
-// 32 x 128 the fused launch takes 135 us, segments 149.  The hand-off must fit the scratch
-// regions it borrows (see SegArgs): at most max_chunks / 2 segments in all.
+// where the strips are few enough that two shorter passes beat the one long chain.  Whole K3
+// backward, K = V = 128, us, without and with segments: eager 317 -> 161 at 8 strips x 512
+// chunks (B1 T32768 H1), 103 -> 81 at 8 x 128, 110 -> 91 at 16 x 128, 491 -> 381 at 24 x 512 and
+// 143 -> 126 at 24 x 128; captured, where the fused launch is the other form, 514 -> 164, 140 ->
+// 85, 184 -> 95, 440 -> 385 and 129 -> 129.  At 32 x 128 the two forms without segments take 149
+// and 135 us, segments 149.  The hand-off must fit the scratch regions it borrows (see SegArgs):
+// at most max_chunks / 2 segments in all.
 constexpr long kBwdSegStrips = 24;
 static SegArgs bwd_segments(const ChunkGeom& g) {
   SegArgs sa;
@@ -2158,7 +2156,7 @@ static int launch_seg_scan(const BwdArgs& a, const SegArgs& sa, hipStream_t stre
   c.max_segs = sa.max;
   c.seqs = (const int2*)a.ws.p[R_SEQS];
   c.start = a.dsfin;
-  c.P = (const bf16*)a.sc.p[S_DQG];
+  c.P = a.sc.p[S_DQG];
   c.sigma = (const float*)a.sc.p[S_DKD];
   c.out = (float*)a.sc.p[S_DKB];
   auto comb = seg_combine_kernel<K, V, true>;

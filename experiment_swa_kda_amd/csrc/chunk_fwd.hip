@@ -1775,7 +1775,7 @@ static int launch_forward(const kda_chunk_problem* p, const ChunkGeom& g, FwdArg
       c.max_segs = g.max_segs;
       c.seqs = (const int2*)a.ws.p[R_SEQS];
       c.start = a.s0;
-      c.P = (const bf16*)a.ws.p[R_SEGP];
+      c.P = a.ws.p[R_SEGP];
       c.sigma = (const float*)a.ws.p[R_SEGS];
       c.out = (float*)a.ws.p[R_SIN];
       auto comb = seg_combine_kernel<K, V, false>;

@@ -37,6 +37,11 @@ __host__ __device__ inline size_t perm_frag_elem(int C, int row, int col) {
   const int e = 4 * ((col % 32) / 16) + col % 4;
   return (((size_t)(row / 16) * (C / 32) + col / 32) * 64 + lane) * 8 + e;
 }
+// f32 operand of v_mfma_f32_16x16x4_f32, 16 x 16 blocks: lane l holds X[row l%16][4(l/16) ..  + 3].
+__host__ __device__ inline size_t f32_frag_elem(int C, int row, int col) {
+  const int lane = row % 16 + 16 * ((col % 16) / 4);
+  return (((size_t)(row / 16) * (C / 16) + col / 16) * 64 + lane) * 4 + col % 4;
+}
 
 // Arrays marked "permuted" keep their fragment shape but order each 32-wide step of the
 // contraction index as 32s + 16(e/4) + 4(l/16) + e%4 for element e of lane l (instead of

@@ -8,10 +8,15 @@ namespace kda {
 
 // S_in(j+1) = P_j S_in(j) + Sigma_j over the segments of one recurrence.  One workgroup per
 // (recurrence, V strip); wave w owns state tiles w * TPW .. (w + 1) * TPW - 1.  Each step the
-// waves publish their tiles as hi + lo bf16 B-operand halves in LDS (about 16 mantissa
-// bits of the state), one barrier, and every wave multiplies its rows of P_j (bf16
-// fragments written by the local kernel, requested a batch of steps ahead) by the whole state.
-// LO: P_j comes as hi + lo bf16 too (the reverse scan, whose one-pass form carries lam X in f32).
+// waves publish their tiles as B operands in LDS, one barrier, and every wave multiplies its
+// rows of P_j (fragments written by the local kernel, requested several steps ahead) by the
+// whole state.
+// F32 = false (the forward): P_j in bf16, the state as hi + lo bf16 halves (about 16 mantissa bits).
+// F32 = true (the reverse scan, whose one-pass form carries lam X in f32): both stay f32, on
+// v_mfma_f32_16x16x4_f32.  The step (tile kt, r) contracts keys 16 kt + 4 (l / 16) + r: the
+// state's operand is the accumulator register it already lies in.  At 23 dependent steps (B1
+// T32768 H1, K = V = 128) the f32 form takes 39 us and the bf16 form 21; with the sets requested
+// a batch at a time, so that each batch began with a memory round trip, 53 and 31.
 constexpr int kCombThreads = 4 * kWave;
 
 struct CombineArgs {
@@ -20,17 +25,91 @@ struct CombineArgs {
   int seg_len, max_segs; // chunks per segment, segments of the longest sequence
   const int2* seqs;      // {first chunk, chunk count} per sequence (fixed_T == 0)
   const float* start;    // [num_seqs][H][V][K] value entering segment 0, or null (zero)
-  const bf16* P;         // [rec][segment] K x K (LO: then its low part), rec = sequence * H + head
+  const void* P;         // [rec][segment] K x K, rec = sequence * H + head: bf16 in perm_frag_elem
+                         // order, F32: f32 in f32_frag_elem order
   const float* sigma;    // [rec][segment][V][K]
   float* out;            // [rec][segment][V][K], segments >= 1
 };
 
-template <int K, int V, bool LO>
+template <int K, bool F32>
+struct CombOps;
+
+template <int K>
+struct CombOps<K, false> {
+  static constexpr int NB = K / 32, TPW = K / 64, kAhead = 8;
+  static constexpr int lds = 2 * NB * kWave * 16;  // [hi/lo][fragment]
+  bf16x8 p[TPW][NB];
+  __device__ void load(const void* P, size_t seg, int wave, int lane) {
+    const bf16* q = (const bf16*)P + seg * K * K;
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+      for (int s = 0; s < NB; ++s) p[t][s] = *(const bf16x8*)(q + (((size_t)(wave * TPW + t) * NB + s) * 64 + lane) * 8);
+  }
+  static __device__ void publish(char* buf, int kt, int lane, const f32x4& S) {
+    bf16x4 hi, lo;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      hi[r] = to_bf16(S[r]);
+      lo[r] = to_bf16(S[r] - to_f32(hi[r]));
+    }
+    char* d = buf + (kt / 2) * (kWave * 16) + lane * 16 + (kt % 2) * 8;
+    *(bf16x4*)d = hi;
+    *(bf16x4*)(d + NB * kWave * 16) = lo;
+  }
+  __device__ void apply(const char* buf, int lane, f32x4 (&acc)[TPW]) const {
+    bf16x8 hi[NB], lo[NB];
+#pragma unroll
+    for (int s = 0; s < NB; ++s) {
+      hi[s] = *(const bf16x8*)(buf + (s * kWave + lane) * 16);
+      lo[s] = *(const bf16x8*)(buf + ((NB + s) * kWave + lane) * 16);
+    }
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+      for (int s = 0; s < NB; ++s) {
+        acc[t] = mfma16(p[t][s], hi[s], acc[t]);
+        acc[t] = mfma16(p[t][s], lo[s], acc[t]);
+      }
+  }
+};
+
+template <int K>
+struct CombOps<K, true> {
+  static constexpr int KT = K / 16, TPW = K / 64, kAhead = 4;
+  static constexpr int lds = KT * kWave * 16;  // [tile] in accumulator order
+  f32x4 p[TPW][KT];
+  __device__ void load(const void* P, size_t seg, int wave, int lane) {
+    const float* q = (const float*)P + seg * K * K;
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+        p[t][kt] = *(const f32x4*)(q + (((size_t)(wave * TPW + t) * KT + kt) * 64 + lane) * 4);
+  }
+  static __device__ void publish(char* buf, int kt, int lane, const f32x4& S) {
+    *(f32x4*)(buf + (kt * kWave + lane) * 16) = S;
+  }
+  __device__ void apply(const char* buf, int lane, f32x4 (&acc)[TPW]) const {
+    f32x4 x[KT];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) x[kt] = *(const f32x4*)(buf + (kt * kWave + lane) * 16);
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[t][kt][r], x[kt][r], acc[t], 0, 0, 0);
+  }
+};
+
+template <int K, int V, bool F32>
 __global__ __launch_bounds__(kCombThreads) void seg_combine_kernel(CombineArgs a) {
-  constexpr int kParts = LO ? 2 : 1, kCombBatch = LO ? 4 : 8;
+  using Ops = CombOps<K, F32>;
+  constexpr int VS = V / 16, TPW = Ops::TPW, kAhead = Ops::kAhead;
   const int max_segs = a.max_segs;
-  constexpr int KT = K / 16, NB = K / 32, VS = V / 16, TPW = KT / 4;
-  __shared__ __attribute__((aligned(16))) char sB[2][2][NB][kWave * 16];  // [parity][hi/lo][frag]
+  __shared__ __attribute__((aligned(16))) char sB[2][Ops::lds];  // [parity]
   const int H = a.H;
   int rec, strip;
   if (!xcd_strip_coords(a.num_seqs * H, VS, rec, strip)) return;
@@ -51,83 +130,42 @@ __global__ __launch_bounds__(kCombThreads) void seg_combine_kernel(CombineArgs a
       S[t] = zero4();
     }
   }
-  const bf16* P0 = a.P + (size_t)rec * max_segs * kParts * K * K;
-  const float* G0 = a.sigma + (size_t)rec * max_segs * V * K + (size_t)v * K;
-  // every step's P rows and Sigma for this wave, requested up front in batches of
-  // kCombBatch steps (one memory round trip per batch instead of one per step)
-  bf16x8 pa[kCombBatch][kParts][TPW][NB];
-  float4 sg[kCombBatch][TPW];
-  for (int j = 0; j + 1 < nseg; ++j) {
-    const int jb = j % kCombBatch;
-    if (jb == 0) {
+  const size_t seg0 = (size_t)rec * max_segs;
+  const float* G0 = a.sigma + seg0 * V * K + (size_t)v * K;
+  // the P rows and Sigma of the next kAhead steps in registers or in flight: a step's set is
+  // requested again as soon as it is used
+  Ops pa[kAhead];
+  float4 sg[kAhead][TPW];
+  auto fetch = [&](int b, int j) {
+    const int jj = min(j, nseg - 2);
+    pa[b].load(a.P, seg0 + jj, wave, lane);
 #pragma unroll
-      for (int b = 0; b < kCombBatch; ++b) {
-        const int jj = min(j + b, nseg - 2);
+    for (int t = 0; t < TPW; ++t) sg[b][t] = *(const float4*)(G0 + (size_t)jj * V * K + 16 * (wave * TPW + t) + 4 * kg);
+  };
 #pragma unroll
-        for (int t = 0; t < TPW; ++t) {
-          const int kt = wave * TPW + t;
+  for (int b = 0; b < kAhead; ++b) fetch(b, b);
+  for (int j0 = 0;; j0 += kAhead) {
 #pragma unroll
-          for (int u = 0; u < kParts; ++u)
+    for (int b = 0; b < kAhead; ++b) {
+      const int j = j0 + b;
+      if (j + 1 >= nseg) return;
+      char* buf = sB[j & 1];
 #pragma unroll
-            for (int s = 0; s < NB; ++s)
-              pa[b][u][t][s] = *(const bf16x8*)(P0 + ((size_t)jj * kParts + u) * K * K + (((size_t)kt * NB + s) * 64 + lane) * 8);
-          sg[b][t] = *(const float4*)(G0 + (size_t)jj * V * K + 16 * kt + 4 * kg);
-        }
+      for (int t = 0; t < TPW; ++t) Ops::publish(buf, wave * TPW + t, lane, S[t]);
+      // LDS only: a fence-free barrier (the loads ahead and earlier stores stay in flight)
+      wait_lgkm0();
+      ring_barrier();
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+        S[t][0] = sg[b][t].x; S[t][1] = sg[b][t].y; S[t][2] = sg[b][t].z; S[t][3] = sg[b][t].w;
       }
+      pa[b].apply(buf, lane, S);
+      fetch(b, j + kAhead);
+      float* out = a.out + (seg0 + j + 1) * V * K + (size_t)v * K;
+#pragma unroll
+      for (int t = 0; t < TPW; ++t)
+        *(float4*)(out + 16 * (wave * TPW + t) + 4 * kg) = make_float4(S[t][0], S[t][1], S[t][2], S[t][3]);
     }
-    char(*buf)[NB][kWave * 16] = sB[j & 1];
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      const int kt = wave * TPW + t;
-      bf16x4 hi, lo;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        hi[r] = to_bf16(S[t][r]);
-        lo[r] = to_bf16(S[t][r] - to_f32(hi[r]));
-      }
-      *(bf16x4*)(buf[0][kt / 2] + lane * 16 + (kt % 2) * 8) = hi;
-      *(bf16x4*)(buf[1][kt / 2] + lane * 16 + (kt % 2) * 8) = lo;
-    }
-    // LDS only: a fence-free barrier (the prefetched loads and earlier stores stay in flight)
-    wait_lgkm0();
-    ring_barrier();
-    bf16x8 Bh[NB], Bl[NB];
-#pragma unroll
-    for (int s = 0; s < NB; ++s) {
-      Bh[s] = *(const bf16x8*)(buf[0][s] + lane * 16);
-      Bl[s] = *(const bf16x8*)(buf[1][s] + lane * 16);
-    }
-    // pick this step's operands (jb is uniform; unrolled select keeps them in registers)
-    bf16x8 pc[kParts][TPW][NB];
-    float4 gc[TPW];
-#pragma unroll
-    for (int b = 0; b < kCombBatch; ++b)
-      if (b == jb) {
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) {
-          gc[t] = sg[b][t];
-#pragma unroll
-          for (int u = 0; u < kParts; ++u)
-#pragma unroll
-            for (int s = 0; s < NB; ++s) pc[u][t][s] = pa[b][u][t][s];
-        }
-      }
-#pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      f32x4 acc;
-      acc[0] = gc[t].x; acc[1] = gc[t].y; acc[2] = gc[t].z; acc[3] = gc[t].w;
-#pragma unroll
-      for (int s = 0; s < NB; ++s) {
-        acc = mfma16(pc[0][t][s], Bh[s], acc);
-        acc = mfma16(pc[0][t][s], Bl[s], acc);
-        if constexpr (LO) acc = mfma16(pc[kParts - 1][t][s], Bh[s], acc);
-      }
-      S[t] = acc;
-    }
-    float* out = a.out + ((size_t)rec * max_segs + j + 1) * V * K + (size_t)v * K;
-#pragma unroll
-    for (int t = 0; t < TPW; ++t)
-      *(float4*)(out + 16 * (wave * TPW + t) + 4 * kg) = make_float4(S[t][0], S[t][1], S[t][2], S[t][3]);
   }
 }
 

@@ -449,6 +449,23 @@ def test_segmented_reverse_scan(lens, H, KV, gate):
     check(gpu_grads(d, gate, do, dsT, cu), oracle_grads(d, gate, do, dsT, cu))
 
 
+@pytest.mark.parametrize("lens,H,KV", [([6400], 3, (128, 128)), ([5000, 0, 1300, 100], 1, (64, 64)),
+                                        ([3001, 3500], 1, (64, 128)), ([8192], 2, (128, 64))])
+def test_segment_hand_off_keeps_f32(lens, H, KV):
+    """With no decay (g = 0), no write (beta = 0) and no output gradient a chunk maps the state
+    gradient to itself, exactly: lam = 1, G = 0, E = 0.  The segmented reverse scan carries it in
+    f32 from segment to segment, so the final-state gradient arrives bit for bit."""
+    K, V = KV
+    T, n = sum(lens), len(lens)
+    d = make_kda_inputs(1, T, H, K, V, seed=T, gate="precomputed", state=True, dist="baseline")
+    cu = torch.tensor(np.cumsum([0] + lens), dtype=torch.int32, device="cuda") if n > 1 else None
+    d["g"] = torch.zeros_like(d["g"])
+    d["beta"] = torch.full_like(d["beta"], -200.0)
+    d["s0"] = torch.randn(n, H, V, K, generator=torch.Generator().manual_seed(3)).cuda()
+    do, dsT = cotangents(d, 11, n_states=n)
+    assert torch.equal(gpu_grads(d, "precomputed", torch.zeros_like(do), dsT, cu)[7], dsT)
+
+
 def test_captured_call_equals_eager_call():
     """A problem of more than a round of tiles uses the fused launch under capture and the
     separate launches outside it (kda_chunk_backward_waits); the gradients of every replay
