@@ -32,6 +32,8 @@ from dataclasses import dataclass
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import ops
 
@@ -72,10 +74,26 @@ def _needs_grad(*tensors):
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
 
-def _untransformed():
-    """No forward-mode level and no functorch transform is active: the autograd functions are
-    what accepts or refuses those, so paths without one ask first."""
-    return torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+_PLAIN_TENSORS = (torch.Tensor, nn.Parameter)
+
+
+def _untransformed(*tensors):
+    """Whether a call on these tensors may skip the autograd functions and library operators of
+    the general path.  Those are what a tracer, a dispatch or function mode, a functorch
+    transform, a forward-mode level, autocast to another type or a tensor subclass (a fake
+    tensor) sees, converts or refuses; a kernel launched beside them would go unseen."""
+    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None:
+        return False
+    if torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    if torch._C._len_torch_dispatch_stack():
+        return False
+    # (torch.device as a context or default is a function mode that changes no call of ours)
+    if torch._C._len_torch_function_stack() and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()):
+        return False
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16:
+        return False
+    return all(t is None or type(t) in _PLAIN_TENSORS for t in tensors)
 
 
 class _LinearBF16(torch.autograd.Function):
@@ -165,18 +183,19 @@ class Linear(nn.Linear):
         bias = None if self.bias is None else self.bias.to(dtype=x.dtype)
         return F.linear(x, self.weight.to(dtype=x.dtype), bias)
 
-    def _few_rows_ok(self, x):
-        return (x.numel() <= 64 * self.in_features and self.bias is None and not _needs_grad(x, self.weight)
-                and _untransformed() and self.weight.device == x.device)
+    def _few_rows_ok(self, x, residual=None):
+        return (x.shape[-1:] == (self.in_features,) and x.numel() <= 64 * self.in_features and self.bias is None
+                and not _needs_grad(x, self.weight, residual) and _untransformed(x, self.weight, residual)
+                and self.weight.device == x.device)
 
     def few_rows(self, x, *, relu2=False, residual=None):
         """``relu(y)^2`` or ``residual + y`` of y = self(x) in one kernel, for the few rows of a
         decode step; None where that kernel does not apply (or a hook wants to see y)."""
         w16 = getattr(self, "_w16", None)
         if (w16 is None or not x.is_cuda or x.dtype != torch.bfloat16 or self._forward_hooks or self._forward_pre_hooks
-                or not self._few_rows_ok(x) or not ops.linear_rows_gains(x, w16)):
+                or not self._few_rows_ok(x, residual) or not ops.linear_rows_gains(x, w16)):
             return None
-        if residual is not None and (residual.dtype != x.dtype or _needs_grad(residual)):
+        if residual is not None and residual.dtype != x.dtype:
             return None
         return ops.linear_rows(x, w16, relu2=relu2, residual=residual)
 
@@ -824,6 +843,9 @@ class KimiDeltaAttention(nn.Module):
         if any(type(m) is not Linear or m.bias is not None for m in linears):
             return False
         params = [self.o_norm.weight, self.A_log, self.dt_bias]
+        carried = () if prompt else (state.memory, state.q_conv, state.k_conv, state.v_conv)
+        if not _untransformed(x, *params, *(m.weight for m in linears), *carried):
+            return False
         cached = self._cached16()
         if cached is None or torch.is_grad_enabled():
             params += [m.weight for m in (*linears, self.q_conv1d, self.k_conv1d, self.v_conv1d)]
@@ -832,15 +854,12 @@ class KimiDeltaAttention(nn.Module):
         if any(p.dtype != torch.float32 or p.device != x.device or not p.is_contiguous() or p.data_ptr() % 16
                for p in params):
             return False
-        carried = () if prompt else (state.memory, state.q_conv, state.k_conv, state.v_conv)
         for t, shape, dtype in zip(carried, ((n_b, H, D, D),) + ((n_b, C, 4),) * 3,
                                    (torch.float32,) + (torch.bfloat16,) * 3):
             if t.shape != shape or t.dtype != dtype or t.device != x.device or not t.is_contiguous() \
                     or t.data_ptr() % 16:
                 return False
-        if _needs_grad(x, *params, *carried):
-            return False
-        return _untransformed()
+        return not _needs_grad(x, *params, *carried)
 
     def _cached16(self):
         cached = (getattr(self, "_w16_in", None), getattr(self, "_conv_w16", None),
@@ -869,7 +888,7 @@ class KimiDeltaAttention(nn.Module):
         """Whether _weights16 can cast: f32 weights of multiples of 8 elements, as laid out."""
         ws = (*self._in_weights(), self.q_conv1d.weight, self.k_conv1d.weight, self.v_conv1d.weight,
               self.f_b_proj.weight, self.o_proj.weight)
-        return type(self.o_proj) is Linear and self.hidden_size % 8 == 0 and all(
+        return type(self.o_proj) is Linear and self.hidden_size % 8 == 0 and _untransformed(*ws) and all(
             w.dtype == torch.float32 and w.is_contiguous() and w.numel() % 8 == 0 and w.data_ptr() % 16 == 0 for w in ws)
 
     def _forward_inference(self, x, state, keep_state, state_in_place):

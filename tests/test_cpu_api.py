@@ -13,7 +13,7 @@ import torch
 
 import experiment_swa_kda_amd as kmod
 from experiment_swa_kda_amd import _lib
-from experiment_swa_kda_amd.kda import KDAState, KimiDeltaAttention, k3_decay_gate, kda
+from experiment_swa_kda_amd.kda import KDAState, KimiDeltaAttention, Linear, k3_decay_gate, kda
 from oracle import kda_oracle as O
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -318,3 +318,18 @@ def test_gemm_selection_file_is_pinned_to_gfx950():
     assert {"PT_VERSION", "HIPBLASLT_VERSION", "ROCBLAS_VERSION"} <= set(val)
     assert any(",tn_32768_8192_384_" in l for l in lines)
     assert os.path.basename(model.GEMM_SELECTION_FILE) == "gemm_selection_gfx950.csv"
+
+
+@pytest.mark.parametrize("rows", [8, 100])
+def test_linear_of_few_rows_is_seen_by_tracers_and_fake_tensors(rows):
+    """A bf16 device call of few rows runs one kernel beside the dispatcher only where nothing
+    looks: fake tensors get a shape and make_fx records the product, at 8 rows as at 100."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+    with FakeTensorMode(), torch.no_grad():
+        layer = Linear(64, 32, bias=False, device="cuda")
+        x = torch.empty(rows, 64, dtype=torch.bfloat16, device="cuda")
+        y = layer(x)
+        assert y.shape == (rows, 32) and y.dtype == torch.bfloat16 and y.is_cuda
+        graph = make_fx(lambda t: layer(t))(x).graph
+    assert any("mm" in str(n.target) or "linear" in str(n.target) for n in graph.nodes)

@@ -426,3 +426,22 @@ def test_decode_step_with_cached_weights_matches_full_forward(B):
         assert rel_err(model(idx[:, :P], kv_cache=cache), full[:, :P]) < 2e-2
         for t in range(P, T):
             assert rel_err(model(idx[:, t:t + 1], kv_cache=cache)[:, 0], full[:, t]) < 2e-2, t
+
+
+def test_linear_of_few_rows_traces():
+    """torch.jit.trace, make_fx and a dispatch mode (the operation counter) see the product of a
+    call of few rows: the traced module gives the eager result on new inputs."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+    from experiment_swa_kda_amd.kda import Linear
+    torch.manual_seed(1)
+    layer = Linear(128, 64, bias=False).cuda()
+    x, x2 = (torch.randn(8, 128, device="cuda").bfloat16() for _ in range(2))
+    with torch.no_grad():
+        y2 = layer(x2)
+        for traced in (torch.jit.trace(layer, x, check_trace=False), make_fx(lambda t: layer(t))(x)):
+            # one bf16 rounding of differently ordered f32 sums
+            assert rel_err(traced(x2), y2) < 4e-3
+        with FlopCounterMode(display=False) as counter:
+            layer(x)
+    assert counter.get_total_flops() == 2 * 8 * 128 * 64
