@@ -32,6 +32,7 @@ from dataclasses import dataclass
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules import module as _module
 from torch.overrides import _get_current_function_mode_stack
 from torch.utils._device import DeviceContext
 
@@ -94,6 +95,17 @@ def _untransformed(*tensors):
     if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16:
         return False
     return all(t is None or type(t) in _PLAIN_TENSORS for t in tensors)
+
+
+def plain(*modules):
+    """Whether calling each module is its class's own forward and nothing else: no hooks (its own
+    or for all modules) and no forward replaced on the instance.  A path that computes with a
+    module's weights instead of calling it asks this, and that its class is the one it stands for."""
+    if (_module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks
+            or _module._global_backward_pre_hooks):
+        return False
+    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                   or "forward" in m.__dict__ for m in modules)
 
 
 class _LinearBF16(torch.autograd.Function):
@@ -188,16 +200,17 @@ class Linear(nn.Linear):
                 and not _needs_grad(x, self.weight, residual) and _untransformed(x, self.weight, residual)
                 and self.weight.device == x.device)
 
-    def few_rows(self, x, *, relu2=False, residual=None):
-        """``relu(y)^2`` or ``residual + y`` of y = self(x) in one kernel, for the few rows of a
-        decode step; None where that kernel does not apply (or a hook wants to see y)."""
-        w16 = getattr(self, "_w16", None)
-        if (w16 is None or not x.is_cuda or x.dtype != torch.bfloat16 or self._forward_hooks or self._forward_pre_hooks
-                or not self._few_rows_ok(x, residual) or not ops.linear_rows_gains(x, w16)):
-            return None
-        if residual is not None and residual.dtype != x.dtype:
-            return None
-        return ops.linear_rows(x, w16, relu2=relu2, residual=residual)
+
+def linear_few_rows(m, x, *, relu2=False, residual=None):
+    """``relu(y)^2`` or ``residual + y`` of y = m(x) in one kernel, for the few rows of a decode
+    step; None where that kernel does not apply (m is no plain Linear, or its copy is not cached)."""
+    w16 = getattr(m, "_w16", None)
+    if (w16 is None or type(m) is not Linear or not plain(m) or not x.is_cuda or x.dtype != torch.bfloat16
+            or not m._few_rows_ok(x, residual) or not ops.linear_rows_gains(x, w16)):
+        return None
+    if residual is not None and residual.dtype != x.dtype:
+        return None
+    return ops.linear_rows(x, w16, relu2=relu2, residual=residual)
 
 
 def _norm_gate_eager(x, gate, weight, eps):

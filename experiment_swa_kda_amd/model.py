@@ -23,7 +23,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops
-from .kda import KDAState, KimiDeltaAttention, Linear
+from .kda import KDAState, KimiDeltaAttention, Linear, linear_few_rows, plain
 
 
 @dataclass
@@ -364,11 +364,11 @@ class MLP(nn.Module):
     def forward(self, x, residual=None):
         """The block's MLP, plus ``residual`` if given (for a decode step's few rows the
         activation and the add run in the projections' epilogues; the same values)."""
-        h = self.c_fc.few_rows(x, relu2=True)
+        h = linear_few_rows(self.c_fc, x, relu2=True)
         h = relu2(self.c_fc(x)) if h is None else h
         if residual is None:
             return self.c_proj(h)
-        y = self.c_proj.few_rows(h, residual=residual)
+        y = linear_few_rows(self.c_proj, h, residual=residual)
         return residual + self.c_proj(h) if y is None else y
 
 
@@ -404,8 +404,7 @@ class Block(nn.Module):
         xin, h = _ResidMixNorm.apply(x, x0, lam_r, lam_0, i, _RMS_EPS)
         mixed = self._mix(h, kv_cache)
         y, h2 = _AddNorm.apply(xin, mixed, _RMS_EPS)
-        return self.mlp(h2, y)
-
+        return self.mlp(h2, y) if type(self.mlp) is MLP and plain(self.mlp) else y + self.mlp(h2)
 
     def _token_ok(self, x, x0, lam_r, lam_0, kv_cache):
         """Whether a one-token step of a few sequences runs as _token: the mixer's own

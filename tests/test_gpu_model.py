@@ -445,3 +445,41 @@ def test_linear_of_few_rows_traces():
         with FlopCounterMode(display=False) as counter:
             layer(x)
     assert counter.get_total_flops() == 2 * 8 * 128 * 64
+
+
+def _small_decoder(seed=0):
+    torch.manual_seed(seed)
+    model = GPT(GPTConfig(sequence_len=64, vocab_size=512, n_layer=2, n_head=1, n_embd=128)).cuda()
+    model.init_weights()
+    with torch.no_grad():
+        for b in model.transformer.h:
+            b.attn.o_proj.weight.normal_(0, 0.03)
+            b.mlp.c_proj.weight.normal_(0, 0.03)
+    return model
+
+
+def test_mlp_hooks_and_replacements_see_the_mlp_alone():
+    """In training a hook of a block's MLP sees mlp(h), not the sum with the residual, and one
+    that takes h alone can stand in its place."""
+    model = _small_decoder()
+    idx = torch.randint(0, 512, (2, 33), device="cuda")
+    loss = model(idx[:, :-1], idx[:, 1:])
+    mlp, seen = model.transformer.h[0].mlp, []
+    handle = mlp.register_forward_hook(lambda m, args, out: seen.append((args, out)) or None)
+    hooked = model(idx[:, :-1], idx[:, 1:])
+    handle.remove()
+    (args, out), = seen
+    assert len(args) == 1 and torch.equal(out, mlp(args[0])) and torch.equal(hooked, loss)
+
+    class Stand(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, x):
+            return self.inner(x)
+
+    model.transformer.h[0].mlp = Stand(mlp)
+    assert torch.equal(model(idx[:, :-1], idx[:, 1:]), loss)
+    mlp.c_fc = Stand(mlp.c_fc)
+    assert torch.equal(model(idx[:, :-1], idx[:, 1:]), loss)
