@@ -853,7 +853,10 @@ class KimiDeltaAttention(nn.Module):
             return False
         linears = (self.q_proj, self.k_proj, self.v_proj, self.g_proj, self.f_a_proj, self.b_proj, self.f_b_proj,
                    self.o_proj)
-        if any(type(m) is not Linear or m.bias is not None for m in linears):
+        convs = (self.q_conv1d, self.k_conv1d, self.v_conv1d)
+        if any(type(m) is not Linear or m.bias is not None for m in linears) or not plain(*linears, *convs):
+            return False
+        if any(type(m) is not ShortConvolution or m.weight.shape != (C, 1, 4) for m in convs):
             return False
         params = [self.o_norm.weight, self.A_log, self.dt_bias]
         carried = () if prompt else (state.memory, state.q_conv, state.k_conv, state.v_conv)
@@ -861,7 +864,7 @@ class KimiDeltaAttention(nn.Module):
             return False
         cached = self._cached16()
         if cached is None or torch.is_grad_enabled():
-            params += [m.weight for m in (*linears, self.q_conv1d, self.k_conv1d, self.v_conv1d)]
+            params += [m.weight for m in (*linears, *convs)]
         elif any(w.device != x.device for w in cached):
             return False
         if any(p.dtype != torch.float32 or p.device != x.device or not p.is_contiguous() or p.data_ptr() % 16
@@ -898,10 +901,11 @@ class KimiDeltaAttention(nn.Module):
                 parts[3].view(d, d))
 
     def _cast_ok(self):
-        """Whether _weights16 can cast: f32 weights of multiples of 8 elements, as laid out."""
+        """Whether _weights16 can cast: f32 weights of multiples of 8 elements, as laid out (and
+        no hook of o_proj, called with its copy, that could change its weight in between)."""
         ws = (*self._in_weights(), self.q_conv1d.weight, self.k_conv1d.weight, self.v_conv1d.weight,
               self.f_b_proj.weight, self.o_proj.weight)
-        return type(self.o_proj) is Linear and self.hidden_size % 8 == 0 and _untransformed(*ws) and all(
+        return type(self.o_proj) is Linear and plain(self.o_proj) and self.hidden_size % 8 == 0 and _untransformed(*ws) and all(
             w.dtype == torch.float32 and w.is_contiguous() and w.numel() % 8 == 0 and w.data_ptr() % 16 == 0 for w in ws)
 
     def _forward_inference(self, x, state, keep_state, state_in_place):

@@ -483,3 +483,23 @@ def test_mlp_hooks_and_replacements_see_the_mlp_alone():
     assert torch.equal(model(idx[:, :-1], idx[:, 1:]), loss)
     mlp.c_fc = Stand(mlp.c_fc)
     assert torch.equal(model(idx[:, :-1], idx[:, 1:]), loss)
+
+
+def test_replaced_submodules_run_at_inference():
+    """A convolution or projection that is not the class the fused path stands for is called."""
+    layer = KimiDeltaAttention(128, 1, 128, mode="project_chunk", allow_fallback=False).cuda()
+
+    class Doubled(type(layer.v_conv1d)):
+        def forward(self, x, *args, **kw):
+            return super().forward(2 * x, *args, **kw)
+
+    x = torch.randn(2, 5, 128, device="cuda").bfloat16()
+    conv = Doubled(128).cuda()
+    conv.load_state_dict(layer.v_conv1d.state_dict())
+    with torch.no_grad():
+        ref, _ = layer(x, output_final_state=True)
+        layer.v_conv1d = conv
+        y, _ = layer(x, output_final_state=True)
+        layer.v_proj.weight.mul_(0.5)
+        y2, _ = layer(x, output_final_state=True)
+    assert rel_err(y, ref) > 0.1 and rel_err(y2, ref) < 2e-2
