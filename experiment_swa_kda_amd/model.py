@@ -410,14 +410,14 @@ class Block(nn.Module):
         """Whether a one-token step of a few sequences runs as _token: the mixer's own
         conditions for its one-token kernel, bf16 weights cached, no module hooks."""
         attn, mlp = self.attn, self.mlp
-        if x.shape[1] != 1 or x.shape[0] > 16 or not attn.mode.startswith("project_") or attn._cached16() is None:
+        if x.shape[1] != 1 or x.shape[0] > 16 or type(attn) is not KimiDeltaAttention or type(mlp) is not MLP:
             return False
-        if type(mlp.c_fc) is not Linear or mlp.c_fc.bias is not None or type(mlp.c_proj) is not Linear \
-                or mlp.c_proj.bias is not None:
+        if not attn.mode.startswith("project_") or attn._cached16() is None or not plain(attn, mlp, mlp.c_fc, mlp.c_proj):
+            return False
+        if any(type(m) is not Linear or m.bias is not None for m in (mlp.c_fc, mlp.c_proj)):
             return False
         w1, w2 = getattr(mlp.c_fc, "_w16", None), getattr(mlp.c_proj, "_w16", None)
-        if w1 is None or w2 is None or any(m._forward_hooks or m._forward_pre_hooks for m in (
-                attn, mlp, mlp.c_fc, mlp.c_proj, attn.o_proj)):
+        if w1 is None or w2 is None or w1.shape[0] % 32 or w2.shape != (x.shape[-1], w1.shape[0]):
             return False
         if torch.is_grad_enabled() and any(t.requires_grad for t in (
                 x, x0, lam_r, lam_0, mlp.c_fc.weight, mlp.c_proj.weight)):
@@ -550,7 +550,7 @@ class GPT(nn.Module):
         mid_out = None
         fused = _norm_fusable(x) and x0.shape == x.shape
         for i, block in enumerate(self.transformer.h):
-            if fused:
+            if fused and (kv_cache is None or (type(block) is Block and plain(block))):
                 x = block.forward_mixed(x, x0, self.resid_lambdas, self.x0_lambdas, i, kv_cache)
             else:
                 x = block(resid_mix(x, x0, self.resid_lambdas, self.x0_lambdas, i).to(torch.bfloat16), kv_cache)

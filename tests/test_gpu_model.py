@@ -458,6 +458,56 @@ def _small_decoder(seed=0):
     return model
 
 
+def _prompt_and_step(model, idx):
+    from experiment_swa_kda_amd.model import KVCache
+    cache = KVCache(idx.shape[0], 1, 64, 128, 2, "cuda", torch.bfloat16)
+    with torch.no_grad():
+        return model(idx[:, :-1], kv_cache=cache), model(idx[:, -1:], kv_cache=cache)
+
+
+_HOOKED = ["", "attn", "mlp", "mlp.c_fc", "mlp.c_proj"] + [
+    "attn." + n for n in ("q_proj", "k_proj", "v_proj", "g_proj", "f_a_proj", "f_b_proj", "b_proj", "o_proj",
+                          "q_conv1d", "k_conv1d", "v_conv1d")]
+
+
+@pytest.mark.parametrize("cached", [False, True])
+def test_hooks_of_every_submodule_fire_while_decoding(cached):
+    """A prompt and a token with a cache call every module that a hook watches, once each, and
+    a hook's replacement output is used; the logits stay those of the fused path (bf16
+    roundings of the intermediate results, 2^-8 through a few of them)."""
+    model = _small_decoder()
+    if cached:
+        model.cache_bf16_weights()
+    idx = torch.randint(0, 512, (2, 9), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    plain = _prompt_and_step(model, idx)
+    block = model.transformer.h[1]
+    for name in _HOOKED:
+        module = block.get_submodule(name)
+        for register in (module.register_forward_hook, module.register_forward_pre_hook):
+            calls = []
+            handle = register(lambda m, args, *out: calls.append(len(args)) or None)
+            got = _prompt_and_step(model, idx)
+            handle.remove()
+            assert len(calls) == 2, (name, register.__name__, calls)
+            for a, b in zip(got, plain):
+                assert rel_err(a, b) < 2e-2, name
+    handle = block.mlp.register_forward_hook(lambda m, args, out: torch.zeros_like(out))
+    zeroed = _prompt_and_step(model, idx)
+    handle.remove()
+    with torch.no_grad():
+        block.mlp.c_proj.weight.zero_()
+        if cached:
+            model.cache_bf16_weights()
+    for a, b in zip(zeroed, _prompt_and_step(model, idx)):
+        assert rel_err(a, b) < 2e-2
+    seen = []
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, args, out: seen.append(m) or None)
+    _prompt_and_step(model, idx)
+    handle.remove()
+    for name in _HOOKED:
+        assert sum(m is block.get_submodule(name) for m in seen) == 2, name
+
+
 def test_mlp_hooks_and_replacements_see_the_mlp_alone():
     """In training a hook of a block's MLP sees mlp(h), not the sum with the residual, and one
     that takes h alone can stand in its place."""
