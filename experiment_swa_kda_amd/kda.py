@@ -94,7 +94,7 @@ def _untransformed(*tensors):
         return False
     if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16:
         return False
-    return all(t is None or type(t) in _PLAIN_TENSORS for t in tensors)
+    return all([t is None or type(t) in _PLAIN_TENSORS for t in tensors])
 
 
 def plain(*modules):
@@ -104,8 +104,8 @@ def plain(*modules):
     if (_module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks
             or _module._global_backward_pre_hooks):
         return False
-    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                   or "forward" in m.__dict__ for m in modules)
+    return not any([m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                    or "forward" in m.__dict__ for m in modules])
 
 
 class _LinearBF16(torch.autograd.Function):
@@ -744,6 +744,10 @@ class ShortConvolution(nn.Conv1d):
         return y, (z[..., z.shape[-1] - width:].clone() if output_final_state else None)
 
 
+_LINEARS = ("q_proj", "k_proj", "v_proj", "g_proj", "f_a_proj", "b_proj", "f_b_proj", "o_proj")
+_CONVS = ("q_conv1d", "k_conv1d", "v_conv1d")
+
+
 class KimiDeltaAttention(nn.Module):
     """The KDA token mixer of one decoder layer (reference kda.py:676-798).
 
@@ -851,20 +855,23 @@ class KimiDeltaAttention(nn.Module):
             return False
         if D not in (64, 128) or self.conv_size != 4 or not -5.0 <= self.lower_bound < 0.0:
             return False
-        linears = (self.q_proj, self.k_proj, self.v_proj, self.g_proj, self.f_a_proj, self.b_proj, self.f_b_proj,
-                   self.o_proj)
-        convs = (self.q_conv1d, self.k_conv1d, self.v_conv1d)
-        if any(type(m) is not Linear or m.bias is not None for m in linears) or not plain(*linears, *convs):
+        # (by name from the dicts: attribute access of a module costs a microsecond each)
+        linears, convs = [self._modules[n] for n in _LINEARS], [self._modules[n] for n in _CONVS]
+        if any([type(m) is not Linear or m._parameters["bias"] is not None for m in linears]) or any(
+                [type(m) is not ShortConvolution or m.kernel_size != (4,) for m in convs]) or not plain(*linears, *convs):
             return False
-        if any(type(m) is not ShortConvolution or m.weight.shape != (C, 1, 4) for m in convs):
-            return False
-        params = [self.o_norm.weight, self.A_log, self.dt_bias]
+        weights = [m._parameters.get("weight") for m in (*linears, *convs)]
+        params = [self._modules["o_norm"].weight, self._parameters.get("A_log"), self._parameters.get("dt_bias")]
         carried = () if prompt else (state.memory, state.q_conv, state.k_conv, state.v_conv)
-        if not _untransformed(x, *params, *(m.weight for m in linears), *carried):
+        if any([p is None for p in (*params, *weights)]) or not _untransformed(x, *params, *weights, *carried):
             return False
         cached = self._cached16()
+        if cached is not None and not self._copies_current(weights):
+            return False
         if cached is None or torch.is_grad_enabled():
-            params += [m.weight for m in (*linears, *convs)]
+            params += weights
+            if any(w.numel() != 4 * C for w in weights[-3:]):
+                return False
         elif any(w.device != x.device for w in cached):
             return False
         if any(p.dtype != torch.float32 or p.device != x.device or not p.is_contiguous() or p.data_ptr() % 16
@@ -878,9 +885,28 @@ class KimiDeltaAttention(nn.Module):
         return not _needs_grad(x, *params, *carried)
 
     def _cached16(self):
+        mods = self._modules
         cached = (getattr(self, "_w16_in", None), getattr(self, "_conv_w16", None),
-                  getattr(self.f_b_proj, "_w16", None), getattr(self.o_proj, "_w16", None))
-        return cached if all(w is not None for w in cached) else None
+                  getattr(mods["f_b_proj"], "_w16", None), getattr(mods["o_proj"], "_w16", None))
+        return None if any([w is None for w in cached]) else cached
+
+    def keep_bf16_copies(self):
+        """Keeps bf16 copies of the stacked input projection and convolution taps, with what
+        tells whether a weight of the mixer has been written or replaced since (an alias keeps
+        its memory, so the address is not another tensor's).  Returns the copies."""
+        self._w16_in = self.stacked_input_weight_bf16()
+        self._conv_w16 = torch.cat([self.q_conv1d.weight, self.k_conv1d.weight, self.v_conv1d.weight]
+                                   ).squeeze(1).to(torch.bfloat16)
+        ws = [self._modules[n].weight for n in _LINEARS + _CONVS]
+        self._w16_of = None if any(w.is_inference() for w in ws) else [(w, w._version, w.detach()) for w in ws]
+        return [self._w16_in, self._conv_w16]
+
+    def _copies_current(self, weights):
+        """Whether the live weights are still those of the copies: the general path reads most of
+        them live, so the fused inference path leaves a call with others to it."""
+        return self._w16_of is not None and all(
+            [w is of and w._version == version and w.data_ptr() == alias.data_ptr()
+             for w, (of, version, alias) in zip(weights, self._w16_of)])
 
     def _weights16(self):
         """(stacked input projection, stacked convolution taps, f_b, o_proj) in bf16: the copies

@@ -464,17 +464,16 @@ class GPT(nn.Module):
     def cache_bf16_weights(self) -> list:
         """Casts the f32 projection weights to bf16 once: every Linear the forward calls and
         each mixer's stacked input projection and stacked convolution weights keep the copy and use it until
-        drop_bf16_weights() (one training update's microsteps all see the same weights).
+        drop_bf16_weights() (one training update's microsteps all see the same weights).  A call
+        with a cache reads the live stacked weights again once one of them has been replaced or
+        written (as autograd counts writes: one through ``.data`` goes unseen until the drop).
         Returns the copies."""
         out = []
         with torch.no_grad():
             stacked = set()
             for m in self.modules():
                 if isinstance(m, KimiDeltaAttention):
-                    m._w16_in = m.stacked_input_weight_bf16()
-                    m._conv_w16 = torch.cat([m.q_conv1d.weight, m.k_conv1d.weight, m.v_conv1d.weight]
-                                            ).squeeze(1).to(torch.bfloat16)
-                    out += [m._w16_in, m._conv_w16]
+                    out += m.keep_bf16_copies()
                     stacked.update(id(w) for w in m._in_weights())
             for m in self.modules():
                 if isinstance(m, Linear) and m.weight.dtype == torch.float32 and id(m.weight) not in stacked:
@@ -487,6 +486,7 @@ class GPT(nn.Module):
             if isinstance(m, KimiDeltaAttention):
                 m._w16_in = None
                 m._conv_w16 = None
+                m._w16_of = None
             if isinstance(m, Linear):
                 m._w16 = None
 

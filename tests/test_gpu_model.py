@@ -553,3 +553,36 @@ def test_replaced_submodules_run_at_inference():
         layer.v_proj.weight.mul_(0.5)
         y2, _ = layer(x, output_final_state=True)
     assert rel_err(y, ref) > 0.1 and rel_err(y2, ref) < 2e-2
+
+
+@pytest.mark.parametrize("change", ["write", "parameter", "data", "load"])
+def test_changed_weights_reach_decoding_with_cached_copies(change):
+    """With cached bf16 copies a prompt and a token that leave a state follow the input
+    projections and convolutions as they are now, however they were changed, as without copies."""
+    model = _small_decoder()
+    attn = model.transformer.h[0].attn
+    x = torch.randn(2, 6, 128, device="cuda").bfloat16()
+
+    def run():
+        with torch.no_grad():
+            y, st = attn(x[:, :5], output_final_state=True)
+            return y, attn(x[:, 5:], state=st, output_final_state=True, mode="project_recurrent")[0]
+
+    for name in ("q_proj", "k_proj", "v_proj", "g_proj", "f_a_proj", "b_proj", "q_conv1d", "k_conv1d", "v_conv1d"):
+        m = getattr(attn, name)
+        model.cache_bf16_weights()
+        before = run()
+        new = torch.randn_like(m.weight) * (m.weight.std() if name != "b_proj" else 1.0)
+        with torch.no_grad():
+            if change == "write":
+                m.weight.copy_(new)
+            elif change == "parameter":
+                m.weight = torch.nn.Parameter(new)
+            elif change == "data":
+                m.weight.data = new
+            else:
+                m.load_state_dict({"weight": new})
+        got = run()
+        model.drop_bf16_weights()
+        for a, b, old in zip(got, run(), before):
+            assert rel_err(a, b) < 1.2e-2 < 2e-2 < rel_err(a, old), name
