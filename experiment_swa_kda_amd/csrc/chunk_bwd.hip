@@ -2104,21 +2104,22 @@ static bool fused_backward_enabled() {
 // under the scan, but each scan member holds a CU that a tile could use, and the tiles' traffic
 // stretches the scan's step (0.45 -> 0.77 us).  It gains where the scan is a long chain on few
 // CUs with more than a round of tiles behind it (K = V = 128, whole K3 backward, fused against
-// separate launches): 98 against 121 us at 384 tiles x 48 strips (B2 T4096 H3), 135 / 165 at
-// 512 x 32, 173 / 176 at 768 x 96.  It loses when the strips fill the chip: 122 / 115 at 512 x
+// separate launches, both captured): 95 against 118 us at 384 tiles x 48 strips (B2 T4096 H3),
+// 135 / 152 at 512 x 32, 173 / 176 at 768 x 96.  It loses when the strips fill the chip: 122 / 115 at 512 x
 // 128, 433 / 322 at 1,536 x 192, 795 / 636 at 3,072 x 192 (B4 T8192 H6); the limit is 3/8 of
 // the CUs.  Its scan members wait for prep workgroups of the same launch, so the strips must
 // leave CUs free in any case: at 256 strips no prep workgroup could start.  A problem of at
 // most a quarter round of tiles has nothing to hide (44 / 45 us at 8 tiles), and the separate
 // launches cannot fail in a wait, so their callers need not read the failure flag.  With
-// K V <= 64^2 a tile is half as long and the lines lie lower: 70 / 73 us at 384 tiles x 24
-// strips, but 50 / 41 at 128 x 16, 83 / 77 at 512 x 32, 192 / 182 at 1,536 x 96.
+// K V <= 64^2 a tile is half as long and the lines lie lower: 73 / 73 us at 384 tiles x 24
+// strips, 83 / 76 at 512 x 32 (an eighth of the CUs: no longer), 192 / 182 at 1,536 x 96, and 50 /
+// 41 at 128 x 16.
 static bool fused_eligible(const ChunkGeom& g) {
   if (!fused_backward_enabled()) return false;
   const int cus = device_cu_count();
   const long tiles = (long)g.max_chunks * g.heads, strips = (long)g.num_seqs * g.heads * (g.V / 16);
   if (bwd_segments(g).len > 0) return false;
-  return g.K * g.V > 64 * 64 ? tiles > cus / 4 && 8 * strips <= 3L * cus : tiles > cus && 8 * strips <= cus;
+  return g.K * g.V > 64 * 64 ? tiles > cus / 4 && 8 * strips <= 3L * cus : tiles > cus && 8 * strips < cus;
 }
 
 // A wait of the fused launch that gives up has to be reported, so its caller reads a flag back

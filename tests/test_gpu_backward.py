@@ -506,6 +506,26 @@ def test_captured_call_equals_eager_call():
             assert x is None or torch.equal(x, y), (i, j)
 
 
+@pytest.mark.parametrize("B,T,H,K,fused", [(2, 4096, 3, 128, 1), (2, 4096, 3, 64, 1),
+                                            (2, 4096, 4, 64, 0),    # strips on an eighth of the CUs
+                                            (1, 8192, 3, 128, 0),   # a segmented scan
+                                            (1, 256, 2, 64, 0)])    # less than a round of tiles
+def test_launch_form_of_a_captured_call(B, T, H, K, fused):
+    """Which captured calls take the fused launch (256 CUs); no eager call does."""
+    import ctypes
+    from experiment_swa_kda_amd import _lib
+    lib = _lib.load()
+    q = torch.empty(B, T, H, K, dtype=torch.bfloat16, device="cuda")
+    p = ops._problem(q, q, None, ops.GATE_MODES["k3"], -5.0, K ** -0.5)
+    waits = lambda: lib.kda_chunk_backward_waits(ctypes.byref(p), torch.cuda.current_stream().cuda_stream)  # noqa: E731
+    assert waits() == 0
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = waits()
+        q.zero_()
+    assert captured == fused
+
+
 @pytest.mark.parametrize("B", [160, 161])
 def test_many_tiles_equal_their_halves(B):
     """1,280 tiles or more start staggered over the CUs; 640 or so do not.  Each sequence's
