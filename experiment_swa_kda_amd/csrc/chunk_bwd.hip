@@ -1787,21 +1787,22 @@ __global__ __launch_bounds__(kVjpThreads) void chunk_bwd_part_kernel(BwdArgs a, 
 // 631 us, this one launch 460 us.
 //
 // At K = V = 128 a workgroup has a CU to itself (its LDS) and every workgroup takes the same
-// time: the chip loads 256 tiles at once at the rate of memory (12 us of the 41 us of a tile,
-// 224 KB each), then computes 256 tiles with memory idle.  So the first workgroup of each CU
-// starts late by up to 31 steps of kStagger, the same step on every XCD (consecutive workgroups
-// go to different XCDs), and from then on some CUs load while others compute.  The start costs
-// up to 20 us and each later round saves about 5.  Medians without -> with: 768 tiles 118 ->
+// time: the chip loads a tile per CU at once at the rate of memory (12 us of the 41 us of a
+// round), then computes them with memory idle.  So the first workgroup of each CU (`staggered`
+// of them: the card's CUs, 0 for none) starts late by up to 31 steps of kStagger, the same step
+// on every XCD (consecutive workgroups go to different XCDs), and from then on some CUs load
+// while others compute.  The start costs up to 20 us and each later round saves about 5, so it
+// is done from kStaggerRounds rounds on.  Medians without -> with: 768 tiles 118 ->
 // 128 us, 1024 161 -> 163, 1280 200 -> 199, 1536 237 -> 230, 2048 307 -> 298, 2560 386 -> 360,
 // 3072 465 -> 442; packed documents of 2,064 tiles 318 -> 294.  Steps of 8, 15, 25, 35 and 45 at
 // 3072: 458, 447, 442, 449, 461 us.
-constexpr int kCUs = 256, kStaggerFrom = 5 * kCUs, kStagger = 25;  // kStagger: 64-clock units
+constexpr int kStaggerRounds = 5, kStagger = 25;  // kStagger: 64-clock units
 
 template <int K, int V>
-__global__ __launch_bounds__(kVjpThreads) void chunk_bwd_tile_kernel(BwdArgs a) {
+__global__ __launch_bounds__(kVjpThreads) void chunk_bwd_tile_kernel(BwdArgs a, int staggered) {
   if constexpr (K == 128 && V == 128) {
-    if (gridDim.x >= kStaggerFrom && blockIdx.x < kCUs)
-      for (int k = blockIdx.x / 8; k > 0; --k) __builtin_amdgcn_s_sleep(kStagger);
+    if ((int)blockIdx.x < staggered)
+      for (int k = blockIdx.x / kXcds; k > 0; --k) __builtin_amdgcn_s_sleep(kStagger);
   }
   const int cidx = blockIdx.x / a.H, h = blockIdx.x % a.H;
   const int4 ch = chunk_entry(a, cidx);
@@ -2257,7 +2258,8 @@ static int launch_backward(const kda_chunk_problem* p, const ChunkGeom& g, BwdAr
     constexpr size_t smem = TileSmem<K, V>::bytes;
     if (ensure_lds_limit((const void*)tiles, (int)smem) != hipSuccess)
       return set_error(KDA_ERR_LAUNCH, "chunk_backward: tile LDS attribute failed");
-    hipLaunchKernelGGL(tiles, dim3(g.max_chunks * p->heads), dim3(kVjpThreads), smem, stream, a);
+    const int cus = device_cu_count(), staggered = (long)g.max_chunks * p->heads >= kStaggerRounds * (long)cus ? cus : 0;
+    hipLaunchKernelGGL(tiles, dim3(g.max_chunks * p->heads), dim3(kVjpThreads), smem, stream, a, staggered);
     KDA_LAUNCH_CHECK("chunk_backward tiles");
   } else if (g.max_chunks > 0 && (dense || decay)) {
     // one part alone (the stage entry points)
