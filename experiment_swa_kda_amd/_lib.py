@@ -60,6 +60,7 @@ SIGNATURES = {
     "kda_chunk_backward_noalloc_max_scratch_bytes": (ctypes.c_size_t, []),
     "kda_chunk_backward_status": (ctypes.c_int, [_PP, _P, _P]),
     "kda_chunk_backward_waits": (ctypes.c_int, [_PP, _P]),
+    "kda_chunk_backward_segment_chunks": (ctypes.c_int, [_PP]),
     "kda_debug_set_wait_limit": (ctypes.c_int, [_L]),
     "kda_chunk_forward_stage": (ctypes.c_int, [_I, _PP] + [_P] * 11 + [_P]),
     "kda_chunk_backward_stage": (ctypes.c_int, [_I, _PP] + [_P] * 20 + [_P]),

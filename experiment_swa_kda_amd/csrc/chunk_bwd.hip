@@ -2398,6 +2398,13 @@ extern "C" int kda_chunk_backward_waits(const kda_chunk_problem* p, hipStream_t 
   return !generic_dims(p) && fused_backward(make_geom(p), stream);
 }
 
+extern "C" int kda_chunk_backward_segment_chunks(const kda_chunk_problem* p) {
+  using namespace kda;
+  if (validate_problem(p, "chunk_backward_segment_chunks") != KDA_OK) return 0;
+  if (padded_route(p)) return padded_segment_chunks(p);
+  return generic_dims(p) ? 0 : bwd_segments(make_geom(p)).len;
+}
+
 extern "C" int kda_chunk_backward_status(const kda_chunk_problem* p, const void* scratch,
                                          hipStream_t stream) {
   using namespace kda;

@@ -38,6 +38,7 @@ int padded_backward(const kda_chunk_problem* p, const void* beta_logits, const f
                     void* scratch, hipStream_t stream);
 int padded_status(const kda_chunk_problem* p, const void* scratch, hipStream_t stream);
 int padded_waits(const kda_chunk_problem* p, hipStream_t stream);
+int padded_segment_chunks(const kda_chunk_problem* p);
 
 constexpr size_t cmax_sz(size_t x, size_t y) { return x > y ? x : y; }
 

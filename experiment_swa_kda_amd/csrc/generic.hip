@@ -988,4 +988,9 @@ int padded_waits(const kda_chunk_problem* p, hipStream_t stream) {
   return kda_chunk_backward_waits(&pp, stream);
 }
 
+int padded_segment_chunks(const kda_chunk_problem* p) {
+  const kda_chunk_problem pp = padded_problem(p);
+  return kda_chunk_backward_segment_chunks(&pp);
+}
+
 }  // namespace kda

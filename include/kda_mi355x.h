@@ -197,6 +197,12 @@ int kda_chunk_backward_status(const kda_chunk_problem* p, const void* scratch, h
 int kda_chunk_backward_waits(const kda_chunk_problem* p, hipStream_t stream);
 
 /*
+ * Chunks per segment of the reverse scan that kda_chunk_backward uses for this problem; 0 if it
+ * runs every sequence in one pass.  Needs no device.  No counterpart in the reference.
+ */
+int kda_chunk_backward_segment_chunks(const kda_chunk_problem* p);
+
+/*
  * Sets the bound of every in-kernel wait of later kda_chunk_backward launches, in ticks of
  * the 100 MHz wall clock (process-wide; negative restores the 2 s default).  For tests of
  * the failure path: a bound of 0 makes every wait that is not already satisfied give up at

@@ -403,10 +403,14 @@ def test_norm_linear_rows_equals_separate_kernels(M, N, J, scalars):
 
 
 @pytest.mark.parametrize("B", [1, 16, 17])
-def test_decode_step_with_cached_weights_matches_full_forward(B):
-    """Cached bf16 weights and at most 16 sequences: five launches per layer (17: the general
-    decode path); every step's logits equal the full-sequence forward at that position."""
+def test_decode_step_with_cached_weights_matches_full_forward(B, monkeypatch):
+    """Cached bf16 weights and at most 16 sequences: five launches per layer, two of them with
+    a norm in front of the projection (17: the general decode path); every step's logits equal
+    the full-sequence forward at that position."""
+    from experiment_swa_kda_amd import ops
     from experiment_swa_kda_amd.model import KVCache
+    calls, launch = [], ops.norm_linear_rows
+    monkeypatch.setattr(ops, "norm_linear_rows", lambda *a, **k: (calls.append(1), launch(*a, **k))[1])
     cfg = GPTConfig(sequence_len=64, vocab_size=512, n_layer=3, n_head=3, n_embd=384)
     torch.manual_seed(0)
     model = GPT(cfg).cuda()
@@ -426,6 +430,7 @@ def test_decode_step_with_cached_weights_matches_full_forward(B):
         assert rel_err(model(idx[:, :P], kv_cache=cache), full[:, :P]) < 2e-2
         for t in range(P, T):
             assert rel_err(model(idx[:, t:t + 1], kv_cache=cache)[:, 0], full[:, t]) < 2e-2, t
+    assert len(calls) == (2 * 3 * (T - P) if B <= 16 else 0)
 
 
 def test_linear_of_few_rows_traces():
