@@ -591,3 +591,22 @@ def test_changed_weights_reach_decoding_with_cached_copies(change):
         model.drop_bf16_weights()
         for a, b, old in zip(got, run(), before):
             assert rel_err(a, b) < 1.2e-2 < 2e-2 < rel_err(a, old), name
+
+
+def test_linear_of_few_rows_answers_as_many_rows_do():
+    """Autocast's type, a tensor subclass and a call of another width are answered at 8 rows as
+    at 100, where the library product runs."""
+    from experiment_swa_kda_amd.kda import Linear
+
+    class Tagged(torch.Tensor):
+        pass
+
+    layer = Linear(128, 64, bias=False).cuda()
+    for rows in (8, 100):
+        x = torch.randn(rows, 128, device="cuda").bfloat16()
+        with torch.no_grad():
+            with torch.autocast("cuda", dtype=torch.float16):
+                assert layer(x).dtype == torch.float16
+            assert type(layer(x.as_subclass(Tagged))) is Tagged
+            with pytest.raises(RuntimeError, match="shapes cannot be multiplied"):
+                layer(x[:, :64].contiguous())
