@@ -951,7 +951,7 @@ class KimiDeltaAttention(nn.Module):
             _record("chunk_forward_conv_norm_gate")
             state = KDAState(memory, windows[0], windows[1], windows[2])
         else:
-            out, state = self._token_core(y.view(n_b, -1), state, state_in_place and keep_state)
+            out, state = self._token_core(y.view(n_b, -1), state, state_in_place)
         return self.o_proj(out.view(n_b, n_t, C), w16=o16), state if keep_state else None
 
     def _token_core(self, y, state, state_in_place):

@@ -610,3 +610,17 @@ def test_linear_of_few_rows_answers_as_many_rows_do():
             assert type(layer(x.as_subclass(Tagged))) is Tagged
             with pytest.raises(RuntimeError, match="shapes cannot be multiplied"):
                 layer(x[:, :64].contiguous())
+
+
+def test_token_updates_the_state_in_place_without_returning_it():
+    """state_in_place writes state.memory whether or not the call returns the state."""
+    from experiment_swa_kda_amd import KDAState
+    layer = KimiDeltaAttention(128, 1, 128, mode="project_chunk", allow_fallback=False).cuda()
+    x = torch.randn(2, 5, 128, device="cuda").bfloat16()
+    with torch.no_grad():
+        _, st = layer(x[:, :4], output_final_state=True)
+        kept = KDAState(st.memory.clone(), st.q_conv, st.k_conv, st.v_conv)
+        y, new = layer(x[:, 4:], state=st, output_final_state=True, mode="project_recurrent")
+        y2, none = layer(x[:, 4:], state=kept, mode="project_recurrent", state_in_place=True)
+    assert none is None and torch.equal(y, y2)
+    assert torch.equal(kept.memory, new.memory) and not torch.equal(kept.memory, st.memory)
