@@ -958,10 +958,11 @@ class KimiDeltaAttention(nn.Module):
         """One token between the projections: the stacked projection's rows y [B, N] and the
         carried state -> (normed output [B, C], new state)."""
         _, conv16, fb16, _ = self._weights16()
+        norm = self.o_norm
         out, memory, windows = ops.mixer_step(
-            y, conv16, (state.q_conv, state.k_conv, state.v_conv), fb16, self.A_log, self.dt_bias, self.o_norm.weight,
+            y, conv16, (state.q_conv, state.k_conv, state.v_conv), fb16, self.A_log, self.dt_bias, norm.weight,
             state.memory, self.num_heads, float(self.lower_bound), float(self.head_dim ** -0.5),
-            float(self.o_norm.eps), out_memory=state.memory if state_in_place else None)
+            float(norm.eps), out_memory=state.memory if state_in_place else None)
         _record("mixer_step")
         return out, KDAState(memory, windows[0], windows[1], windows[2])
 

@@ -409,18 +409,20 @@ class Block(nn.Module):
     def _token_ok(self, x, x0, lam_r, lam_0, kv_cache):
         """Whether a one-token step of a few sequences runs as _token: the mixer's own
         conditions for its one-token kernel, bf16 weights cached, no module hooks."""
-        attn, mlp = self.attn, self.mlp
+        # (submodules from the dicts: attribute access of a module costs a microsecond each)
+        attn, mlp = self._modules["attn"], self._modules["mlp"]
         if x.shape[1] != 1 or x.shape[0] > 16 or type(attn) is not KimiDeltaAttention or type(mlp) is not MLP:
             return False
-        if not attn.mode.startswith("project_") or attn._cached16() is None or not plain(attn, mlp, mlp.c_fc, mlp.c_proj):
+        fc, proj = mlp._modules["c_fc"], mlp._modules["c_proj"]
+        if not attn.mode.startswith("project_") or attn._cached16() is None or not plain(attn, mlp, fc, proj):
             return False
-        if any(type(m) is not Linear or m.bias is not None for m in (mlp.c_fc, mlp.c_proj)):
+        if type(fc) is not Linear or type(proj) is not Linear or fc.bias is not None or proj.bias is not None:
             return False
-        w1, w2 = getattr(mlp.c_fc, "_w16", None), getattr(mlp.c_proj, "_w16", None)
+        w1, w2 = getattr(fc, "_w16", None), getattr(proj, "_w16", None)
         if w1 is None or w2 is None or w1.shape[0] % 32 or w2.shape != (x.shape[-1], w1.shape[0]):
             return False
         if torch.is_grad_enabled() and any(t.requires_grad for t in (
-                x, x0, lam_r, lam_0, mlp.c_fc.weight, mlp.c_proj.weight)):
+                x, x0, lam_r, lam_0, fc.weight, proj.weight)):
             return False
         return w1.device == x.device and attn._inference_ok(
             x, kv_cache.get_kda_state(attn.layer_idx), "project_recurrent")
@@ -428,14 +430,15 @@ class Block(nn.Module):
     def _token(self, x, x0, lam_r, lam_0, i, kv_cache):
         """forward_mixed for one token in five launches: mix + norm + input projection, mixer
         step, output projection, add + norm + c_fc + relu^2, c_proj + add."""
-        attn, layer = self.attn, self.attn.layer_idx
+        attn, mlp = self._modules["attn"], self._modules["mlp"]._modules
+        layer = attn.layer_idx
         w_in, _, _, o16 = attn._weights16()
         s, y = ops.norm_linear_rows(x, x0, w_in, _RMS_EPS, a=lam_r, b=lam_0, slot=i)
         out, state = attn._token_core(y.view(x.shape[0], -1), kv_cache.get_kda_state(layer), kv_cache.inplace_state)
         kv_cache.set_kda_state(layer, state)
         mixed = ops.linear_rows(out.view(x.shape), o16)
-        s, h = ops.norm_linear_rows(s, mixed, self.mlp.c_fc._w16, _RMS_EPS, relu2=True)
-        return ops.linear_rows(h, self.mlp.c_proj._w16, residual=s)
+        s, h = ops.norm_linear_rows(s, mixed, mlp["c_fc"]._w16, _RMS_EPS, relu2=True)
+        return ops.linear_rows(h, mlp["c_proj"]._w16, residual=s)
 
 
 class GPT(nn.Module):
