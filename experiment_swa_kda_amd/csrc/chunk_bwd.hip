@@ -19,18 +19,19 @@
 // MI355X mapping:
 //  * scan kernel: one workgroup per (sequence, head, 16-wide V strip); dS columns are
 //    independent, so the 128x16 f32 slice of dS lives in VGPRs as MFMA accumulators of four
-//    compute waves, fed by two loader waves through an LDS ring of direct global->LDS loads.
+//    compute waves; -G comes straight into their registers, E and lam through an LDS ring that a
+//    loader wave fills.  Long sequences with few strips run in segments (chunk_bwd_seg_kernel).
 //    The launch also carries cache-warming workgroups for the CUs the scan leaves idle.
 //  * dense and decay VJPs: one workgroup per (chunk, head) tile runs the dense and then the
-//    decay part, handing the dense results over on chip.  Dense: 16x16x32 bf16 MFMA tiles with f32 accumulation, every global
-//    operand requested in one batch.  Decay: the decay-scaled operands are built once per
+//    decay part, handing the dense results over on chip.  Dense: 16x16x32 bf16 MFMA tiles with
+//    f32 accumulation, every global operand requested in one batch.  Decay: the decay-scaled operands are built once per
 //    tile around the first (row side) or last (column side) row of each 16-row block, so
 //    every factor is <= 1 or bounded by the block's span; a tile with a block whose decay
 //    span exceeds 80 nats runs an exact per-pair f32 loop instead.
-//  * fused launch (the whole backward in one call): the scan members, the prep workgroups
-//    and the tile workgroups share one grid; a tile runs its dense and decay parts as soon as the scan
-//    has finalised its chunk, so the VJP work overlaps the latency-bound scan (see
-//    chunk_bwd_fused_kernel).  The staged entry points keep the separate launches.
+//  * fused launch (captured calls that gain from it, see fused_backward): the scan members, the
+//    prep workgroups and the tile workgroups share one grid; a tile runs its dense and decay
+//    parts as soon as the scan has finalised its chunk, so the VJP work overlaps the
+//    latency-bound scan (see chunk_bwd_fused_kernel).  Other calls run separate launches.
 #include "chunk_host.hpp"
 #include "kda_device.hpp"
 #include "seg_combine.hpp"
