@@ -469,7 +469,8 @@ class GPT(nn.Module):
         each mixer's stacked input projection and stacked convolution weights keep the copy and use it until
         drop_bf16_weights() (one training update's microsteps all see the same weights).  A call
         with a cache reads the live stacked weights again once one of them has been replaced or
-        written (as autograd counts writes: one through ``.data`` goes unseen until the drop).
+        written (as autograd counts writes: one through ``.data`` or by a replayed graph goes
+        unseen until the drop).
         Returns the copies."""
         out = []
         with torch.no_grad():
